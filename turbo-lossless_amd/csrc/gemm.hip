@@ -33,7 +33,8 @@
 //     in the LDS tile.
 //
 // Fast path requirements: K % 64 == 0, 0 <= base_exp <= 240, 16-byte aligned
-// activation rows.  Everything else goes to the general kernel below.
+// activation rows.  Everything else goes to the general kernel below.  3 .. 64 rows, where the weight stream is the
+// bound, have a kernel of their own (gemm_ring.h) and, on short or few rows, the whole-row sweep.
 
 #include <map>
 #include <mutex>
@@ -44,6 +45,9 @@
 #include "t12_device.h"
 #include "t12_host.h"
 #include "dense16_plan.h"
+#include "gemm_params.h"
+#include "gemm_ring.h"
+#include "ring_plan.h"
 
 // library-internal (hidden: not part of the ABI)
 extern "C" __attribute__((visibility("hidden"))) void t12_glue_release_stream(hipStream_t st);      // glue.hip
@@ -56,49 +60,6 @@ constexpr int TM = 128;         // weight rows per workgroup
 constexpr int PCAP = 2048;      // escape entries a workgroup can stage in LDS
 constexpr int PATCH_BYTES = PCAP * 4 + (TM + 1) * 4 + 12;
 constexpr int NO_ESCAPE = 0x7FFFFFFF;
-
-constexpr int GMAX = 16;        // segments of one launch (a grouped launch: gate and up of eight experts)
-static_assert(GMAX >= T12_MAX_SEGMENTS, "t12_gemm takes T12_MAX_SEGMENTS segments");
-
-// One launch multiplies up to GMAX tensors.  t12_gemm: all of them with the same activations [B, K]; a grouped
-// launch (t12_gemm_grouped): segment i with its own seg_act[i] of seg_B[i] rows.  The tile kernel and the K-split
-// reduction read the per-segment fields, which t12_gemm fills with the shared values; the other kernels read
-// act / B / act_stride.
-struct GemmParams {
-    T12Segment seg[GMAX];
-    int blk_start[GMAX + 1];               // first row-tile of each segment
-    int seg_row0[GMAX];                    // first row of each segment among all rows of the launch
-    const uint16_t* seg_act[GMAX];
-    int seg_B[GMAX];
-    int seg_act_stride[GMAX];
-    // partial sums of segment i, split z, element (b, m): ws[z * split_stride + seg_ws0[i] + b * seg_ld[i] + m]
-    //   t12_gemm: seg_ws0 = seg_row0, seg_ld = m_total (rows of length m_total, what t12_gemm_deferred describes)
-    //   grouped:  seg_ws0 = sum of B * M over the segments before, seg_ld = M
-    size_t seg_ws0[GMAX];
-    int seg_ld[GMAX];
-    size_t split_stride;
-    int nseg;
-    int K, B;                              // B: t12_gemm's batch; grouped: the largest seg_B
-    int act_stride;
-    int ksplit;                            // workgroups along K
-    int kslice;                            // columns per K split (multiple of KC)
-    int m_total;                           // sum of M over segments
-    const uint16_t* act;
-    float* ws;                             // partial sums when ksplit > 1
-    uint16_t* out_bf16;                    // SwiGLU mode: bf16 [B, out_bf16_ld], silu(seg 2i) * seg 2i+1 of pair i
-    int out_bf16_ld;
-    float act_a, act_b;                    // EPI launches: the constants of the unary function
-    T12Glu glu = t12_silu_glu();           // SwiGLU mode: the unit
-    int npair = 1;                         // SwiGLU mode: (gate, up) pairs of the launch; blk_start[i] = first tile of pair i
-    // Rows per group known on the device only (the experts of a mixture-of-experts layer, counted by the routing
-    // kernel): group_of_seg[s] picks an entry of dev_counts / dev_base, the segment's batch is dev_counts[.] and its
-    // activations, outputs (fp32 and bf16) start dev_base[.] rows into the pointers given.  The grid then has one
-    // workgroup per row tile, which walks the group's batch tiles.  nullptr: seg_B as given.
-    const int* dev_counts = nullptr;
-    const int* dev_base = nullptr;
-    int group_of_seg[GMAX];
-    int n_first = 0;                       // mixed small-batch launch: segments [0, n_first) take the larger workgroups
-};
 
 // LDS slot of (unit, row) in a [units][rows] array of 16-byte units.  Rows are rotated
 // inside their aligned block of eight by the unit index, so that both access patterns are
@@ -115,23 +76,6 @@ __device__ __forceinline__ constexpr int stage_unit_order(int pos, int nact, int
     const int dec_before = pos * ndec / nu;              // decode units placed before pos
     const bool is_dec = (pos + 1) * ndec / nu > dec_before;
     return is_dec ? nact + dec_before : pos - dec_before;
-}
-
-__device__ __forceinline__ int find_segment(const GemmParams& p, int tile)
-{
-    int s = 0;
-#pragma unroll
-    for (int i = 1; i < GMAX; i++)
-        if (i < p.nseg && tile >= p.blk_start[i]) s = i;
-    return s;
-}
-__device__ __forceinline__ int find_pair(const GemmParams& p, int tile)
-{
-    int s = 0;
-#pragma unroll
-    for (int i = 1; i < GMAX / 2; i++)
-        if (i < p.npair && tile >= p.blk_start[i]) s = i;
-    return s;
 }
 
 // ---------------------------------------------------------------------------
@@ -1135,6 +1079,69 @@ int launch_mfma(GemmParams& p, int tiles, hipStream_t st)
 }
 
 
+template <int RW, int KW, int NBT, bool GLU = false, int EPI = T12_ACT_NONE, bool DEV = false>
+int launch_ring(GemmParams& p, int tiles, hipStream_t st)
+{
+    const dim3 grid(tiles, DEV ? 1 : (p.B + 16 * NBT - 1) / (16 * NBT), p.ksplit);
+    hipLaunchKernelGGL((gemm_ring_kernel<RW, KW, NBT, GLU, EPI, DEV>), grid, dim3(RW * KW * 64), 0, st, p);
+    T12_CHECK_LAUNCH("t12_gemm(ring)");
+    return T12_OK;
+}
+
+// CUs of the current device (a launch of one workgroup per CU is one round of the small-batch kernel).
+int device_cus()
+{
+    static std::mutex mu;
+    static int cus[16] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return 256;
+    std::lock_guard<std::mutex> lock(mu);
+    if (!cus[dev]) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+        cus[dev] = n;
+    }
+    return cus[dev];
+}
+
+// The ring kernel's form for a launch of p's segments (0 .. nseg - 1), or none: 3 .. 64 rows, K of whole 128-column
+// windows, planes that 16-byte copies may be taken from.
+RingPlan ring_plan_of(const GemmParams& p, int nseg)
+{
+    RingPlan none = {0, 0, 1, 0.0f};
+    if (p.B < 3 || p.B > RING_MAX_B || p.K % RING_WC) return none;
+    int rows[GMAX];
+    for (int i = 0; i < nseg; i++) {
+        if ((uintptr_t)p.seg[i].sm % 16 || (uintptr_t)p.seg[i].gr % 16) return none;
+        rows[i] = p.seg[i].M;
+    }
+    return plan_ring(rows, nseg, p.K, p.B, device_cus());
+}
+
+template <int NBT, bool GLU>
+int launch_ring_nbt(const RingPlan& r, GemmParams& p, int sets, hipStream_t st)
+{
+    if (r.kw == 1) return launch_ring<8, 1, NBT, GLU>(p, sets, st);
+    if (r.kw == 2) return launch_ring<4, 2, NBT, GLU>(p, sets, st);
+    if constexpr (NBT <= 2) {
+        if (r.kw == 4) return launch_ring<2, 4, NBT, GLU>(p, sets, st);
+    }
+    if constexpr (NBT == 1) {
+        if (r.kw == 8) return launch_ring<1, 8, NBT, GLU>(p, sets, st);
+    }
+    t12_set_error("t12_gemm: no ring form %d x %d for %d batch tiles", r.rw, r.kw, NBT);
+    return T12_EINVAL;
+}
+
+template <bool GLU = false>
+int launch_ring_form(const RingPlan& r, GemmParams& p, int sets, hipStream_t st)
+{
+    const int nbt = ring_batch_tiles(p.B);
+    if (nbt == 1) return launch_ring_nbt<1, GLU>(r, p, sets, st);
+    if (nbt == 2) return launch_ring_nbt<2, GLU>(r, p, sets, st);
+    return launch_ring_nbt<4, GLU>(r, p, sets, st);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1164,48 +1171,15 @@ int t12_gemm_glu(const T12Segment* gate, const T12Segment* up, const T12Glu* glu
     T12_REQUIRE(gate->M >= 1 && gate->M == up->M, "t12_gemm_glu: gate has %d rows, up has %d", gate->M, up->M);
     T12_REQUIRE(out_stride >= gate->M, "t12_gemm_glu: out_stride %d < M %d", out_stride, gate->M);
     const T12Segment* two[2] = {gate, up};
-    bool fast = (K % KC == 0) && (act_stride % 8 == 0) && ((uintptr_t)act_bf16 % 16 == 0) && B > 64;
+    const bool aligned = act_stride % 8 == 0 && (uintptr_t)act_bf16 % 16 == 0;
+    bool exps = true;
     for (const T12Segment* g : two) {
         T12_REQUIRE(g->sm && g->gr, "t12_gemm_glu: a plane is null");
         T12_REQUIRE(!g->row_off || (g->cols && g->correct && g->wrong), "t12_gemm_glu: row_off without lists");
         T12_REQUIRE(g->base_exp >= -1 && g->base_exp <= 254, "t12_gemm_glu: base_exp %d out of range", g->base_exp);
-        if (g->base_exp < 0 || g->base_exp > 240) fast = false;
+        if (g->base_exp < 0 || g->base_exp > 240) exps = false;
     }
-    // 5 .. 8 batch rows: the whole-row sweep over 32 rows of gate and the same rows of up per workgroup.  Measured on
-    // 2 x 14336 x 4096 against t12_gemm + launch_silu_mul_bf16_batch: 43.6 / 44.7 us at B = 5 / 8 against 44.3 / 47.1; no
-    // gain at B <= 4 (43.9 against 44.2; B = 2: 44.5 against 39) nor above 8, where the unfused launch balances its
-    // last round (B = 9 / 12 / 16: 45.3 / 46.7 / 49.0 against 45.5 / 46.6 / 48.4).
-    bool sweep = K % 128 == 0 && act_stride % 8 == 0 && (uintptr_t)act_bf16 % 16 == 0 && B >= 5 && B <= 8;
-    for (const T12Segment* g : two)
-        if (g->base_exp < 0 || g->base_exp > 240) sweep = false;
-    if (sweep) {
-        const int rg = 4;
-        GemmParams p;
-        p.glu = *glu;
-        p.seg[0] = *gate;
-        p.seg[1] = *up;
-        p.nseg = 2;
-        p.K = K;
-        p.B = B;
-        p.act_stride = act_stride;
-        p.act = (const uint16_t*)act_bf16;
-        p.ws = nullptr;
-        p.ksplit = 1;
-        p.kslice = K;
-        p.m_total = gate->M;
-        const int sets = (gate->M + 8 * rg - 1) / (8 * rg);
-        p.blk_start[0] = 0;
-        p.blk_start[1] = p.blk_start[2] = sets;
-        p.out_bf16 = (uint16_t*)out_bf16;
-        p.out_bf16_ld = out_stride;
-        hipStream_t st = (hipStream_t)stream;
-        hipLaunchKernelGGL((gemm_dense16_swiglu_kernel<8, 2, 4>), dim3(sets), dim3(512), 0, st, p);
-        T12_CHECK_LAUNCH("t12_gemm_glu(dense16)");
-        return T12_OK;
-    }
-    const int tiles = (gate->M + TM / 2 - 1) / (TM / 2);
-    const int btiles = B > 128 ? (B + 255) / 256 : 1;
-    if (!fast || tiles * btiles * 4 < 256 * 3) return 1;      // would need a K split: partial sums cannot be gated
+    hipStream_t st = (hipStream_t)stream;
     GemmParams p;
     p.glu = *glu;
     p.seg[0] = *gate;
@@ -1217,19 +1191,47 @@ int t12_gemm_glu(const T12Segment* gate, const T12Segment* up, const T12Glu* glu
     p.act = (const uint16_t*)act_bf16;
     p.ws = nullptr;
     p.ksplit = 1;
-    p.kslice = ((K + 2 * KC - 1) / (2 * KC)) * 2 * KC;
     p.m_total = gate->M;
-    p.seg_act[0] = p.act;                  // the SwiGLU tile reads the fields of segment 0
+    p.seg_act[0] = p.act;                  // the paired kernels read the fields of segment 0
     p.seg_B[0] = B;
     p.seg_act_stride[0] = act_stride;
-    p.blk_start[0] = 0;
-    p.blk_start[1] = p.blk_start[2] = tiles;
     p.seg_row0[0] = p.seg_row0[1] = 0;
     p.out_bf16 = (uint16_t*)out_bf16;
     p.out_bf16_ld = out_stride;
+    if (B <= 64) {
+        // The form that t12_gemm would take for the two tensors, so that the sums are the same bit for bit; above 8 rows
+        // only where that fills the chip (the fp32 round trip of both projections and a launch of their own for the unit are
+        // 4.8 us at 28672 rows and B = 64).
+        const bool fast = K % 128 == 0 && aligned && exps && B >= 5;
+        const RingPlan ring = fast ? ring_plan_of(p, 2) : RingPlan{0, 0, 1, 0.0f};
+        if (ring.rw && ring.ks == 1 && (B <= 8 || (ring.kw == 1 && gate->M >= 64 * 128))) {
+            const int sets = (gate->M + 8 * ring.rw - 1) / (8 * ring.rw);
+            p.kslice = K;
+            p.blk_start[0] = 0;
+            p.blk_start[1] = p.blk_start[2] = sets;
+            return launch_ring_form<true>(ring, p, sets, st);
+        }
+        if (!fast || B > 8 || ring.rw) return 1;
+        // 5 .. 8 batch rows on fewer or shorter rows: the whole-row sweep over 32 rows of gate and the same rows of up per
+        // workgroup (no gain at B <= 4, nor above 8, where the unfused launch balances its last round)
+        const int sets = (gate->M + 31) / 32;
+        p.kslice = K;
+        p.blk_start[0] = 0;
+        p.blk_start[1] = p.blk_start[2] = sets;
+        hipLaunchKernelGGL((gemm_dense16_swiglu_kernel<8, 2, 4>), dim3(sets), dim3(512), 0, st, p);
+        T12_CHECK_LAUNCH("t12_gemm_glu(dense16)");
+        return T12_OK;
+    }
+    const bool fast = K % KC == 0 && aligned && exps;
+    const int tiles = (gate->M + TM / 2 - 1) / (TM / 2);
+    const int btiles = B > 128 ? (B + 255) / 256 : 1;
+    if (!fast || tiles * btiles * 4 < 256 * 3) return 1;      // would need a K split: partial sums cannot be gated
+    p.kslice = ((K + 2 * KC - 1) / (2 * KC)) * 2 * KC;
+    p.blk_start[0] = 0;
+    p.blk_start[1] = p.blk_start[2] = tiles;
     // batch tile of 256 rows, or of 128 for 65 .. 128 rows (one accumulator pair per wave)
-    if (B <= 128) return launch_mfma<4, 2, 1, 2, true>(p, tiles, (hipStream_t)stream);
-    return launch_mfma<4, 2, 2, 2, true>(p, tiles, (hipStream_t)stream);
+    if (B <= 128) return launch_mfma<4, 2, 1, 2, true>(p, tiles, st);
+    return launch_mfma<4, 2, 2, 2, true>(p, tiles, st);
 }
 
 // out_bf16[b, m] = bf16(act(W[m,:] . X[b,:])) with the function in the GEMM's epilogue.  Returns T12_OK when launched, 1
@@ -1277,22 +1279,6 @@ int t12_gemm_act(const T12Segment* seg, const void* act_bf16, int act_stride, in
 }  // extern "C"
 
 namespace {
-
-// CUs of the current device (a launch of one workgroup per CU is one round of the small-batch kernel).
-int device_cus()
-{
-    static std::mutex mu;
-    static int cus[16] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return 256;
-    std::lock_guard<std::mutex> lock(mu);
-    if (!cus[dev]) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-        cus[dev] = n;
-    }
-    return cus[dev];
-}
 
 // The small-batch launch with rg row groups per workgroup whose last round would fill only part of the chip: every
 // tensor is cut into a head, swept rg groups per workgroup in whole rounds, and a tail swept in fewer groups per
@@ -1432,6 +1418,58 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         T12_CHECK_LAUNCH("t12_gemm(rows)");
         return T12_OK;
     }
+    // K split: where the partial sums of p.ksplit slices go, and who adds them up
+    auto take_workspace = [&]() {
+        const size_t need = (size_t)p.ksplit * B * m_total * sizeof(float);
+        if (static_ws) {
+            T12_REQUIRE(need <= STATIC_WS_BYTES,
+                        "t12_gemm_noalloc: this shape splits K %d ways and needs %zu bytes of partial sums, the fixed "
+                        "workspace holds %zu (B %d x %d rows): use t12_gemm, or a smaller batch", p.ksplit, need, STATIC_WS_BYTES, B,
+                        m_total);
+            p.ws = static_workspace();
+            if (!p.ws) {
+                t12_set_error("t12_gemm_noalloc: hipGetSymbolAddress of the fixed workspace failed");
+                return T12_ELAUNCH;
+            }
+            return T12_OK;
+        }
+        p.ws = workspace(need, st);
+        if (!p.ws) {
+            t12_set_error("%s: cannot allocate %zu bytes of K-split workspace", who, need);
+            return T12_ELAUNCH;
+        }
+        return T12_OK;
+    };
+    auto finish = [&]() {
+        if (p.ksplit > 1 && part) {
+            part->ws = p.ws;
+            part->nsplit = p.ksplit;
+            part->ld = m_total;
+            part->split_stride = (size_t)B * m_total;
+        } else if (p.ksplit > 1) {
+            launch_reduce(p, B, st);
+            T12_CHECK_LAUNCH("t12_gemm(reduce)");
+        }
+        return T12_OK;
+    };
+    const RingPlan ring = ring_plan_of(p, nseg);
+    if (ring.rw) {
+        int sets = 0;
+        for (int i = 0; i < nseg; i++) {
+            p.blk_start[i] = sets;
+            sets += (segs[i].M + 16 * ring.rw - 1) / (16 * ring.rw);
+        }
+        p.blk_start[nseg] = sets;
+        const int per = (K / RING_WC + ring.ks - 1) / ring.ks;
+        p.ksplit = ring.ks;
+        p.kslice = per * RING_WC;
+        if (p.ksplit > 1) {
+            const int rc = take_workspace();
+            if (rc) return rc;
+        }
+        const int rc = launch_ring_form(ring, p, sets, st);
+        return rc ? rc : finish();
+    }
     if (B > 16 && B <= 32 && K % 128 == 0) {
         // 17 .. 32 batch rows on tensors of few rows: the same sweep with two batch tiles per weight load and decode.
         // One round of workgroups takes ~4.5 us + (K / 4096) (3.7 + 0.2 B) us whatever the row count, because every
@@ -1508,41 +1546,15 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
     ks = (K + kslice - 1) / kslice;
     p.ksplit = ks;
     p.kslice = kslice;
-    if (ks > 1 && static_ws) {
-        const size_t need = (size_t)ks * B * m_total * sizeof(float);
-        T12_REQUIRE(need <= STATIC_WS_BYTES,
-                    "t12_gemm_noalloc: this shape splits K %d ways and needs %zu bytes of partial sums, the fixed "
-                    "workspace holds %zu (B %d x %d rows): use t12_gemm, or a smaller batch", ks, need, STATIC_WS_BYTES, B,
-                    m_total);
-        p.ws = static_workspace();
-        if (!p.ws) {
-            t12_set_error("t12_gemm_noalloc: hipGetSymbolAddress of the fixed workspace failed");
-            return T12_ELAUNCH;
-        }
-    } else if (ks > 1) {
-        p.ws = workspace((size_t)ks * B * m_total * sizeof(float), st);
-        if (!p.ws) {
-            t12_set_error("%s: cannot allocate %zu bytes of K-split workspace", who,
-                          (size_t)ks * B * m_total * sizeof(float));
-            return T12_ELAUNCH;
-        }
+    if (ks > 1) {
+        const int rc_ws = take_workspace();
+        if (rc_ws) return rc_ws;
     }
     int rc;
     if (B <= 64) rc = launch_mfma<2, 4, 1, 1>(p, tiles, st);
     else if (B <= 128 || tb128) rc = launch_mfma<2, 4, 2, 1>(p, tiles, st);
     else rc = launch_mfma<4, 2, 2, 2>(p, tiles, st);
-    if (rc) return rc;
-
-    if (ks > 1 && part) {
-        part->ws = p.ws;
-        part->nsplit = ks;
-        part->ld = m_total;
-        part->split_stride = (size_t)B * m_total;
-    } else if (ks > 1) {
-        launch_reduce(p, B, st);
-        T12_CHECK_LAUNCH("t12_gemm(reduce)");
-    }
-    return T12_OK;
+    return rc ? rc : finish();
 }
 
 }  // namespace
