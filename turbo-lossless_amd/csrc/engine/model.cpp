@@ -471,7 +471,7 @@ Model* create_synthetic_model(const ModelConfig& cfg, uint64_t seed, int max_seq
     m->config = cfg;
     const int n = cfg.n_embd, ff = cfg.n_ff;
     const int kv = cfg.n_head_kv * (n / cfg.n_head);
-    const size_t biggest = std::max({(size_t)cfg.n_vocab * n, (size_t)ff * n});
+    const size_t biggest = (size_t)std::max({cfg.n_vocab, ff, n}) * n;      // kv <= n: wk and wv are covered by wq
     uint16_t* stage = device_alloc<uint16_t>(biggest);
     uint64_t s = seed;
     bool ok = true;
