@@ -44,6 +44,8 @@ void launch_rope_store_attention(float*, float*, const float*, int8_t*, int8_t*,
                                  int, int, int, int, float, float, int, int, hipStream_t);
 void launch_rope_store_attention_regions(float*, float*, const float*, int8_t*, int8_t*, float*, float*, int16_t*,
                                          const int*, int, int, int, int, float, float, int, int, int, hipStream_t);
+bool t12_rope_store_prompt_attention(float*, float*, const float*, int8_t*, int8_t*, float*, float*, int16_t*, const int*, int,
+                                     int, int, int, int, float, float, const T12GemmPartials*, int, hipStream_t);
 void t12_rope_store_attention_copies(float*, float*, const float*, int8_t*, int8_t*, float*, float*, int16_t*, const int*,
                                      int, int, int, int, float, float, int, int, hipStream_t);
 void launch_rope_store_attention_partials_regions(float*, float*, const float*, int8_t*, int8_t*, float*, float*, int16_t*,
@@ -472,7 +474,9 @@ KvView kv_view(const InferenceState* state)
 // position of the rows (a length hint for the attention launch).  Logits: for every row into
 // state->logits (LOGITS_ALL), for the rows the request names, or not at all.
 // copies: the rows are copies of one sequence at one position on a shared cache (the lock-step batch of forward()).
-void forward_rows(InferenceState* state, int R, const KvView& kv, int pos0, const LogitsRequest& lr, bool copies = false)
+// first >= 0: the rows are positions first, first + 1 .. of one sequence.
+void forward_rows(InferenceState* state, int R, const KvView& kv, int pos0, const LogitsRequest& lr, bool copies = false,
+                  int first = -1)
 {
     Model* m = state->model;
     const ModelConfig& c = m->config;
@@ -511,7 +515,12 @@ void forward_rows(InferenceState* state, int R, const KvView& kv, int pos0, cons
         const size_t kv_off = (size_t)layer * kv.layer_kv;
         const size_t sc_off = (size_t)layer * kv.layer_sc;
         // RoPE (Q, K) + INT8 KV store + GQA attention
-        if (qkv_part.nsplit > 1 && kv.head_major)
+        if (first >= 0 && B > 1 &&
+            t12_rope_store_prompt_attention(state->q_buf, state->k_buf, state->v_buf, kv.k + kv_off, kv.v + kv_off,
+                                            kv.sk + sc_off, kv.sv + sc_off, bf16_a, state->d_positions, B, first, c.n_head,
+                                            c.n_head_kv, head_dim, c.rope_theta, scale, &qkv_part, kv.head_major, st))
+            ;
+        else if (qkv_part.nsplit > 1 && kv.head_major)
             launch_rope_store_attention_partials_regions(state->q_buf, state->k_buf, state->v_buf, kv.k + kv_off,
                                                          kv.v + kv_off, kv.sk + sc_off, kv.sv + sc_off, bf16_a,
                                                          state->d_positions, pos0, c.n_head, c.n_head_kv, head_dim,
@@ -677,7 +686,8 @@ void llama_prompt(InferenceState* state, const PromptPass& p)
         for (int r = 0; r < R; r++) pos[r] = p0 + done + r;
         (void)hipMemcpyAsync(w->d_tokens, p.tokens + done, R * sizeof(int), hipMemcpyHostToDevice, w->stream);
         (void)hipMemcpyAsync(w->d_positions, pos.data(), R * sizeof(int), hipMemcpyHostToDevice, w->stream);
-        forward_rows(w, R, kv, p0 + done + (R > 1 ? R - 1 : 0), pass_logits(p, done, R, taken, c.n_vocab, row_logits, picked));
+        forward_rows(w, R, kv, p0 + done + (R > 1 ? R - 1 : 0), pass_logits(p, done, R, taken, c.n_vocab, row_logits, picked),
+                     false, p0 + done);
         // pos[] is reused by the next pass: the copies above read it when they are issued (pageable memory)
         done += R;
     }

@@ -26,6 +26,12 @@
 #include "t12_device.h"
 #include "t12_host.h"
 
+extern "C" {
+bool t12_prompt_attention_takes(const float*, const int8_t*, const int8_t*, const int16_t*, int, int, int, int, int, float);
+void t12_prompt_attention(const float*, const int8_t*, const int8_t*, const float*, const float*, int16_t*, int, int, int, int, int,
+                          float, int, hipStream_t);
+}
+
 extern "C" void t12_rope_freqs(int head_dim, float theta, float factor, float low_freq_factor, float high_freq_factor,
                                float original_ctx, float* out);
 
@@ -1824,6 +1830,30 @@ static void rope_store_attention_partials(float* q, float* k, const float* v, in
                       QkvPartials{partials, nsplit, ld, split_stride}, (size_t)kv_stride, hm);
     launch_attn(q, kv_k, kv_v, scale_k, scale_v, output, positions, position + 1, n_head, n_head_kv, head_dim, scale,
                 batch_size, (size_t)kv_stride, stream, nullptr, hm);
+}
+
+// Library-internal (the engine's prompt passes): launch_rope_store_attention, or its form on partial sums (part.nsplit >
+// 1), for rows that are the consecutive positions first, first + 1 .. of ONE sequence; region_positions as above, 0 = the
+// reference's layout.  False, with nothing launched, where the row by row kernels are the better ones: below 64 workgroups
+// of 64 (row, head) pairs.  32 / 8 heads of 128, after 0 / 500 / 2000 positions: 128 rows 9.3 / 18.0 / 43.8 us against
+// 9.8 / 25.8 / 73.7, 64 rows 8.9 / 17.7 / 42.6 against 6.0 / 16.4 / 42.1, 16 rows 8.8 / 17.5 / 41.4 against 5.2 / 11.0 / 25.5.
+extern "C" __attribute__((visibility("hidden"))) bool t12_rope_store_prompt_attention(
+    float* q, float* k, const float* v, int8_t* kv_k, int8_t* kv_v, float* scale_k, float* scale_v, int16_t* output,
+    const int* positions, int rows, int first, int n_head, int n_head_kv, int head_dim, float theta, float scale,
+    const T12GemmPartials* part, int region_positions, hipStream_t stream)
+{
+    const int attn_mode_now = g_attn_mode.load(std::memory_order_relaxed);
+    if ((long long)rows * n_head < 4096 || !g_attn_fast || (attn_mode_now & (1 << 25))) return false;
+    if (!t12_prompt_attention_takes(q, kv_k, kv_v, output, rows, first, n_head, n_head_kv, head_dim, scale)) return false;
+    const bool sums = part->nsplit > 1;
+    launch_rope_kv<3>(q, k, v, kv_k, kv_v, scale_k, scale_v, positions, first, head_dim, n_head, n_head_kv,
+                      n_head * head_dim, n_head_kv * head_dim, theta, rows, stream,
+                      sums ? QkvPartials{part->ws, part->nsplit, part->ld, part->split_stride} : QkvPartials{nullptr, 0, 0, 0}, 0,
+                      region_positions);
+    t12_prompt_attention(q, kv_k, kv_v, scale_k, scale_v, output, rows, first, n_head, n_head_kv, head_dim, scale,
+                         region_positions, stream);
+    report("prompt attention");
+    return true;
 }
 
 void launch_rope_store_attention_partials(float* q, float* k, const float* v, int8_t* kv_k, int8_t* kv_v,
