@@ -127,3 +127,30 @@ def test_deferred_partial_sums_add_up_to_the_same_bits(t12):
     for z in range(part.nsplit):
         tot += ws.view(part.nsplit, B, part.ld)[z, :, :M]
     assert torch.equal(tot, want)
+
+
+@pytest.mark.parametrize("T,K,ff,one", [(9, 128, 257, False), (24, 384, 1000, False), (70, 640, 384, False), (20, 256, 2100, True), (64, 1152, 300, True)])
+def test_experts(t12, T, K, ff, one):
+    """The launch over experts, whose rows are counted on the device: 1 / 2 / 4 batch tiles by the hint, experts without
+    rows, every token at one expert (several passes of its batch tiles).  Gate and up sums are as above; their unit is
+    rounded to bf16, where a value may differ by one place: 2^-8 of the output's norm."""
+    from turbo_lossless_amd import moe
+    E, k = 8, 2
+    Ws = [[weight(M, Kc, 100 * e + i, 2e-3 if e % 2 else 2e-2, 0.05) for i, (M, Kc) in enumerate(((ff - ff % 64 + 64, K),) * 2 + ((K, ff - ff % 64 + 64),))]
+          for e in range(E)]
+    X = acts(T, K, T)
+    g = torch.Generator(device=dev()).manual_seed(7 + T)
+    ids = torch.stack([torch.randperm(E - 1, generator=g, device=dev())[:k] for _ in range(T)])         # the last expert has none
+    if one:
+        ids[:, 0], ids[:, 1] = 3, 4 * torch.arange(T, device=dev()) % 7
+        ids[:, 1] = torch.where(ids[:, 1] == 3, 5, ids[:, 1])
+    w = torch.rand((T, k), generator=g, device=dev())
+    layer = moe.MoeLayer([moe.Expert(*[t12.pack_device(m) for m in e]) for e in Ws])
+    got = layer(X.view(torch.int16), ids, w).double()
+    want = torch.zeros((T, K), dtype=torch.float64, device=dev())
+    for e in range(E):
+        a, b = X.double() @ Ws[e][0].double().T, X.double() @ Ws[e][1].double().T
+        h = (torch.nn.functional.silu(a) * b).to(torch.bfloat16).double()
+        share = torch.where(ids == e, w, torch.zeros_like(w)).sum(1).double()
+        want += share[:, None] * (h @ Ws[e][2].double().T)
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -8

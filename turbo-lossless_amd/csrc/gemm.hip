@@ -1727,11 +1727,23 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
     p.npair = swiglu ? nseg / 2 : 1;
     if (!swiglu) p.blk_start[nseg] = tiles;
     hipStream_t st = (hipStream_t)stream;
+    // More than a few rows per group: the ring kernel, whose workgroups of 128 rows stream at the memory's rate.  Eight
+    // experts of 4096 / 14336, two per token, whole layer: 12 / 40 / 64 / 128 tokens 340 / 359 / 372 / 425 us, 458 / 462 /
+    // 478 / 502 through the tile kernel; 8 tokens (hint 8) 285 against 398 by the sweep below.  It stops at a hint of 6: with
+    // a few of many small experts named there are too few workgroups (64 experts of 2048 / 1408, six per token: 4 tokens,
+    // hint 3, 236 us against the sweep's 177, 16 tokens, hint 7, 245 against 309; 32 of 4096 / 768, hint 5: 186 against 179).
+    bool ring = !swiglu && hint_b > 6 && hint_b <= RING_MAX_B && K % RING_WC == 0;
+    for (int i = 0; i < nseg; i++) ring = ring && (uintptr_t)segs[i].sm % 16 == 0 && (uintptr_t)segs[i].gr % 16 == 0;
+    if (ring) {
+        p.kslice = K;
+        const int nbt = ring_batch_tiles(hint_b);
+        if (nbt == 1) return launch_ring<8, 1, 1, false, T12_ACT_NONE, true>(p, tiles, st);
+        if (nbt == 2) return launch_ring<8, 1, 2, false, T12_ACT_NONE, true>(p, tiles, st);
+        return launch_ring<8, 1, 4, false, T12_ACT_NONE, true>(p, tiles, st);
+    }
     if (!swiglu && hint_b <= 8 && K % 128 == 0) {
         // a few rows per group (a decode step of a mixture-of-experts model): bound by the weight stream, so the kernel
-        // that sweeps 16 whole rows per workgroup; groups without rows cost a workgroup's exit.  (Measured on the
-        // Mixtral shape: 1 token 0.16 ms against 0.25 through the tile kernel, 4 tokens 0.46 against 0.52; at 16
-        // tokens -- 4 rows per expert, hint 12 -- the tile kernel is level again: 0.52 against 0.55.)
+        // that sweeps 16 whole rows per workgroup; groups without rows cost a workgroup's exit
         int groups = 0;
         for (int i = 0; i < nseg; i++) {
             p.blk_start[i] = groups;

@@ -14,7 +14,8 @@
 //     the decoded one in its register; the entry behind it is read along with the planes.
 // Measured (28672 x 4096, us, B = 16 / 32 / 64): 34.4 / 34.3 / 39.9 = 5.1 / 5.1 / 4.4 TB/s; the whole-row sweep and the
 // tile kernel, which took these launches before, 44.3 / 46.9 / 48.2.  A plain read of the same planes in the same
-// order takes 27.5 .. 33.  4096 x 14336 (8 or 4 K slices, their sum not counted): 19.2 / 20.3 / 23.2, before 28.4 / 26.6 / 27.8.
+// order takes 27.5 .. 33.  Experts (DEV: a group's rows are read from device memory, batch tiles in a loop): gate|up and down
+// of eight of 4096 / 14336 at 40 tokens 232 + 118 us = 6.1 and 6.0 TB/s, the tile kernel 333 + 158.  4096 x 14336 (8 or 4 K slices, their sum not counted): 19.2 / 20.3 / 23.2, before 28.4 / 26.6 / 27.8.
 #pragma once
 #include <type_traits>
 
@@ -55,14 +56,15 @@ __device__ __forceinline__ uint32_t ring_read32(uint32_t at)
 
 // LDS of a workgroup: the planes' ring (two windows per wave), the activations' ring (three windows per K wave), the
 // escape list.
-template <int RW, int KW, int NBT>
+template <int RW, int KW, int NBT, bool DEV = false>
 struct RingLds {
     static constexpr int W = RW * KW * 2 * RING_W_BYTES;
     static constexpr int XWIN = 16 * NBT * RING_WC * 2;
     static constexpr int X = KW * XWIN;                                // one round's
     static constexpr int ROWS = 16 * RW;
     static constexpr int TABLE = ROWS + 4;                             // row offsets into the list
-    static constexpr int ROOM = (160 * 1024 - W - 3 * X - TABLE * 4) / 4;
+    // (a launch over experts has many rounds of workgroups: two per CU, so that one starts while the other streams)
+    static constexpr int ROOM = ((DEV && NBT <= 2 ? 80 : 160) * 1024 - W - 3 * X - TABLE * 4) / 4;
     static constexpr int CAP = ROOM > 8192 ? 8192 : (ROOM & ~63);      // escape entries held
     static_assert(CAP >= 1024, "room for the escapes of a tile");
     static_assert((KW - 1) * RW * NBT * 64 * 16 <= W, "the sums of the K waves reuse the rings");
@@ -73,7 +75,7 @@ template <int RW, int KW, int NBT, bool GLU, int EPI, bool DEV>
 __device__ __forceinline__ bool gemm_ring_body(const GemmParams& p, const int bt, uint8_t* const x0, uint8_t* const x1, uint8_t* const x2,
                                                uint8_t* const wr, int* const lrow, uint32_t* const lpat, t12_f32x4* const red)
 {
-    using L = RingLds<RW, KW, NBT>;
+    using L = RingLds<RW, KW, NBT, DEV>;
     constexpr int NT = RW * KW * 64, BP = 16 * NBT;
     constexpr int NXI = 4 * NBT;                              // activation copies of a window (4 rows of 256 bytes each)
     constexpr int NX = (NXI + RW - 1) / RW;                   // of them, per wave (the last may be one less)
@@ -447,10 +449,10 @@ __device__ __forceinline__ bool gemm_ring_body(const GemmParams& p, const int bt
 }
 
 template <int RW, int KW, int NBT, bool GLU = false, int EPI = T12_ACT_NONE, bool DEV = false>
-__global__ __launch_bounds__(RW * KW * 64) void gemm_ring_kernel(const GemmParams p)
+__global__ __launch_bounds__(RW * KW * 64, DEV && NBT <= 2 ? 4 : 2) void gemm_ring_kernel(const GemmParams p)
 {
     // (arrays of their own: the compiler then knows that a read of one needs no wait for copies into another)
-    using L = RingLds<RW, KW, NBT>;
+    using L = RingLds<RW, KW, NBT, DEV>;
     __shared__ __attribute__((aligned(16))) uint8_t x0[L::X], x1[L::X], x2[L::X], wr[L::W];
     __shared__ int lrow[L::TABLE];
     __shared__ uint32_t lpat[L::CAP];
