@@ -307,7 +307,9 @@ int t12_delta_rule(const T12DeltaRule* d, const float* in, const float* bias, in
     p.out_ld = out_ld;
     int rc;
     switch (d->dim_p) {
-        case 64: rc = launch_rule<4, 16>(p, st); break;
+        // (tokens between two barriers: handing a chunk over costs a wave that is alone on its SIMD about 1 us.  512 tokens, 16
+        // heads of 64: 81 us with 16, 66 us with 32, 100 KB of LDS; heads of 128 have room for 16)
+        case 64: rc = launch_rule<4, 32>(p, st); break;
         case 128: rc = launch_rule<8, 16>(p, st); break;
         case 256: rc = launch_rule<16, 0>(p, st); break;
         default: rc = launch_rule<32, 0>(p, st); break;
