@@ -154,3 +154,9 @@ def test_experts(t12, T, K, ff, one):
         share = torch.where(ids == e, w, torch.zeros_like(w)).sum(1).double()
         want += share[:, None] * (h @ Ws[e][2].double().T)
     assert float((got - want).norm() / want.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("Ms,K,B", [([8192, 64], 2048, 200), ([4224], 4096, 130), ([4224], 4096, 100), ([8576], 2048, 300), ([1100, 3124], 1152, 128)])
+def test_splits_that_would_be_a_few_workgroups_more_than_the_chip(t12, Ms, K, B):
+    """More than 64 rows, where the usual K split comes to 257 .. 288 workgroups: fewer slices, odd counts of them."""
+    check(t12, Ms, K, B, 2e-3)

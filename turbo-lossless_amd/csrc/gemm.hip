@@ -1331,6 +1331,17 @@ bool launch_dense16_mixed(GemmParams p, int nseg, int rg, hipStream_t st)
     return true;
 }
 
+#define NOALLOC_TOO_LARGE                                                                                          \
+    "t12_gemm_noalloc: this shape splits K %d ways and needs %zu bytes of partial sums, the fixed "               \
+    "workspace holds %zu (B %d x %d rows): use t12_gemm, or a smaller batch"
+
+// Slices that ks slices of whole windows of two stages come to.
+int t12_slices(int K, int ks)
+{
+    const int windows = (K + 2 * KC - 1) / (2 * KC), per = (windows + ks - 1) / ks;
+    return (windows + per - 1) / per;
+}
+
 // The body of t12_gemm / t12_gemm_deferred / t12_gemm_noalloc.  static_ws: the K-split partial sums go to the
 // library's fixed device array instead of a grown hipMalloc buffer, and a launch that needs more is refused.
 int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_stride, int out_stride, int K,
@@ -1422,10 +1433,7 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
     auto take_workspace = [&]() {
         const size_t need = (size_t)p.ksplit * B * m_total * sizeof(float);
         if (static_ws) {
-            T12_REQUIRE(need <= STATIC_WS_BYTES,
-                        "t12_gemm_noalloc: this shape splits K %d ways and needs %zu bytes of partial sums, the fixed "
-                        "workspace holds %zu (B %d x %d rows): use t12_gemm, or a smaller batch", p.ksplit, need, STATIC_WS_BYTES, B,
-                        m_total);
+            T12_REQUIRE(need <= STATIC_WS_BYTES, NOALLOC_TOO_LARGE, p.ksplit, need, STATIC_WS_BYTES, B, m_total);
             p.ws = static_workspace();
             if (!p.ws) {
                 t12_set_error("t12_gemm_noalloc: hipGetSymbolAddress of the fixed workspace failed");
@@ -1535,13 +1543,39 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         while (tiles * btiles * ks * 2 <= 256 + 32 && K / (ks * 2) >= 8 * KC && ks < T12_MAX_KSPLIT) ks *= 2;
         return ks;
     };
-    int ks = splits_for(B > 128 ? (B + 255) / 256 : 1);
+    const int btiles = B > 128 ? (B + 255) / 256 : 1, btiles128 = (B + 127) / 128, cus = device_cus();
+    int ks = splits_for(btiles);
     // A 256-row batch tile whose K slice is under 16 stages (O of the Llama layer: 32 row tiles, 8 splits of 512
     // columns) spends its time filling and draining, and leaves twice the partial sums: such a launch takes 128-row
     // batch tiles and half the splits (O at B = 256 32 -> 27.5 us with the reduction; down, whose slices are long,
     // 55 -> 58 us and QKV 34 -> 37 us the same way, so they keep the 256-row tile).
-    const bool tb128 = B > 128 && ks > 1 && K / ks < 16 * KC;
-    if (tb128) ks = splits_for((B + 127) / 128);
+    bool tb128 = B > 128 && ks > 1 && K / ks < 16 * KC;
+    const int ks_full = tb128 ? splits_for(btiles128) : ks;
+    if (static_ws) {
+        // what t12_gemm_noalloc refuses is said by the full split, whatever is taken below
+        p.ksplit = t12_slices(K, ks_full);
+        const size_t need = (size_t)p.ksplit * B * m_total * sizeof(float);
+        T12_REQUIRE(p.ksplit == 1 || need <= STATIC_WS_BYTES, NOALLOC_TOO_LARGE, p.ksplit, need, STATIC_WS_BYTES, B, m_total);
+    }
+    // A few workgroups more than CUs are a second round of everything: fewer slices then, by  rounds x (6.5 us + stages x c)
+    // + what the partial sums cost (2.5 us and 4 TB/s, as for the ring kernel), c = 0.95 us for a stage of 256 batch rows, 0.65
+    // for 128.  8256 x 2048 at B = 512: 260 workgroups of 2 slices 47.4 us and a reduction of 11, unsplit 38.0; 4224 x 4096:
+    // 264 of 4 slices 47.7, 3 slices 34.1; 8704 x 8192: 272 of 2 slices 138, unsplit 120.
+    const bool over = ks > 1 && tiles * btiles * ks > cus;
+    tb128 = tb128 && !over && tiles * btiles128 * ks_full <= cus;
+    if (tb128) ks = ks_full;
+    if (over) {
+        const int windows = (K + 2 * KC - 1) / (2 * KC);
+        float best = 1e30f;
+        for (int k = ks; k >= 1; k--) {
+            const int rounds = (tiles * btiles * k + cus - 1) / cus, per = (windows + k - 1) / k;
+            const float us = rounds * (6.5f + 2 * per * (B > 128 ? 0.95f : 0.65f)) + (k > 1 ? 2.5f + (float)k * B * m_total * 1e-6f : 0.0f);
+            if (us < best) {
+                best = us;
+                ks = k;
+            }
+        }
+    }
     int kslice = (((K + 2 * KC - 1) / (2 * KC) + ks - 1) / ks) * 2 * KC;      // whole windows of two stages
     ks = (K + kslice - 1) / kslice;
     p.ksplit = ks;
