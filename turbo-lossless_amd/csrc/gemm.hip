@@ -1079,11 +1079,11 @@ int launch_mfma(GemmParams& p, int tiles, hipStream_t st)
 }
 
 
-template <int RW, int KW, int NBT, bool GLU = false, int EPI = T12_ACT_NONE, bool DEV = false>
+template <int RW, int KW, int NBT, bool GLU = false, bool DEV = false>
 int launch_ring(GemmParams& p, int tiles, hipStream_t st)
 {
     const dim3 grid(tiles, DEV ? 1 : (p.B + 16 * NBT - 1) / (16 * NBT), p.ksplit);
-    hipLaunchKernelGGL((gemm_ring_kernel<RW, KW, NBT, GLU, EPI, DEV>), grid, dim3(RW * KW * 64), 0, st, p);
+    hipLaunchKernelGGL((gemm_ring_kernel<RW, KW, NBT, GLU, DEV>), grid, dim3(RW * KW * 64), 0, st, p);
     T12_CHECK_LAUNCH("t12_gemm(ring)");
     return T12_OK;
 }
@@ -1771,9 +1771,9 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
     if (ring) {
         p.kslice = K;
         const int nbt = ring_batch_tiles(hint_b);
-        if (nbt == 1) return launch_ring<8, 1, 1, false, T12_ACT_NONE, true>(p, tiles, st);
-        if (nbt == 2) return launch_ring<8, 1, 2, false, T12_ACT_NONE, true>(p, tiles, st);
-        return launch_ring<8, 1, 4, false, T12_ACT_NONE, true>(p, tiles, st);
+        if (nbt == 1) return launch_ring<8, 1, 1, false, true>(p, tiles, st);
+        if (nbt == 2) return launch_ring<8, 1, 2, false, true>(p, tiles, st);
+        return launch_ring<8, 1, 4, false, true>(p, tiles, st);
     }
     if (!swiglu && hint_b <= 8 && K % 128 == 0) {
         // a few rows per group (a decode step of a mixture-of-experts model): bound by the weight stream, so the kernel

@@ -70,8 +70,8 @@ struct RingLds {
     static_assert((KW - 1) * RW * NBT * 64 * 16 <= W, "the sums of the K waves reuse the rings");
 };
 
-// GLU: a wave's 16 rows are 8 rows of gate and the same 8 rows of up.  EPI: T12_ACT_* of every sum, stored as bf16.
-template <int RW, int KW, int NBT, bool GLU, int EPI, bool DEV>
+// GLU: a wave's 16 rows are 8 rows of gate and the same 8 rows of up.
+template <int RW, int KW, int NBT, bool GLU, bool DEV>
 __device__ __forceinline__ bool gemm_ring_body(const GemmParams& p, const int bt, uint8_t* const x0, uint8_t* const x1, uint8_t* const x2,
                                                uint8_t* const wr, int* const lrow, uint32_t* const lpat, t12_f32x4* const red)
 {
@@ -419,16 +419,6 @@ __device__ __forceinline__ bool gemm_ring_body(const GemmParams& p, const int bt
         return true;
     }
     const int m = wm0 + n;
-    if (EPI != T12_ACT_NONE) {
-#pragma unroll
-        for (int u = 0; u < NBT; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int b = b0 + 16 * u + 4 * g + r;
-                if (m < M && b < B) p.out_bf16[(size_t)b * p.out_bf16_ld + m] = t12_f32_to_bf16(t12_apply_act<EPI>(sum[u][r], p.act_a, p.act_b));
-            }
-        return true;
-    }
     float* dst;
     size_t ld;
     if (p.ksplit > 1) {
@@ -448,7 +438,7 @@ __device__ __forceinline__ bool gemm_ring_body(const GemmParams& p, const int bt
     return true;
 }
 
-template <int RW, int KW, int NBT, bool GLU = false, int EPI = T12_ACT_NONE, bool DEV = false>
+template <int RW, int KW, int NBT, bool GLU = false, bool DEV = false>
 __global__ __launch_bounds__(RW * KW * 64, DEV && NBT <= 2 ? 4 : 2) void gemm_ring_kernel(const GemmParams p)
 {
     // (arrays of their own: the compiler then knows that a read of one needs no wait for copies into another)
@@ -457,7 +447,7 @@ __global__ __launch_bounds__(RW * KW * 64, DEV && NBT <= 2 ? 4 : 2) void gemm_ri
     __shared__ int lrow[L::TABLE];
     __shared__ uint32_t lpat[L::CAP];
     for (int bt = blockIdx.y;; bt++) {
-        if (!gemm_ring_body<RW, KW, NBT, GLU, EPI, DEV>(p, bt, x0, x1, x2, wr, lrow, lpat, (t12_f32x4*)wr) || !DEV) break;
+        if (!gemm_ring_body<RW, KW, NBT, GLU, DEV>(p, bt, x0, x1, x2, wr, lrow, lpat, (t12_f32x4*)wr) || !DEV) break;
         __syncthreads();                                   // the next tile reuses the rings
     }
 }
