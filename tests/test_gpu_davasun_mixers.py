@@ -404,6 +404,28 @@ def test_gated_units(t12):
             assert rel_err(host(out), want) < (1e-6 if fp32 else 5e-3)
 
 
+@pytest.mark.parametrize("slope, offset, limit", [(1.0, 0.0, float("inf")), (1.702, 1.0, 7.0)])
+def test_gated_units_over_their_range(t12, slope, offset, limit):
+    """g sigmoid(slope g) (u + offset) in 32 bits against 64: one unit (2^-23) each for the power of two and the reciprocal with its Newton
+    step, half a unit for the sum, both products and u + offset: four in all.  Values that 32 bits cannot hold normalised come out within
+    2^-126 u g; infinities and NaN as in the plain formula."""
+    g = np.concatenate([np.linspace(-90, 90, 36001), np.geomspace(1e-30, 60, 4001), -np.geomspace(1e-30, 60, 4001),
+                        [0.0, -0.0, -87.0, -88.0, -89.0, -104.0, -1e4, -3e38, 3e38, np.inf, -np.inf, np.nan]]).astype(np.float32)
+    u = np.resize(np.array([1.0, -0.75, 3.5], np.float32), g.size)
+    gd, ud, out = up(g), up(u), torch.empty(g.size, device=dev())
+    t12.check(t12.lib.t12_glu(gd.data_ptr(), ud.data_ptr(), C.byref(t12.Glu(limit, slope, offset)), out.data_ptr(), 1, g.size, t12.current_stream()))
+    with np.errstate(all="ignore"):
+        gg = np.fmin(g, np.float32(limit)).astype(np.float64)
+        x = (np.float32(slope) * np.fmin(g, np.float32(limit))).astype(np.float64)
+        v = np.clip(u, -limit, limit).astype(np.float64) + offset
+        want = np.where(np.isneginf(gg), np.nan, gg / (1 + np.exp(-x)) * v)
+        got = host(out).astype(np.float64)
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        gap = np.abs(got[fin] - want[fin]) - 4 * 2.0 ** -23 * np.abs(want[fin])
+        assert (gap <= 2.0 ** -125 * np.abs(v[fin]) * np.maximum(1, np.minimum(np.abs(gg[fin]), 200))).all(), gap.max()
+
+
 @pytest.mark.parametrize("M, K", [(96, 64), (130, 1024), (64, 2064), (1000, 4096)])
 def test_gated_decode_gemv(t12, oracle, M, K):
     rng = np.random.default_rng(M + K)
