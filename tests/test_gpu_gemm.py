@@ -51,6 +51,37 @@ def test_gemm_shapes(t12, oracle, synth, M, K, B):
     assert rel_err(un, oracle.gemm(p, X, patched=False)) < TOL
 
 
+@pytest.mark.parametrize("B", [65, 200, 260])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 448])
+def test_gemm_few_stages(t12, oracle, synth, K, B):
+    """As few stages of 64 columns as the tile kernel requests ahead, and fewer; half a window at the end of the last row; a list that takes
+    a workgroup's threads more than one entry each."""
+    M = 257
+    p = oracle.pack(synth.weights_llm(M, K, seed=K, p_outlier=3e-2))
+    X = synth.activations(B, K, seed=B)
+    (got,) = run_gemm(t12, [p], X)
+    assert rel_err(got, oracle.gemm(p, X)) < TOL
+
+
+@pytest.mark.parametrize("patched", [(True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("M, K, B", [(12300, 192, 70), (12300, 320, 200)])
+def test_gemm_swiglu_with_one_list(t12, synth, M, K, B, patched):
+    g = torch.Generator(device=dev()).manual_seed(K)
+    pair = []
+    for k in range(2):
+        w = torch.randn((M, K), generator=g, device=dev()) * 0.02
+        pair.append(t12.pack_device(torch.where(torch.rand((M, K), generator=g, device=dev()) < 2e-3, 8.0, w).to(torch.bfloat16)))
+    X = torch.randn((B, K), generator=g, device=dev()).to(torch.bfloat16).view(torch.int16)
+    outs = [torch.empty((B, M), device=dev()) for _ in range(2)]
+    segs = [w.segment(o, use) for w, o, use in zip(pair, outs, patched)]
+    st = t12.current_stream()
+    t12.check(t12.lib.t12_gemm(t12._seg_array(segs), 2, X.data_ptr(), K, M, K, B, st))
+    want, got = (torch.empty((B, M), dtype=torch.int16, device=dev()) for _ in range(2))
+    t12.lib.launch_silu_mul_bf16_batch(outs[0].data_ptr(), outs[1].data_ptr(), want.data_ptr(), M, B, st)
+    assert t12.lib.t12_gemm_swiglu(t12._seg_array(segs[:1]), t12._seg_array(segs[1:]), X.data_ptr(), K, K, B, got.data_ptr(), M, st) == 0
+    assert torch.equal(got, want)
+
+
 def test_gemm_every_k_split(t12, oracle, synth):
     """One row tile (M = 128): the launch splits K across workgroups as far as its rule allows, so the length of K
     picks the number of splits.  The number the library chose is read back through t12_gemm_deferred; every count from

@@ -61,6 +61,17 @@ constexpr int PCAP = 2048;      // escape entries a workgroup can stage in LDS
 constexpr int PATCH_BYTES = PCAP * 4 + (TM + 1) * 4 + 12;
 constexpr int NO_ESCAPE = 0x7FFFFFFF;
 
+// How far apart two arrays lie, one value in the wave.  A lane that picks one of the two tensors of a pair adds it or not: between the
+// pointers themselves the compiler would choose a pointer to load, a chain of loads per lane.
+__device__ __forceinline__ int64_t apart(const void* a, const void* b)
+{
+    const uint64_t d = (uint64_t)(uintptr_t)b - (uint64_t)(uintptr_t)a;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)d), hi = __builtin_amdgcn_readfirstlane((uint32_t)(d >> 32));
+    return (int64_t)((uint64_t)hi << 32 | lo);
+}
+// A word that is one value in the wave and that no kernel in flight writes.
+__device__ __forceinline__ int scalar_load(const int* p) { return *(const __attribute__((address_space(4))) int*)(uintptr_t)p; }
+
 // LDS slot of (unit, row) in a [units][rows] array of 16-byte units.  Rows are rotated
 // inside their aligned block of eight by the unit index, so that both access patterns are
 // bank-conflict free: the staging writes (neighbouring lanes = the units of one row) and
@@ -106,7 +117,7 @@ __device__ __forceinline__ constexpr int stage_unit_order(int pos, int nact, int
 // (engine/kernels.hip:447-459) and the fp32 round trip of both projections folded away.
 // EPI (T12_ACT_*, one segment, no K split): the unary function of every sum is stored as bf16 to out_bf16.
 // bt: batch tile.  Returns false when the tile lies past the segment's rows (nothing was done).
-template <int WB, int WM, int FB, int FM, bool SWI = false, int EPI = T12_ACT_NONE>
+template <int WB, int WM, int FB, int FM, bool SWI, int EPI, bool DEV>
 __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt)
 {
     static_assert(!SWI || FM == 2, "the SwiGLU epilogue pairs the two row tiles of a wave");
@@ -129,26 +140,22 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
     const int pair = SWI ? find_pair(p, tile) : 0;
     const int s = SWI ? 2 * pair : find_segment(p, tile);          // SWI: the gate segment of the tile's pair
     const T12Segment& sg = p.seg[s];
+    const T12Segment& sg1 = p.seg[SWI ? s + 1 : s];
     const int M = sg.M, K = p.K;
-    const int B = p.dev_counts ? p.dev_counts[p.group_of_seg[s]] : p.seg_B[s];
-    const int row_base = p.dev_base ? p.dev_base[p.group_of_seg[s]] : 0;     // first row of this group in act / out
+    const int B = DEV ? p.dev_counts[p.group_of_seg[s]] : p.seg_B[s];
+    const int row_base = DEV ? p.dev_base[p.group_of_seg[s]] : 0;            // first row of this group in act / out
     const int act_stride = p.seg_act_stride[s];
     const uint16_t* const act = p.seg_act[s] + (size_t)row_base * act_stride;
     if (bt * (WB * FB * 32) >= B) return false;            // grouped launch: this segment has fewer batch tiles than the grid
     const int m0 = SWI ? (tile - p.blk_start[pair]) * (TM / 2) : (tile - p.blk_start[s]) * TM;
-    // local row r of the tile -> segment and matrix row
-    auto row_seg = [&](int r) { return SWI ? s + ((r >> 5) & 1) : s; };
+    // local row r of the tile -> matrix row
     auto row_mat = [&](int r) { return SWI ? m0 + ((r >> 6) << 5) + (r & 31) : m0 + r; };
     const int b0 = bt * TB;
     const int k_begin = blockIdx.z * p.kslice;
     const int k_end = min(K, k_begin + p.kslice);
     const int nstage = (k_end - k_begin) / KC;
-    uint32_t be2s[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int be = p.seg[SWI ? s + j : s].base_exp;
-        be2s[j] = t12_opaque(((uint32_t)be << 7) | ((uint32_t)be << 23));
-    }
+    const int be0 = __builtin_amdgcn_readfirstlane(sg.base_exp), be1 = __builtin_amdgcn_readfirstlane(sg1.base_exp);
+    const int64_t sm_apart = SWI ? apart(sg.sm, sg1.sm) : 0, gr_apart = SWI ? apart(sg.gr, sg1.gr) : 0;
 
     // ---- this thread's share of the global -> LDS staging
     //  acts: item idx = tid + NT*i -> batch row idx / 8, unit idx % 8 (8 lanes = 128 contiguous bytes)
@@ -176,12 +183,13 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
 #pragma unroll
         for (int y = 0; y < 2; y++) {
             const int r = (hi ^ y) ? r_hi : r_lo;
-            const T12Segment& g = p.seg[row_seg(r)];
+            const bool second = SWI && ((r >> 5) & 1);
             const size_t e = (size_t)min(row_mat(r), M - 1) * K + k_begin + 64 * y + 16 * cc;
             w_row[y][i] = r;
-            w_be2[y][i] = be2s[SWI ? (r >> 5) & 1 : 0];
-            s_src[y][i] = g.sm + e;
-            g_src[y][i] = g.gr + (e >> 1);
+            const uint32_t be = second ? be1 : be0;
+            w_be2[y][i] = t12_opaque((be << 7) | (be << 23));
+            s_src[y][i] = sg.sm + ((second ? sm_apart : 0) + (int64_t)e);
+            g_src[y][i] = sg.gr + ((second ? gr_apart : 0) + (int64_t)(e >> 1));
             w_dst[y][i][0] = ACT_UNITS * 16 + lds_slot(2 * cc, r, TM) * 16;
             w_dst[y][i][1] = ACT_UNITS * 16 + lds_slot(2 * cc + 1, r, TM) * 16;
         }
@@ -232,35 +240,76 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
     //      their entries are one contiguous slice [e0, e1) of cols[] / correct[].
     //      esc_mode: 0 none, 1 staged (exact values written over the decoded ones in LDS),
     //      2 too many for LDS (or K > 65536): wrong values multiplied, corrected in the epilogue.
+    //      What a workgroup waits for before its first product is a chain of loads, 1 us each: the rows' offsets, the
+    //      list, the tiles.  So the ends of the slice come by scalar loads, every row's offset and the first stages'
+    //      tiles are requested along with them, the list behind the first two stages' tiles, and the rest of the tiles
+    //      behind the list (4096 x 4096 at B = 100 / 256, 8 / 4 slices: 18.5 / 23.3 -> 17.0 / 22.5 us).
     uint32_t* lpat = (uint32_t*)(lds + 2 * STAGE_BYTES);       // col | correct << 16
     int* lrow = (int*)(lpat + PCAP);                           // [TM + 1] offsets into lpat (SWI: [2][TM/2 + 1])
+    constexpr int ER = SWI ? TM / 2 : TM;                      // rows of a tensor
+    const bool has0 = sg.row_off, has1 = SWI && sg1.row_off;
     int esc_mode = 0;
-    if (SWI) {
-        // two slices: the 64 gate rows, then the 64 up rows
-        const T12Segment& g0 = p.seg[s];
-        const T12Segment& g1 = p.seg[s + 1];
-        const int r_lo = min(m0, M), r_hi = min(m0 + TM / 2, M);
-        const int e00 = g0.row_off ? g0.row_off[r_lo] : 0, e10 = g1.row_off ? g1.row_off[r_lo] : 0;
-        const int n0 = g0.row_off ? g0.row_off[r_hi] - e00 : 0, n1 = g1.row_off ? g1.row_off[r_hi] - e10 : 0;
-        if (g0.row_off || g1.row_off) esc_mode = (n0 + n1 <= PCAP && K <= 65536) ? 1 : 2;
-        if (esc_mode == 1) {
-            for (int t = tid; t < n0; t += NT)
-                lpat[t] = (uint32_t)g0.cols[e00 + t] | ((uint32_t)(uint16_t)g0.correct[e00 + t] << 16);
-            for (int t = tid; t < n1; t += NT)
-                lpat[n0 + t] = (uint32_t)g1.cols[e10 + t] | ((uint32_t)(uint16_t)g1.correct[e10 + t] << 16);
-            for (int t = tid; t <= TM / 2; t += NT) {
-                lrow[t] = g0.row_off ? g0.row_off[min(m0 + t, M)] - e00 : 0;
-                lrow[TM / 2 + 1 + t] = n0 + (g1.row_off ? g1.row_off[min(m0 + t, M)] - e10 : 0);
+    int e00 = 0, e10 = 0, n0 = 0, n1 = 0;                      // first entry and number of entries, per tensor
+    int my_off = 0;                                            // thread t: offset of row t (SWI: of up's row t - ER - 1)
+    if (has0 || has1) {
+        // (a tensor without a list: any readable address)
+        const int* r0 = has0 ? sg.row_off : (const int*)sg.sm;
+        const int* r1 = has1 ? sg1.row_off : (const int*)sg.sm;
+        const int lo = min(m0, M), hi = min(m0 + ER, M);
+        e00 = scalar_load(r0 + (has0 ? lo : 0));
+        n0 = scalar_load(r0 + (has0 ? hi : 0));
+        e10 = scalar_load(r1 + (has1 ? lo : 0));
+        n1 = scalar_load(r1 + (has1 ? hi : 0));
+        if (SWI && tid > ER) {
+            if (has1 && tid <= 2 * ER + 1) my_off = sg1.row_off[min(m0 + tid - ER - 1, M)];
+        } else if (has0 && tid <= ER) {
+            my_off = sg.row_off[min(m0 + tid, M)];
+        }
+    }
+    // window w (0 or 1) of the slice; what lies past its end is not used: the last window, or its first half, again
+    auto load_first = [&](int w) {
+        const int win = min(w, (nstage - 1) / 2), back = 2 * win + 1 < nstage ? 0 : KC;
+#pragma unroll
+        for (int i = 0; i < W_LD; i++)
+#pragma unroll
+            for (int y = 0; y < 2; y++) {
+                rs[w][y][i] = *(const uint4*)(s_src[y][i] + win * (2 * KC) - y * back);
+                rg[w][y][i] = *(const uint2*)(g_src[y][i] + ((win * (2 * KC) - y * back) >> 1));
             }
+    };
+    // (in the order in which the loop requests them, so that its waits count the same loads on the way in and around)
+#pragma unroll
+    for (int d = 0; d < 2; d++)
+#pragma unroll
+        for (int u = 0; u < ACT_LD; u++) load_act(d, min(d, nstage - 1), u);
+    load_first(0);
+    if (has0 || has1) {
+        n0 = has0 ? n0 - e00 : 0;
+        n1 = has1 ? n1 - e10 : 0;
+        esc_mode = (n0 + n1 <= PCAP && K <= 65536) ? 1 : 2;
+    }
+    const int64_t cols_apart = SWI ? apart(sg.cols, sg1.cols) : 0, exact_apart = SWI ? apart(sg.correct, sg1.correct) : 0;
+    auto list_entry = [&](int t, uint32_t& col, uint32_t& exact) {
+        const bool second = SWI && t >= n0;
+        const int64_t e = second ? e10 + t - n0 : e00 + t;
+        col = *(const uint32_t*)((const uint8_t*)sg.cols + ((second ? cols_apart : 0) + 4 * e));
+        exact = *(const uint16_t*)((const uint8_t*)sg.correct + ((second ? exact_apart : 0) + 2 * e));
+    };
+    uint32_t col = (uint32_t)my_off, exact = col;              // (any value: a constant would draw the shift below, and a wait, into the branch)
+    if (esc_mode == 1 && tid < n0 + n1) list_entry(tid, col, exact);
+#pragma unroll
+    for (int d = 2; d < DA; d++)
+#pragma unroll
+        for (int u = 0; u < ACT_LD; u++) load_act(d, min(d, nstage - 1), u);
+    load_first(1);
+    if (esc_mode == 1) {
+        if (tid < n0 + n1) lpat[tid] = col | exact << 16;
+        for (int t = tid + NT; t < n0 + n1; t += NT) {
+            list_entry(t, col, exact);
+            lpat[t] = col | exact << 16;
         }
-    } else if (sg.row_off) {
-        const int e0 = sg.row_off[min(m0, M)], e1 = sg.row_off[min(m0 + TM, M)];
-        esc_mode = (e1 - e0 <= PCAP && K <= 65536) ? 1 : 2;
-        if (esc_mode == 1) {
-            for (int t = tid; t < e1 - e0; t += NT)
-                lpat[t] = (uint32_t)sg.cols[e0 + t] | ((uint32_t)(uint16_t)sg.correct[e0 + t] << 16);
-            for (int t = tid; t <= TM; t += NT) lrow[t] = sg.row_off[min(m0 + t, M)] - e0;
-        }
+        if (tid <= ER) lrow[tid] = has0 ? my_off - e00 : 0;
+        else if (SWI && tid <= 2 * ER + 1) lrow[tid] = n0 + (has1 ? my_off - e10 : 0);
     }
     // Per piece kind and item: cursor into its row's slice and the column of the next entry.  The
     // thread that decoded 16 columns of a row into LDS also overwrites the escapes among them
@@ -356,18 +405,7 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
         __syncthreads();
     };
 
-    // prologue: activation stages 0..3 and weight windows 0, 1 in flight, escape list visible,
-    // stage 0 into LDS
-#pragma unroll
-    for (int d = 0; d < DA; d++)
-        if (d < nstage) {
-#pragma unroll
-            for (int u = 0; u < ACT_LD; u++) load_act(d, d, u);
-        }
-#pragma unroll
-    for (int w = 0; w < 2; w++)
-#pragma unroll
-        for (int u = 0; u < 4 * W_LD; u++) load_w(w, w, u, 2 * w < nstage, 2 * w + 1 < nstage);
+    // escape list visible, stage 0 into LDS
     __syncthreads();
     if (esc_mode == 1) {
 #pragma unroll
@@ -384,11 +422,6 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
                 if (q < qe) nc[y][i] = (int)(lpat[q] & 0xFFFFu);
             }
     }
-    // All prologue loads have landed before the loop is entered: the compiler's wait-count
-    // bookkeeping then sees only the loop's own loads at the loop head and waits for exactly
-    // the ring slot it needs (with loads pending across the entry edge it drains all of them
-    // once per trip).
-    __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0)
     if (nstage > 0) {
 #pragma unroll
         for (int u = 0; u < NSU; u++) store_unit(0, 0, 0, 0, u);
@@ -496,11 +529,11 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
 // Batch tiles: one per workgroup (blockIdx.y), except when the rows per group are known on the device only: such
 // a launch has one workgroup per row tile, which takes the group's batch tiles one after the other (a group within
 // the tile -- the usual case -- is streamed once, a larger one once per tile; no group's rows can fall outside the grid).
-template <int WB, int WM, int FB, int FM, bool SWI = false, int EPI = T12_ACT_NONE>
+template <int WB, int WM, int FB, int FM, bool SWI = false, int EPI = T12_ACT_NONE, bool DEV = false>
 __global__ __launch_bounds__(WB * WM * 64) void gemm_mfma_kernel(const GemmParams p)
 {
     for (int bt = blockIdx.y;; bt++) {
-        if (!gemm_mfma_body<WB, WM, FB, FM, SWI, EPI>(p, bt) || !p.dev_counts) break;
+        if (!gemm_mfma_body<WB, WM, FB, FM, SWI, EPI, DEV>(p, bt) || !DEV) break;
         __syncthreads();                                   // the next tile reuses the staging buffers
     }
 }
@@ -1049,13 +1082,13 @@ float* static_workspace()
 }
 
 
-template <int WB, int WM, int FB, int FM, bool SWI = false, int EPI = T12_ACT_NONE>
+template <int WB, int WM, int FB, int FM, bool SWI = false, int EPI = T12_ACT_NONE, bool DEV = false>
 int launch_mfma(GemmParams& p, int tiles, hipStream_t st)
 {
     constexpr int TB = WB * FB * 32;
     constexpr int STAGE_BYTES = TB * 8 * 16 + TM * 128;
     const dim3 grid(tiles, (p.B + TB - 1) / TB, p.ksplit);   // batch tiles of one row tile are neighbours in time
-    auto kfn = gemm_mfma_kernel<WB, WM, FB, FM, SWI, EPI>;
+    auto kfn = gemm_mfma_kernel<WB, WM, FB, FM, SWI, EPI, DEV>;
     static bool attr_done[16] = {};                    // the attribute is per device
     static std::mutex attr_mutex;
     int dev = 0;
@@ -1788,12 +1821,12 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
         return T12_OK;
     }
     if (swiglu) {
-        if (hint_b <= 128) return launch_mfma<4, 2, 1, 2, true>(p, tiles, st);
-        return launch_mfma<4, 2, 2, 2, true>(p, tiles, st);
+        if (hint_b <= 128) return launch_mfma<4, 2, 1, 2, true, T12_ACT_NONE, true>(p, tiles, st);
+        return launch_mfma<4, 2, 2, 2, true, T12_ACT_NONE, true>(p, tiles, st);
     }
-    if (hint_b <= 64) return launch_mfma<2, 4, 1, 1>(p, tiles, st);
-    if (hint_b <= 128) return launch_mfma<2, 4, 2, 1>(p, tiles, st);
-    return launch_mfma<4, 2, 2, 2>(p, tiles, st);
+    if (hint_b <= 64) return launch_mfma<2, 4, 1, 1, false, T12_ACT_NONE, true>(p, tiles, st);
+    if (hint_b <= 128) return launch_mfma<2, 4, 2, 1, false, T12_ACT_NONE, true>(p, tiles, st);
+    return launch_mfma<4, 2, 2, 2, false, T12_ACT_NONE, true>(p, tiles, st);
 }
 
 // The library keeps device buffers per (device, stream): the K-split partial sums of t12_gemm*, the argmax partials and the
