@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 import numpy as np
 
@@ -272,7 +273,12 @@ def _torch():
 
 
 def current_stream() -> int:
-    return _torch().cuda.current_stream().cuda_stream
+    """torch's current stream on the current device, as the handle the C ABI takes.  (Without a Stream object around it: 0.3 us
+    against 3.0, a third of what one small product costs the host.)"""
+    torch = _torch()
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dp(t):
@@ -317,6 +323,24 @@ def _seg_array(segs):
     return arr
 
 
+_SEGMENT = struct.Struct("7Q4i")
+assert _SEGMENT.size == C.sizeof(Segment)
+
+
+def _segments(tensors, outs, patched):
+    """_seg_array of the tensors' segments, packed as bytes: 0.6 us a tensor where a Structure takes 1.3."""
+    if any(type(t) is not DeviceTensor12 for t in tensors):
+        return _seg_array([t.segment(o, patched) for t, o in zip(tensors, outs)])
+    raw = []
+    for t, o in zip(tensors, outs):
+        lists = (0, 0, 0, 0)
+        if patched and t.row_off is not None and t.P > 0:            # no escapes: no list
+            lists = (t.row_off.data_ptr(), t.cols.data_ptr(), t.correct.data_ptr(), t.wrong.data_ptr())
+        raw.append(_SEGMENT.pack(t.sm.data_ptr(), t.gr.data_ptr(), *lists, o.data_ptr(), t.M, t.base_exp,
+                                 o.stride(0) if o.dim() == 2 else 0, 0))
+    return (Segment * len(raw)).from_buffer_copy(b"".join(raw))
+
+
 def gemv(tensors, act, outs=None, patched=True, stream=None):
     """Fused decode-GEMV (B = 1) over one or more tensors sharing `act` (bf16 [K])."""
     torch = _torch()
@@ -325,7 +349,7 @@ def gemv(tensors, act, outs=None, patched=True, stream=None):
     K = tensors[0].K
     if outs is None:
         outs = [torch.empty(t.M, dtype=torch.float32, device=act.device) for t in tensors]
-    segs = _seg_array([t.segment(o, patched) for t, o in zip(tensors, outs)])
+    segs = _segments(tensors, outs, patched)
     st = current_stream() if stream is None else stream
     check(lib.t12_gemv(segs, len(tensors), act.data_ptr(), K, st), "t12_gemv")
     return outs
@@ -341,7 +365,7 @@ def gemm(tensors, X, outs=None, patched=True, stream=None):
     if outs is None:
         outs = [torch.empty((B, t.M), dtype=torch.float32, device=X.device) for t in tensors]
     stride = outs[0].stride(0)      # every segment carries its own stride; this is the default
-    segs = _seg_array([t.segment(o, patched) for t, o in zip(tensors, outs)])
+    segs = _segments(tensors, outs, patched)
     st = current_stream() if stream is None else stream
     check(lib.t12_gemm(segs, len(tensors), X.data_ptr(), X.stride(0), stride, K, B, st), "t12_gemm")
     return outs
