@@ -15,32 +15,30 @@
 
 namespace {
 
-// 16 elements per lane per step; n16 = number of whole 16-element pieces.
+// Eight elements per lane and step (whole lines of loads and stores per wave), two steps in flight; n16 = number of whole 16-element pieces.
 __global__ __launch_bounds__(256) void decompress_vec_kernel(const uint8_t* __restrict__ sm,
                                                              const uint8_t* __restrict__ gr,
                                                              uint32_t be2, uint16_t* __restrict__ out,
                                                              size_t n16)
 {
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    const size_t n8 = n16 * 2, stride = (size_t)gridDim.x * 512;
     be2 = t12_opaque(be2);
-    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n16; q += stride) {
-        const uint4 S = t12_ldg_stream16(sm + q * 16);
-        const uint2 G = t12_ldg_stream8(gr + q * 8);
-        uint32_t a[4], b[4];
-        t12_decode8(S.x, S.y, G.x, be2, a);     // a[i] = {w[i+4], w[i]}
-        t12_decode8(S.z, S.w, G.y, be2, b);
-        uint4 o0, o1;
-        o0.x = __builtin_amdgcn_perm(a[1], a[0], 0x05040100u);   // {w1, w0}
-        o0.y = __builtin_amdgcn_perm(a[3], a[2], 0x05040100u);   // {w3, w2}
-        o0.z = __builtin_amdgcn_perm(a[1], a[0], 0x07060302u);   // {w5, w4}
-        o0.w = __builtin_amdgcn_perm(a[3], a[2], 0x07060302u);   // {w7, w6}
-        o1.x = __builtin_amdgcn_perm(b[1], b[0], 0x05040100u);
-        o1.y = __builtin_amdgcn_perm(b[3], b[2], 0x05040100u);
-        o1.z = __builtin_amdgcn_perm(b[1], b[0], 0x07060302u);
-        o1.w = __builtin_amdgcn_perm(b[3], b[2], 0x07060302u);
-        uint4* dst = (uint4*)(out + q * 16);
-        t12_stg_stream16(dst, o0);
-        t12_stg_stream16(dst + 1, o1);
+    for (size_t q0 = (size_t)blockIdx.x * 512 + threadIdx.x; q0 < n8; q0 += stride) {
+        const size_t q1 = q0 + 256;
+        const bool two = q1 < n8;
+        uint2 S[2] = {t12_ldg_stream8(sm + q0 * 8), make_uint2(0, 0)};
+        uint32_t G[2] = {__builtin_nontemporal_load((const uint32_t*)(gr + q0 * 4)), 0};
+        if (two) {
+            S[1] = t12_ldg_stream8(sm + q1 * 8);
+            G[1] = __builtin_nontemporal_load((const uint32_t*)(gr + q1 * 4));
+        }
+        uint32_t a[4];
+        t12_decode8_seq(S[0].x, S[0].y, G[0], be2, a);
+        t12_stg_stream16(out + q0 * 8, make_uint4(a[0], a[1], a[2], a[3]));
+        if (two) {
+            t12_decode8_seq(S[1].x, S[1].y, G[1], be2, a);
+            t12_stg_stream16(out + q1 * 8, make_uint4(a[0], a[1], a[2], a[3]));
+        }
     }
 }
 
@@ -63,35 +61,27 @@ __global__ __launch_bounds__(256) void decompress_patched_kernel(const uint8_t* 
     // the slice of the list is requested before the planes: it is used last
     const int e0 = row_off[r_lo], e1 = row_off[r_hi + 1];
     be2 = t12_opaque(be2);
-    uint4 S[PIECES];
-    uint2 G[PIECES];
+    // Units of eight elements, unit u * 256 + thread: both loads and the 16-byte store of a unit are whole lines of a wave.  (Pieces of 16
+    // per lane store 16 bytes in every 32: 14336 x 4096, buffers changing, 40.1 us, this 36.4; into one that the cache holds 41.1, 31.1.)
+    constexpr int UNITS = PIECES * 2;
+    const size_t n8 = n16 * 2, first = (size_t)blockIdx.x * (256 * UNITS) + threadIdx.x;
+    uint2 S[UNITS];
+    uint32_t G[UNITS];
 #pragma unroll
-    for (int u = 0; u < PIECES; u++) {
-        const size_t q = (size_t)blockIdx.x * (256 * PIECES) + u * 256 + threadIdx.x;
-        if (q < n16) {
-            S[u] = t12_ldg_stream16(sm + q * 16);
-            G[u] = t12_ldg_stream8(gr + q * 8);
+    for (int u = 0; u < UNITS; u++) {
+        const size_t q = first + u * 256;
+        if (q < n8) {
+            S[u] = t12_ldg_stream8(sm + q * 8);
+            G[u] = __builtin_nontemporal_load((const uint32_t*)(gr + q * 4));
         }
     }
 #pragma unroll
-    for (int u = 0; u < PIECES; u++) {
-        const size_t q = (size_t)blockIdx.x * (256 * PIECES) + u * 256 + threadIdx.x;
-        if (q < n16) {
-            uint32_t a[4], b[4];
-            t12_decode8(S[u].x, S[u].y, G[u].x, be2, a);
-            t12_decode8(S[u].z, S[u].w, G[u].y, be2, b);
-            uint4 o0, o1;
-            o0.x = __builtin_amdgcn_perm(a[1], a[0], 0x05040100u);
-            o0.y = __builtin_amdgcn_perm(a[3], a[2], 0x05040100u);
-            o0.z = __builtin_amdgcn_perm(a[1], a[0], 0x07060302u);
-            o0.w = __builtin_amdgcn_perm(a[3], a[2], 0x07060302u);
-            o1.x = __builtin_amdgcn_perm(b[1], b[0], 0x05040100u);
-            o1.y = __builtin_amdgcn_perm(b[3], b[2], 0x05040100u);
-            o1.z = __builtin_amdgcn_perm(b[1], b[0], 0x07060302u);
-            o1.w = __builtin_amdgcn_perm(b[3], b[2], 0x07060302u);
-            uint4* dst = (uint4*)(out + q * 16);
-            t12_stg_stream16(dst, o0);
-            t12_stg_stream16(dst + 1, o1);
+    for (int u = 0; u < UNITS; u++) {
+        const size_t q = first + u * 256;
+        if (q < n8) {
+            uint32_t a[4];
+            t12_decode8_seq(S[u].x, S[u].y, G[u], be2, a);
+            t12_stg_stream16(out + q * 8, make_uint4(a[0], a[1], a[2], a[3]));
         }
     }
     if (e0 == e1) return;                                // (workgroup-uniform)
@@ -150,8 +140,7 @@ extern "C" int t12_decompress(const void* sm, const void* gr, int base_exp, cons
     const size_t n16 = vec_ok ? n / 16 : 0;
     if (n16 && n16 * 16 == n && patched && row_off && (n + 4095) / 4096 <= 0x7FFFFFFFull) {
         const uint32_t be2 = ((uint32_t)base_exp << 7) | ((uint32_t)base_exp << 23);
-        // one 16-element piece per lane: two and four pieces in flight per lane measured 5-8 % slower (42.6 / 43.3 us
-        // against 40.5 on 14336 x 4096)
+        // (two units per lane and 4096 elements per workgroup; with pieces of 16, two and four times as many were 5-8 % slower)
         hipLaunchKernelGGL(decompress_patched_kernel<1>, dim3((unsigned)((n + 4095) / 4096)), dim3(256), 0, st, (const uint8_t*)sm,
                            (const uint8_t*)gr, be2, (const int32_t*)row_off, (const int32_t*)cols, (const int16_t*)correct,
                            (uint16_t*)out_bf16, n16, M, K);
