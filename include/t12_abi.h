@@ -264,6 +264,13 @@ int t12_pack_planes(const void* w_bf16, int M, int K, int base_exp, void* sm, vo
 int t12_pack_row_offsets(const void* row_cnt, int M, void* row_off, void* stream);
 int t12_pack_escapes(const void* w_bf16, int M, int K, int base_exp, const void* row_off, void* cols,
                      void* correct, void* wrong, void* stream);
+/*   t12_pack_begin     : histogram, base exponent (to base_exp, i32 in device memory), planes, counts and row offsets,
+ *                        enqueued in one call: the host reads base_exp and row_off[M] once, where it needs them
+ *   t12_pack_escapes_plane: t12_pack_escapes reading the nibble plane (a zero is an escape) */
+int t12_pack_begin(const void* w_bf16, int M, int K, void* hist_u64x256, void* base_exp, void* sm, void* gr, void* row_cnt, void* row_off,
+                   void* stream);
+int t12_pack_escapes_plane(const void* w_bf16, const void* gr, int M, int K, int base_exp, const void* row_off, void* cols,
+                           void* correct, void* wrong, void* stream);
 
 /* ---- reference-named launchers (same signatures and semantics) -------------
  * For host code written against the reference's launch layer.

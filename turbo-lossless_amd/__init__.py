@@ -113,6 +113,8 @@ _SIGS = {
     "t12_pack_planes": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "t12_pack_row_offsets": (_i, [_vp, _i, _vp, _vp]),
     "t12_pack_escapes": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
+    "t12_pack_begin": (_i, [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "t12_pack_escapes_plane": (_i, [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
     "t12_gemv": (_i, [C.POINTER(Segment), _i, _vp, _i, _vp]),
     "t12_synth_normal_bf16": (_i, [_vp, C.c_size_t, C.c_uint64, C.c_float, C.c_float, C.c_float, _vp]),
     "t12_fill_f32": (_i, [_vp, C.c_size_t, C.c_float, _vp]),
@@ -399,24 +401,29 @@ def pack_device(w, base_exp=None, stream=None) -> DeviceTensor12:
     assert w.dim() == 2 and w.is_contiguous() and w.element_size() == 2
     M, K = w.shape
     st = current_stream() if stream is None else stream
-    if base_exp is None:
-        base_exp = find_base_exp_device(w, st)
     n = M * K
     dev = w.device
     sm = torch.empty(n, dtype=torch.uint8, device=dev)
     gr = torch.empty((n + 1) // 2, dtype=torch.uint8, device=dev)
     cnt = torch.empty(M, dtype=torch.int32, device=dev)
-    row_off = torch.empty(M + 1, dtype=torch.int32, device=dev)
-    check(lib.t12_pack_planes(w.data_ptr(), M, K, base_exp, sm.data_ptr(), gr.data_ptr(), cnt.data_ptr(), st),
-          "t12_pack_planes")
-    check(lib.t12_pack_row_offsets(cnt.data_ptr(), M, row_off.data_ptr(), st), "t12_pack_row_offsets")
-    P = int(row_off[M].item())                      # synchronises
+    off = torch.empty(M + 2, dtype=torch.int32, device=dev)           # row offsets, and behind them the base exponent
+    row_off = off[:M + 1]
+    if base_exp is None:
+        hist = torch.empty(256, dtype=torch.int64, device=dev)
+        check(lib.t12_pack_begin(w.data_ptr(), M, K, hist.data_ptr(), off.data_ptr() + 4 * (M + 1), sm.data_ptr(), gr.data_ptr(),
+                                 cnt.data_ptr(), off.data_ptr(), st), "t12_pack_begin")
+        P, base_exp = off[M:].tolist()              # synchronises
+    else:
+        check(lib.t12_pack_planes(w.data_ptr(), M, K, base_exp, sm.data_ptr(), gr.data_ptr(), cnt.data_ptr(), st),
+              "t12_pack_planes")
+        check(lib.t12_pack_row_offsets(cnt.data_ptr(), M, row_off.data_ptr(), st), "t12_pack_row_offsets")
+        P = int(row_off[M].item())                  # synchronises
     cols = torch.empty(P, dtype=torch.int32, device=dev)
     correct = torch.empty(P, dtype=torch.int16, device=dev)
     wrong = torch.empty(P, dtype=torch.int16, device=dev)
     if P:
-        check(lib.t12_pack_escapes(w.data_ptr(), M, K, base_exp, row_off.data_ptr(), cols.data_ptr(),
-                                   correct.data_ptr(), wrong.data_ptr(), st), "t12_pack_escapes")
+        check(lib.t12_pack_escapes_plane(w.data_ptr(), gr.data_ptr(), M, K, base_exp, row_off.data_ptr(), cols.data_ptr(),
+                                         correct.data_ptr(), wrong.data_ptr(), st), "t12_pack_escapes_plane")
     return DeviceTensor12(M, K, base_exp, sm, gr, row_off, cols, correct, wrong)
 
 
