@@ -273,6 +273,49 @@ def test_delta_scan_of_runs_that_end_inside_a_chunk(t12, heads, dim, n):
     assert rel_err(D.feed(x[n:], range(n, n + 6), 0), want[n:]) < 1e-4
 
 
+@pytest.mark.parametrize("heads, dim, rank", [(2, 64, 64), (3, 48, 65), (1, 32, 5), (2, 33, 1), (1, 31, 3)])
+@pytest.mark.parametrize("n", [39, 40, 48, 49, 64, 65, 113])
+@pytest.mark.parametrize("decay", [0.0, float(np.exp(-0.5)), 1.0, 1.5])
+def test_delta_chunks_equal_the_tokens_one_by_one(t12, heads, dim, rank, n, decay):
+    """Runs of 40 tokens and more of heads of 32 to 64 channels go through the chunked kernels at decay rates up to one, portions of
+    13 token by token: same outputs, same state, from a state that is not zero."""
+    x = np.random.default_rng(n + dim).standard_normal((n + 7, Delta(t12, heads, dim, rank).ld))
+    x[20, dim * heads] = 30.0                                          # a key that dwarfs the others
+    got = []
+    for cuts in ([n], [13] * (n // 13) + [n % 13] * (n % 13 > 0)):
+        D = Delta(t12, heads, dim, rank)
+        D.d.decay_rate = decay
+        D.feed(x[:7], range(7), 0)
+        out, pos = [], 7
+        for c in cuts:
+            out.append(D.feed(x[pos:pos + c], range(pos, pos + c), 0))
+            pos += c
+        got.append((np.concatenate(out), D.state.view(2, -1)[D.parity[0]].cpu().numpy()))
+    # (32-bit sums of up to 64 terms, state and outputs of the order of their terms: some 1e-7 each)
+    assert rel_err(got[0][1], got[1][1]) < 1e-5
+    assert rel_err(got[0][0], got[1][0]) < 1e-5
+
+
+@pytest.mark.parametrize("field", ["k", "v", "a", "w1", "r"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_a_token_that_is_not_finite_leaves_those_before_it_alone(t12, field, value):
+    D, n, at = Delta(t12, 2, 64, 8), 60, 37
+    x = np.random.default_rng(5).standard_normal((n, D.ld))
+    want = D.feed(x, range(n), 0)
+    col = getattr(D.d, field + "_off") + (0 if field == "w1" else 64 + 3)
+    x[at, col] = value
+    got = D.feed(x, range(n), 0)
+    if field in ("a", "w1") and value == float("inf"):
+        assert np.isfinite(got).all()                                  # a removal rate of one; a tanh of one
+        assert np.array_equal(got[:at], want[:at])
+        return
+    hit = slice(0, 128) if field == "w1" else slice(64, 128)           # (W2 takes w1 to every head)
+    assert np.array_equal(got[:at], want[:at])
+    assert np.isnan(got[at, hit]).any() and np.isnan(got[at:, hit]).any(axis=1).sum() == (1 if field == "r" else n - at)
+    if field != "w1":
+        assert np.array_equal(got[:, :64], want[:, :64])               # the other head
+
+
 def test_delta_state_survives_long_sequences_and_restarts_at_zero(t12):
     D = Delta(t12, 2, 64, 16)
     x = np.random.default_rng(1).standard_normal((700, D.ld))

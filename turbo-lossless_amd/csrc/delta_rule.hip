@@ -10,7 +10,10 @@
 // once per token and head and leaves it in a workspace.  The output is taken from the OLD state as well,
 // S_new^T r = S^T (w r) - (r . a u) (u^T S) + (r . k) v, so that of a token's two reductions only u^T S is in the way of
 // the next token; the other one is put off and taken for sixteen tokens at once.
+//
+// Runs of heads of 32 to 64 channels take sixteen tokens at a time instead (CHUNK below), on the matrix cores.
 
+#include <algorithm>
 #include <mutex>
 
 #include "delta_rule.h"
@@ -21,6 +24,14 @@
 using namespace delta_rule;
 
 namespace {
+
+constexpr int CHUNK_FLOATS = 6 * 16 * 64 + 64;
+// Fewest tokens taken in chunks, whole calls of 16 heads of 64, token by token against chunks: 31 / 33 tokens 15.4 / 15.9 us against 16.1 / 16.1,
+// 64 / 100 / 512 tokens 19.4 / 24.5 / 72.6 against 15.8 / 18.3 / 37.7 (64 heads: 105.5 against 60.9).
+constexpr int CHUNK_FROM = 40;
+// The most a chunk's floats come to per token of a run: 49 tokens are four chunks.
+constexpr int CHUNK_ROW = (4 * CHUNK_FLOATS + 48) / 49;
+static_assert(CHUNK_FROM > 33 && CHUNK_FROM <= 49, "CHUNK_ROW is that of the shortest run of four chunks");
 
 // Workgroup = 16 tokens of one head.  Dynamic LDS: tanh(w1) [rank][16].
 constexpr int PREP_TOK = 16;
@@ -243,6 +254,364 @@ __global__ __launch_bounds__(64) void delta_run_direct_kernel(const DeltaParams 
     C.store();
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// A run of tokens, sixteen at a time, for heads of 32 to 64 channels.
+//
+// Inside a chunk let P_t be the product of the decays of its tokens up to t (per key channel) and S0 the state before it.  With
+//   u~_t = u_t P_(t-1),  r~_t = r_t P_t,   z_t = u_t^T S_(t-1) (what the rule takes away),
+// the recurrence written out is
+//   z_t = u~_t S0 + sum over s < t of [ (u~_t . k_s / P_s) v_s - (u~_t . a_s / P_s) z_s ],          a_s = (a u)_s
+//   o_t = r~_t S0 + sum over s <= t of [ (r~_t . k_s / P_s) v_s - (r~_t . a_s / P_s) z_s ],
+//   S   = P S0 + sum over s of (P / P_s) (k_s v_s - a_s z_s)                                         P: the whole chunk's decay.
+// The first line is a unit lower triangular system: solved once per chunk for the columns of u~ and for those of the v term, it is
+//   z = TU S0 + Y,   o = RU S0 + Q,   S = P S0 + K~^T v - A~^T z,
+// and everything but S0 is known beforehand: delta_chunk_kernel forms it for all chunks side by side, and what is left of the chain
+// is two dependent products of 16 x 16 x 64 per sixteen tokens (delta_scan_kernel) in place of sixteen reductions.
+//
+// 1 / P_s stays below e^(16 decay_rate): the path is for decay rates up to one (9e6 at most; 1.6e4 at e^-0.5).  All in 32 bits: the fp32
+// matrix instruction multiplies and adds like FMAs, and S is rounded once per chunk instead of three times per token.  Error of
+// outputs / state against 64 bits, mean of eight inputs, 16 heads of 64 over 512 tokens: 2.34e-7 / 2.70e-7, token by token 2.47e-7 / 2.85e-7;
+// 4 heads of 32 over 300: 1.80e-7 / 1.70e-7 and 1.83e-7 / 1.76e-7.
+//
+// Times (16 heads of 64, 512 tokens): delta_chunk_kernel 17 us, two workgroups per CU, each a serial chain of its own (memory, sums over 64 channels, the
+// triangular solution); delta_scan_kernel 18.6, 0.58 us per chunk: two products of four dependent matrix instructions and one
+// exchange through LDS.  Token by token they were 12 and 67.
+//
+// A token that is not finite (in k, a, w or v) must not reach the tokens before it, which a product with a zero would do: the chunk is
+// formed without the tokens from it on, their outputs and the state behind the chunk are NaN, as the norm over a head's
+// outputs makes them anyway.  (An r that is not finite stays in its own token's row.)
+// ---------------------------------------------------------------------------------------------------------------------
+constexpr int CHUNK = 16, CD = 64;
+constexpr int CDP = CD + 4, CP = CHUNK + 4;                // LDS rows of 68 and 20 floats: sixteen rows read 16 bytes each over all banks
+// A chunk in the workspace, [head][chunk][CHUNK_FLOATS]: TU, RU, -A~, K~, v, Y of 16 x 64 floats each, in the order in which the scan's waves take
+// them (a wave's load is one stretch of 1 KB; row by row they were 4 to 16 pieces, and the scan waited for its cache), then P [64].
+//   token order (-A~, K~, v, Y): [channel / 16][token / 4][channel % 16][token % 4]
+//   key order   (TU, RU):        [channel / 16][channel / 4 % 4][token][channel % 4]
+enum { C_TU, C_RU, C_NA, C_K, C_V, C_Y, C_P };
+constexpr int C_ARRAY = CHUNK * CD;
+
+// x times a 64-bit factor given as the sum of two floats
+struct Factor {
+    float hi, lo;
+    __device__ __forceinline__ explicit Factor(double x) : hi((float)x), lo((float)(x - (double)(float)x)) {}
+    __device__ __forceinline__ float operator*(float x) const { return fmaf(x, hi, x * lo); }     // (rounded once)
+};
+
+// Workgroup = one chunk of one head.  Wave w has the channels 16 w .. 16 w + 15, lane group g of it the tokens 4 g .. 4 g + 3: where the
+// matrix product with W2 leaves them.  Dynamic LDS: tanh(w1) [16][rank rounded up to 64, + 4].
+__global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
+{
+    extern __shared__ float4 th4[];
+    float* th = (float*)th4;
+    __shared__ __align__(16) float us[CHUNK * CDP], as[CHUNK * CDP], ks[CHUNK * CDP], rs[CHUNK * CDP], vs[CHUNK * CDP], pair[4][CHUNK * CP];
+    __shared__ float norm[4][CHUNK];
+    __shared__ int bad;
+    const T12DeltaRule& d = p.d;
+    const int head = blockIdx.y, t0 = blockIdx.x * CHUNK, nt = min(CHUNK, p.n - t0);
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, m = lane & 15, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int D = d.dim, rank = d.rank, HD = d.heads * D, rank_p = (rank + 63) & ~63, th_row = rank_p + 4;
+    const int ch = wave * 16 + m, hc = head * D + min(ch, D - 1);
+    float k[4], a[4], r[4], v[4], w[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float* y = p.in + (size_t)(t0 + min(g * 4 + j, nt - 1)) * p.ld + hc;
+        k[j] = y[d.k_off];
+        a[j] = y[d.a_off];
+        r[j] = y[d.r_off];
+        v[j] = y[d.v_off];
+    }
+    const float bk = p.bias[d.k_off + hc], ba = p.bias[d.a_off + hc], br = p.bias[d.r_off + hc], bv = p.bias[d.v_off + hc], w0 = d.w0[hc];
+    // W2, sixty-four rows at a time (the first of them ahead of all that waits): step e of sixteen rows contracts its rows 4 g + e
+    auto w2_at = [&](int q0, int e) __attribute__((always_inline)) { return d.w2t[(size_t)(uint32_t)(min(q0 + (e & 12) * 4 + g * 4 + (e & 3), rank - 1) * HD) + hc]; };
+    float w2[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) w2[e] = w2_at(0, e);
+    if (tid == 0) bad = CHUNK;
+    for (int q = tid; q < CHUNK * rank_p; q += 256) {      // (past the rank: zeros)
+        const int t = q / rank_p, c = q % rank_p, from = d.w1_off + min(c, rank - 1);
+        const float x = tanhf(p.in[(size_t)(t0 + min(t, nt - 1)) * p.ld + from] + p.bias[from]);
+        th[t * th_row + c] = c < rank ? x : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        k[j] = ch < D ? k[j] + bk : 0.0f;
+        const float ss = row_sum16(k[j] * k[j]);
+        if (m == 0) norm[wave][g * 4 + j] = ss;
+    }
+    __syncthreads();
+    t12_f32x4 z = (t12_f32x4)(0.0f);
+    {
+        const float* x = th + m * th_row + g * 4;
+        for (int q0 = 0; q0 < rank_p; q0 += 64) {
+            if (q0)
+#pragma unroll
+                for (int e = 0; e < 16; e++) w2[e] = w2_at(q0, e);
+#pragma unroll
+            for (int e = 0; e < 16; e++) z = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q0 + (e & 12) * 4 + (e & 3)], w2[e], z, 0, 0, 0);
+        }
+    }
+    double own = 1.0;                                      // decay of the thread's four tokens
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int t = g * 4 + j;
+        const bool in = t < nt && ch < D;
+        const float u = k[j] * (1.0f / sqrtf((norm[0][t] + norm[1][t]) + (norm[2][t] + norm[3][t]) + d.unit_eps));
+        a[j] = t12_sigmoid(a[j] + ba) * u;
+        w[j] = expf(-d.decay_rate * t12_sigmoid(z[j] + w0));
+        v[j] += bv;
+        const bool fine = __builtin_isfinite(k[j]) && __builtin_isfinite(a[j]) && __builtin_isfinite(w[j]) && __builtin_isfinite(v[j]);
+        if (in && !fine) atomicMin(&bad, t);
+        if (!in || !__builtin_isfinite(w[j])) w[j] = 1.0f; // (tokens and channels that are not there leave the state alone)
+        r[j] = in ? r[j] + br : 0.0f;
+        z[j] = in ? u : 0.0f;                              // from here on: u
+        if (!in) k[j] = a[j] = v[j] = 0.0f;
+        own *= w[j];
+    }
+    // (64-bit products of the decays: every scaled operand is rounded once)
+    double before = 1.0, after = 1.0, all = 1.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const double x = __shfl(own, q * 16 + m);
+        if (q < g) before *= x;
+        if (q > g) after *= x;
+        all *= x;
+    }
+    __syncthreads();
+    const int first_bad = bad;
+    float* chunk = p.rec + ((size_t)head * gridDim.x + blockIdx.x) * CHUNK_FLOATS;
+    float* out = chunk + tid * 4;
+    {
+        t12_f32x4 na, kt, vt;
+#pragma unroll
+        for (int j = 3; j >= 0; j--) {
+            if (g * 4 + j >= first_bad) k[j] = a[j] = v[j] = z[j] = 0.0f;
+            const Factor tail(after);                      // decay of the tokens behind this one
+            na[j] = -(tail * a[j]);
+            kt[j] = tail * k[j];
+            vt[j] = v[j];
+            after *= w[j];
+        }
+        *(t12_f32x4*)(out + C_NA * C_ARRAY) = na;
+        *(t12_f32x4*)(out + C_K * C_ARRAY) = kt;
+        *(t12_f32x4*)(out + C_V * C_ARRAY) = vt;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int at = (g * 4 + j) * CDP + ch;
+        us[at] = Factor(before) * z[j];
+        before *= w[j];
+        const Factor here(before);
+        const float guess = 1.0f / here.hi;                // 1 / before: what is left of one step from there
+        const Factor back(fma((double)guess, fma(-before, (double)guess, 1.0), (double)guess));
+        as[at] = back * a[j];
+        ks[at] = back * k[j];
+        rs[at] = here * r[j];
+        vs[at] = v[j];
+    }
+    if (g == 0) chunk[C_P * C_ARRAY + ch] = first_bad < CHUNK ? __builtin_nanf("") : (float)all;
+    __syncthreads();
+    {
+        // wave 0: u~ . a / P (token, earlier token; the other way round in LDS), 1: u~ . k / P, 2: - r~ . a / P, 3: r~ . k / P
+        const float *x = (wave < 2 ? us : rs) + m * CDP + g * 4, *y = (wave & 1 ? ks : as) + m * CDP + g * 4;
+        t12_f32x4 part[8], acc;                            // (short sums: the products of a long one would each be rounded to the size of all)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const t12_f32x4 xa = *(const t12_f32x4*)(x + q * 16), yb = *(const t12_f32x4*)(y + q * 16);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                part[q * 2 + e / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[e], yb[e], e & 1 ? part[q * 2 + e / 2] : (t12_f32x4)(0.0f), 0, 0, 0);
+        }
+        acc = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int t = g * 4 + e;
+            const float c = m < t + (wave >> 1) ? acc[e] : 0.0f;
+            pair[wave][wave ? t * CP + m : m * CP + t] = wave == 2 ? -c : c;
+        }
+    }
+    __syncthreads();
+    // the v terms, sixteen value channels per wave; that of z goes where k was
+    t12_f32x4 bv4 = (t12_f32x4)(0.0f), lv = (t12_f32x4)(0.0f);
+    {
+        const t12_f32x4 cb = *(const t12_f32x4*)(pair[1] + m * CP + g * 4), cl = *(const t12_f32x4*)(pair[3] + m * CP + g * 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float x = vs[(g * 4 + e) * CDP + wave * 16 + m];
+            bv4 = __builtin_amdgcn_mfma_f32_16x16x4f32(cb[e], x, bv4, 0, 0, 0);
+            lv = __builtin_amdgcn_mfma_f32_16x16x4f32(cl[e], x, lv, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) ks[(g * 4 + e) * CDP + wave * 16 + m] = bv4[e];
+    }
+    __syncthreads();
+    if (wave < 2) {                                        // wave 0: the columns of u~, wave 1: those of the v term; solved in place
+        float* col = (wave ? ks : us) + lane;
+        float x[CHUNK];
+#pragma unroll
+        for (int t = 0; t < CHUNK; t++) x[t] = col[t * CDP];
+#pragma unroll
+        for (int t = 0; t < CHUNK; t++) {
+#pragma unroll
+            for (int q = 0; q < CHUNK / 4; q++)
+                if (q * 4 + 3 > t) {
+                    const t12_f32x4 c = *(const t12_f32x4*)(pair[0] + t * CP + q * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (q * 4 + e > t) x[q * 4 + e] -= c[e] * x[t];
+                }
+            col[t * CDP] = x[t];
+        }
+    }
+    __syncthreads();
+    // what a token takes off its own output and off that of those behind it: sixteen columns each of RU and of Q per wave
+    t12_f32x4 ru = (t12_f32x4)(0.0f), taken = (t12_f32x4)(0.0f), y;
+    {
+        const t12_f32x4 cm = *(const t12_f32x4*)(pair[2] + m * CP + g * 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int at = (g * 4 + e) * CDP + ch;
+            y[e] = ks[at];
+            ru = __builtin_amdgcn_mfma_f32_16x16x4f32(cm[e], us[at], ru, 0, 0, 0);
+            taken = __builtin_amdgcn_mfma_f32_16x16x4f32(cm[e], y[e], taken, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) ru[e] += rs[(g * 4 + e) * CDP + ch];
+    lv += taken;
+    *(t12_f32x4*)(out + C_Y * C_ARRAY) = y;
+    *(t12_f32x4*)(out + C_TU * C_ARRAY) = *(const t12_f32x4*)(us + m * CDP + wave * 16 + g * 4);
+#pragma unroll
+    for (int e = 0; e < 4; e++) rs[(g * 4 + e) * CDP + ch] = ru[e];      // (turned round inside the wave's own sixteen columns)
+    float* o = p.o + ((size_t)t0 * d.heads + head) * D + ch;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int t = g * 4 + e;
+        if (t < nt && ch < D) o[(size_t)t * HD] = t < first_bad ? lv[e] : __builtin_nanf("");
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    *(t12_f32x4*)(out + C_RU * C_ARRAY) = *(const t12_f32x4*)(rs + m * CDP + wave * 16 + g * 4);
+}
+
+// What a wave takes of one chunk: operands of its sixteen key channels and sixteen value channels.  The four registers of an operand are
+// the four steps of a product: step e contracts the indices 4 g + e of lane groups g, which is where a product's result has them.
+struct ChunkOperands {
+    t12_f32x4 tu, ru, na, k, v, y, decay;
+    float q;
+};
+// Buffer loads: their 32-bit offsets (bytes from the head's first chunk) are all the address arithmetic, which as 64-bit pointers takes longer
+// than a chunk's products, and what is requested past the last chunk or token is past the buffer's end and reads as zero.
+typedef __amdgpu_buffer_rsrc_t Buffer;
+__device__ __forceinline__ Buffer buffer_of(const float* x, size_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)bytes, 0x00027000);     // raw, 32-bit elements
+}
+__device__ __forceinline__ float load1(Buffer b, uint32_t at)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, at, 0, 0));
+}
+__device__ __forceinline__ t12_f32x4 load4(Buffer b, uint32_t at)
+{
+    return __builtin_bit_cast(t12_f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, at, 0, 0));
+}
+__device__ __forceinline__ void store1(float x, Buffer b, uint32_t at)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, x), b, at, 0, 0);
+}
+// a quarter of a chunk's requests; keys, values: where in the chunk the wave's key channels and its value channels start for this lane
+__device__ __forceinline__ void request_step(ChunkOperands& x, int e, Buffer b, uint32_t keys, uint32_t values, uint32_t decay)
+{
+    if (e == 0) x.tu = load4(b, keys + C_TU * C_ARRAY * 4);
+    if (e == 0) x.k = load4(b, keys + C_K * C_ARRAY * 4);
+    if (e == 1) x.v = load4(b, values + C_V * C_ARRAY * 4);
+    if (e == 1) x.ru = load4(b, keys + C_RU * C_ARRAY * 4);
+    if (e == 2) x.y = load4(b, values + C_Y * C_ARRAY * 4);
+    if (e == 2) x.na = load4(b, keys + C_NA * C_ARRAY * 4);
+    if (e == 3) x.decay = load4(b, decay + C_P * C_ARRAY * 4);
+}
+
+// Workgroup = sixteen value channels of one head; wave w holds S of the key channels 16 w .. 16 w + 15.  z and o are sums over the key
+// channels, so over the waves: they cross through LDS, one barrier per chunk (two buffers).  Operands are requested three chunks ahead.
+__global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaParams p)
+{
+    __shared__ t12_f32x4 zs[2][4][64], os[2][4][64];
+    const T12DeltaRule& d = p.d;
+    const int head = blockIdx.x, j0 = blockIdx.y * 16, lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const T12Row first = p.rows[0];
+    const size_t region = (size_t)(first.slot >> 1) * 2 * d.state_elems;
+    const size_t cell = ((size_t)head * d.dim + min(j0 + m, d.dim - 1)) * CD + wave * 16 + g * 4;
+    t12_f32x4 S = (t12_f32x4)(0.0f);
+    if (first.position != 0) S = *(const t12_f32x4*)(d.state + region + (size_t)(first.slot & 1) * d.state_elems + cell);
+    const int chunks = (p.n + CHUNK - 1) / CHUNK, o_step = d.heads * d.dim;
+    float* o_head = p.o + (size_t)head * d.dim + j0;
+    constexpr uint32_t STEP = CHUNK_FLOATS * 4;            // bytes from chunk to chunk
+    const Buffer operands = buffer_of(p.rec + (size_t)head * chunks * CHUNK_FLOATS, (size_t)chunks * STEP);
+    const Buffer outs = buffer_of(o_head, ((size_t)(p.n - 1) * o_step + d.dim - j0) * 4);
+    const uint32_t keys = (uint32_t)(wave * 64 + lane) * 16, values = (uint32_t)(blockIdx.y * 64 + lane) * 16, decay = (uint32_t)(wave * 4 + g) * 16;
+    const uint32_t o_at = (uint32_t)((g * 4 + wave) * o_step + m) * 4;
+    ChunkOperands op[4];
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) request_step(op[f], e, operands, f * STEP + keys, f * STEP + values, f * STEP + decay);
+        op[f].q = load1(outs, (uint32_t)(f * CHUNK * o_step) * 4 + o_at);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("" : "+v"(S));                            // (waited for here, not by a wait at the loop's head that would hold for the others too)
+    const float* ow = (const float*)&os[0][0][lane] + wave;
+    // Each wave finishes the outputs of the tokens 4 g + wave of a chunk, one chunk later (and in the end).
+    uint32_t store_at = 0xFFFFFFFFu;                       // (outside the buffer: not stored)
+    float q = 0.0f;
+    // (chunks past the last one, up to three, are gone through on zeros without their S: with ways out of the loop inside it the
+    // compiler moves the operands' registers about and waits for all of them)
+    for (int c = 0; c < chunks; c += 4) {
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+            ChunkOperands &x = op[f], &y = op[(f + 3) & 3];
+            const int buf = f & 1;
+            const uint32_t ahead = (uint32_t)(c + f + 3) * STEP;
+            t12_f32x4 z = (t12_f32x4)(0.0f), o = (t12_f32x4)(0.0f), in = (t12_f32x4)(0.0f), out = (t12_f32x4)(0.0f);
+#pragma unroll
+            for (int e = 0; e < 4; e++) z = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tu[e], S[e], z, 0, 0, 0);
+            zs[buf][wave][lane] = z;
+            __syncthreads();                               // (a buffer is written again two chunks on, behind the next barrier)
+            t12_f32x4 part[4];
+            float done[4];
+#pragma unroll
+            for (int w = 0; w < 4; w++) part[w] = zs[buf][w][lane];
+#pragma unroll
+            for (int w = 0; w < 4; w++) done[w] = ow[(buf ^ 1) * 1024 + w * 256];
+            // what the chain does not need runs while these are on their way
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                __builtin_amdgcn_sched_barrier(0);
+                in = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[e], x.v[e], in, 0, 0, 0);
+                request_step(y, e, operands, ahead + keys, ahead + values, ahead + decay);
+                o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.ru[e], S[e], o, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            z = (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[e] += x.y[e];
+#pragma unroll
+            for (int e = 0; e < 4; e++) out = __builtin_amdgcn_mfma_f32_16x16x4f32(x.na[e], z[e], out, 0, 0, 0);
+            os[buf][wave][lane] = o;
+            store1((done[0] + done[1]) + (done[2] + done[3]) + q, outs, store_at);
+            q = x.q;
+            y.q = load1(outs, (uint32_t)((c + f + 3) * CHUNK * o_step) * 4 + o_at);
+            store_at = j0 + m < d.dim ? (uint32_t)((c + f) * CHUNK * o_step) * 4 + o_at : 0xFFFFFFFFu;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {                  // (S is rounded once per chunk)
+                const float next = fmaf(x.decay[e], S[e], in[e] + out[e]);
+                S[e] = c + f < chunks ? next : S[e];
+            }
+        }
+    }
+    __syncthreads();
+    store1((ow[1024] + ow[1280]) + (ow[1536] + ow[1792]) + q, outs, store_at);
+    if (j0 + m < d.dim) *(t12_f32x4*)(d.state + region + (size_t)((first.slot & 1) ^ 1) * d.state_elems + cell) = S;
+}
+
 // One wave per (row, head): o over its RMS, times the plain weight and the sigmoid gate.
 template <bool F32>
 __global__ __launch_bounds__(256) void delta_out_kernel(const DeltaParams p)
@@ -304,7 +673,7 @@ int t12_delta_plan(T12DeltaRule* d)
     d->dim_p = 64;
     while (d->dim_p < d->dim) d->dim_p *= 2;
     d->state_elems = (size_t)d->heads * d->dim * d->dim_p;
-    d->work_elems = (size_t)d->heads * (rec_floats(d->dim_p) + d->dim);
+    d->work_elems = (size_t)d->heads * ((d->dim_p == 64 ? std::max(CHUNK_ROW, rec_floats(64)) : rec_floats(d->dim_p)) + d->dim);
     return T12_OK;
 }
 
@@ -330,21 +699,22 @@ int t12_delta_rule(const T12DeltaRule* d, const float* in, const float* bias, in
     p.run = run;
     p.out_scale = out_scale;
     p.rec = work;
-    p.o = work + (size_t)n * d->heads * rec_floats(d->dim_p);
+    // (the factors of a chunk are those of decay rates up to one; heads of 16 channels: sums so short that token by token is the more
+    // exact, 1.37e-7 against 1.46e-7 over 48 tokens; 2^20 tokens: 32-bit offsets in the scan)
+    const bool chunked = run && d->dim_p == 64 && d->dim >= 32 && n >= CHUNK_FROM && n <= 1 << 20 && d->decay_rate >= 0.0f && d->decay_rate <= 1.0f;
+    p.o = work + (size_t)n * d->heads * (chunked ? CHUNK_ROW : rec_floats(d->dim_p));
     p.out = out;
     p.out_ld = out_ld;
     int rc;
+    if (chunked) {
+        hipLaunchKernelGGL(delta_chunk_kernel, dim3((n + CHUNK - 1) / CHUNK, d->heads), dim3(256),
+                           (size_t)CHUNK * (((d->rank + 63) & ~63) + 4) * sizeof(float), st, p);
+        hipLaunchKernelGGL(delta_scan_kernel, dim3(d->heads, (d->dim + 15) / 16), dim3(256), 0, st, p);
+        T12_CHECK_LAUNCH("t12_delta_rule(chunks)");
+        rc = T12_OK;
+    } else
     switch (d->dim_p) {
-        // Tokens between two barriers: with 32, 100 KB of LDS, a workgroup has its CU to itself, 16 (52 KB) share it with others and
-        // with the window attention of the same layer on another stream.  Alone the two take the same (16 heads, 512 tokens: 72
-        // us) while 32 fit the chip at once; beside the attention of 32 heads, 512 / 1500 tokens of four layers of width 4096, 32
-        // tokens against 16:  8 heads 1.99 / 5.20 ms against 2.05 / 5.39, 24 heads 2.13 / 5.58 against 2.17 / 5.66, 28 heads
-        // 2.16 / 5.83 against 2.17 / 5.79, 32 heads 2.49 / 6.71 against 2.45 / 6.45, 64 heads 2.88 / 7.77 against 2.67 / 7.05.
-        // So 32 up to three quarters of the CUs, and from 32 tokens on.
-        case 64:
-            if (n >= 32 && d->heads * ((d->dim + 7) / 8) <= 192) rc = launch_rule<4, 32>(p, st);
-            else rc = launch_rule<4, 16>(p, st);
-            break;
+        case 64: rc = launch_rule<4, 16>(p, st); break;    // (short runs, and decay rates the chunks are not for)
         case 128: rc = launch_rule<8, 16>(p, st); break;
         case 256: rc = launch_rule<16, 0>(p, st); break;
         default: rc = launch_rule<32, 0>(p, st); break;
