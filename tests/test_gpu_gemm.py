@@ -63,6 +63,22 @@ def test_gemm_few_stages(t12, oracle, synth, K, B):
     assert rel_err(got, oracle.gemm(p, X)) < TOL
 
 
+@pytest.mark.parametrize("B", [70, 200, 300])
+@pytest.mark.parametrize("first", [0, 48, 60, 240, 1008])
+def test_gemm_escapes_side_by_side(t12, oracle, synth, B, first):
+    """Sixteen neighbouring escapes in every row, at the start, the end and across the edge of a stage or window: with 128 rows exactly the 2048
+    entries the LDS list holds.  The entry behind a row's last one is the next row's."""
+    M, K = 128, 1024
+    w = synth.weights_llm(M, K, seed=first, p_outlier=0.0)
+    w[(w & 0x7F80) < (0x70 << 7)] = 0x3C00                             # nothing else needs an escape
+    w[:, first:first + 16] = 0x4100 + np.arange(16, dtype=w.dtype)
+    p = oracle.pack(w)
+    assert p.P == 2048
+    X = synth.activations(B, K, seed=B)
+    (got,) = run_gemm(t12, [p], X)
+    assert rel_err(got, oracle.gemm(p, X)) < TOL
+
+
 @pytest.mark.parametrize("patched", [(True, False), (False, True), (False, False)])
 @pytest.mark.parametrize("M, K, B", [(12300, 192, 70), (12300, 320, 200)])
 def test_gemm_swiglu_with_one_list(t12, synth, M, K, B, patched):

@@ -78,16 +78,19 @@ __device__ __forceinline__ int scalar_load(const int* p) { return *(const __attr
 // the fragment reads (neighbouring lanes = consecutive rows of one unit).
 __device__ __forceinline__ int lds_slot(int u, int r, int rows) { return u * rows + (r & ~7) + ((r + u) & 7); }
 
-// Order in which a thread's staging units are stored: the ndec decode units (18 VALU each) evenly
-// among the nact activation units (4 VALU each).  Position pos -> unit index (activation units
-// 0 .. nact-1, decode units nact .. nact+ndec-1).
+// Order in which a thread's staging units are stored: the ndec decode units (18 VALU each) and as many of the nact activation units (4
+// VALU each) in turn, then the other activation units; the escapes among the decoded go over them in between, under the stage's last
+// products.  Behind the last one, in front of the barrier, they and their two reads of the list cost 28672 x 4096 at 512 rows 149.0 us (2e-4 of the weights)
+// and 149.4 (1e-3); now 143.2 both; without any escapes 138.  8256 x 2048 at 512 36.7 / 39.2 -> 34.7 / 35.3, 28672 x 4096 at 100 49.2 / 52.8 -> 47.7 / 49.6.
+// Position pos -> unit index (activation units 0 .. nact-1, decode units nact .. nact+ndec-1).
 __device__ __forceinline__ constexpr int stage_unit_order(int pos, int nact, int ndec)
 {
-    const int nu = nact + ndec;
-    const int dec_before = pos * ndec / nu;              // decode units placed before pos
-    const bool is_dec = (pos + 1) * ndec / nu > dec_before;
-    return is_dec ? nact + dec_before : pos - dec_before;
+    const int mixed = nact < ndec ? nact : ndec;
+    if (pos < 2 * mixed) return pos & 1 ? pos / 2 : nact + pos / 2;
+    return nact < ndec ? nact + pos - mixed : pos - ndec;
 }
+// position of the last decode unit
+__device__ __forceinline__ constexpr int last_decode_unit(int nact, int ndec) { return nact < ndec ? nact + ndec - 1 : 2 * ndec - 2; }
 
 // ---------------------------------------------------------------------------
 // LDS stage layout (one of two buffers), unit u = (k % 64) / 8 = eight bf16 of one row,
@@ -311,16 +314,22 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
         if (tid <= ER) lrow[tid] = has0 ? my_off - e00 : 0;
         else if (SWI && tid <= 2 * ER + 1) lrow[tid] = n0 + (has1 ? my_off - e10 : 0);
     }
-    // Per piece kind and item: cursor into its row's slice and the column of the next entry.  The
-    // thread that decoded 16 columns of a row into LDS also overwrites the escapes among them
+    // Per piece kind and item: cursor into its row's slice, the column of the next entry, the entry itself and the one behind
+    // it.  The thread that decoded 16 columns of a row into LDS also overwrites the escapes among them
     // there (same wave, LDS executes its writes in order: no barrier needed in between).  A
     // thread owns its X row in even stages and its Y row in odd ones; entries of the stages in
-    // between are stepped over.
+    // between are stepped over.  An entry is in registers a stage before its turn at the latest, unless the row has three close
+    // together: a wave that read the list when it came to an entry held the seven others up.
     int pp[2][W_LD], pe[2][W_LD], nc[2][W_LD];
+    uint32_t cur[2][W_LD], behind[2][W_LD];
 #pragma unroll
     for (int y = 0; y < 2; y++)
 #pragma unroll
-        for (int i = 0; i < W_LD; i++) { pp[y][i] = pe[y][i] = 0; nc[y][i] = NO_ESCAPE; }
+        for (int i = 0; i < W_LD; i++) {
+            pp[y][i] = pe[y][i] = 0;
+            nc[y][i] = NO_ESCAPE;
+            cur[y][i] = behind[y][i] = 0;
+        }
     auto patch_stage = [&](int y, int buf, int kabs) {
         if (esc_mode != 1) return;
         uint8_t* base_ = lds + buf * STAGE_BYTES + ACT_UNITS * 16;
@@ -330,10 +339,11 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
                 const int e = nc[y][i] - kabs - 16 * cc;            // 0..15: one of this piece's
                 if ((unsigned)e < 16u) {
                     const int off = lds_slot(2 * cc + (e >> 3), w_row[y][i], TM) * 16 + (e & 3) * 4 + ((e >> 2) & 1) * 2;
-                    *(uint16_t*)(base_ + off) = (uint16_t)(lpat[pp[y][i]] >> 16);
+                    *(uint16_t*)(base_ + off) = (uint16_t)(cur[y][i] >> 16);
                 }
-                pp[y][i]++;
-                nc[y][i] = pp[y][i] < pe[y][i] ? (int)(lpat[pp[y][i]] & 0xFFFFu) : NO_ESCAPE;
+                cur[y][i] = behind[y][i];
+                nc[y][i] = ++pp[y][i] < pe[y][i] ? (int)(cur[y][i] & 0xFFFFu) : NO_ESCAPE;
+                behind[y][i] = lpat[pp[y][i] + 1];                  // (at most one past the list: the offsets behind it)
             }
         }
     };
@@ -347,6 +357,7 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
     constexpr int NSU = ACT_LD + 2 * W_LD;               // store units per stage
     constexpr int NLU_ODD = ACT_LD + 4 * W_LD;           // load units of an odd stage
     constexpr int NCH = NMMA >= 2 * NSU ? NSU : NMMA;    // chunks of staging work per stage
+    constexpr int PATCH_AT = last_decode_unit(ACT_LD, 2 * W_LD) * NCH / NSU;
     auto run_stage = [&](int d, int stg, bool ld_act, bool ld_x, bool ld_y, bool do_store) {
         const int buf = d & 1;
         const bool odd = d & 1;
@@ -395,13 +406,16 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
                             for (int u = 0; u < NSU; u++)
                                 if (do_store && u * NCH / NSU == c)
                                     store_unit(n_aslot, n_wslot, n_y, n_buf, stage_unit_order(u, ACT_LD, 2 * W_LD));
+                            if (do_store && c == PATCH_AT) {
+                                __builtin_amdgcn_sched_barrier(0);
+                                patch_stage(n_y, n_buf, k_begin + (stg + 1) * KC);
+                            }
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     }
                 }
             }
         }
-        if (do_store) patch_stage(n_y, n_buf, k_begin + (stg + 1) * KC);
         __syncthreads();
     };
 
@@ -419,7 +433,11 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
                 while (q < qe && (int)(lpat[q] & 0xFFFFu) < k_begin) q++;   // K split: skip earlier columns
                 pp[y][i] = q;
                 pe[y][i] = qe;
-                if (q < qe) nc[y][i] = (int)(lpat[q] & 0xFFFFu);
+                if (q < qe) {
+                    cur[y][i] = lpat[q];
+                    behind[y][i] = lpat[q + 1];
+                    nc[y][i] = (int)(cur[y][i] & 0xFFFFu);
+                }
             }
     }
     if (nstage > 0) {
