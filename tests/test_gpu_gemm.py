@@ -63,6 +63,22 @@ def test_gemm_few_stages(t12, oracle, synth, K, B):
     assert rel_err(got, oracle.gemm(p, X)) < TOL
 
 
+@pytest.mark.parametrize("B", [3, 4, 5, 8, 9, 16, 17, 20, 31, 32])
+@pytest.mark.parametrize("M, K", [(1, 128), (15, 256), (17, 1152), (33, 896), (513, 2176)])
+def test_gemm_sweep_with_loads_turned_through_lds(t12, oracle, synth, B, M, K):
+    """Row groups and batch tiles that end inside a load of 4, 8 or 16 rows, fewer and uneven blocks of 128 columns per wave.  A row of
+    NaN stays in its row."""
+    p = oracle.pack(synth.weights_llm(M, K, seed=M, p_outlier=5e-3))
+    X = synth.activations(B, K, seed=B)
+    (got,) = run_gemm(t12, [p], X)
+    assert rel_err(got, oracle.gemm(p, X)) < TOL
+    X[B // 2] = 0x7FC0
+    (nan,) = run_gemm(t12, [p], X)
+    assert np.isnan(nan[B // 2]).all()
+    rest = np.arange(B) != B // 2
+    assert np.array_equal(nan[rest], got[rest])
+
+
 @pytest.mark.parametrize("B", [70, 200, 300])
 @pytest.mark.parametrize("first", [0, 48, 60, 240, 1008])
 def test_gemm_escapes_side_by_side(t12, oracle, synth, B, first):

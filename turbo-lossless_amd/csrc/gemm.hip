@@ -38,6 +38,7 @@
 
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -669,8 +670,9 @@ __global__ __launch_bounds__(256) void gemm_general_kernel(const GemmParams p)
 //     block a lane loads 2 x 16 bytes of sign/mantissa (columns 32g .. 32g+15 and 32g+16 .. 32g+31: the four lanes
 //     of a row cover its 128-byte line in two back-to-back instructions) and 16 bytes of nibbles, rebuilds them
 //     with t12_decode8 and feeds four MFMAs;
-//   * the activations are not staged: lane (b, g) reads the 8 columns an MFMA needs straight from memory (they are
+//   * the activations are not shared between waves: lane (b, g) takes the 8 columns an MFMA needs (they are
 //     B x K bf16, resident in L2) and pairs them in registers to match t12_decode8's order;
+//   * with one row group or two batch tiles the loads are turned through LDS on their way to these lanes (NX below);
 //   * no barrier until the end, where the waves' partial 16 x 16 tiles are added through LDS in wave order;
 //   * escapes: the streamed value of a group-0 weight is its "wrong" value; wave w adds (correct - wrong) * x[b, col]
 //     for the entries w, w + NW, ... of each row (the four lanes of a row each for their four batch rows).
@@ -685,9 +687,20 @@ __global__ __launch_bounds__(256) void gemm_general_kernel(const GemmParams p)
 // are 16 RG / 2 rows of gate, the others the same rows of up, and the thread that finishes an element of both stores
 // bf16( silu(gate) * up ) to out_bf16 instead of the two sums (the arithmetic of silu_mul_kernel, so the result is
 // what t12_gemm + launch_silu_mul_bf16_batch give, bit for bit).
-template <int NW, int D, int RG, bool DEV, int NBT = 1, bool SWI = false>
-__device__ __forceinline__ void gemm_dense16_body(const GemmParams& p, t12_f32x4 (*red)[NW][64])
+// NX > 0 (at most 4 NX batch rows per batch tile): neighbouring lanes load neighbouring bytes, and the operands' lanes get theirs by way of LDS, a buffer of
+// D16_TURN bytes per wave at `turn` (rows of 144, 80 and 272 bytes: sixteen lanes reading 16 bytes of sixteen rows meet no bank twice).
+// Loaded as the operands lie, sixteen lanes touch sixteen rows: 64 cache lines per load instruction, 448 per block against 48 .. 64, and a
+// CU's cache looks up one per clock.  us per call, as the operands lie -> turned: 4096 x 14336 at 4 / 8 / 16 rows 20.7 / 23.4 / 23.0 -> 18.5 / 19.9 / 23.1,
+// 2048 x 8192 at 8 13.6 -> 11.0, 4096 x 4096 at 16 / 24 / 32 10.2 / 13.1 / 14.4 -> 9.2 / 11.0 / 11.3, 4096 x 2048 at 24 10.5 -> 7.7; many rows are level
+// (28672 x 4096 at 4: 34).  Three to six blocks ahead instead of two are no faster (19.9 -> 20.5 .. 21.3), nor are sixteen waves.  Row
+// counts known on the device only keep the other form: level within 0.5 % (experts of 1 .. 6 rows stream at the rate of memory).
+constexpr int D16_SM = 144, D16_GR = 80, D16_ACT = 272;
+constexpr int d16_turn_bytes(int nx) { return 16 * (D16_SM + D16_GR) + 4 * nx * D16_ACT; }
+template <int NW, int D, int RG, bool DEV, int NBT = 1, bool SWI = false, int NX = 0>
+__device__ __forceinline__ void gemm_dense16_body(const GemmParams& p, t12_f32x4 (*red)[NW][64], uint8_t* turn = nullptr)
 {
+    static_assert(NX == 0 || (!SWI && !DEV && (NBT == 1 || NX == 4)), "no turned form");
+    constexpr bool TURN = NX > 0;
     static_assert(!SWI || (RG % 2 == 0 && !DEV && NBT == 1), "the SwiGLU form pairs row groups");
     constexpr int RH = SWI ? RG / 2 : RG;             // row groups of one tensor
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -722,6 +735,7 @@ __device__ __forceinline__ void gemm_dense16_body(const GemmParams& p, t12_f32x4
     int e_beg[RG], e_end[RG];
     const uint8_t* smp[RG];
     const uint8_t* grp[RG];
+    const uint8_t* smp8[RG];                          // TURN: rows 8 .. 15
 #pragma unroll
     for (int rg = 0; rg < RG; rg++) {
         const T12Segment& sr = p.seg[SWI && rg >= RH ? 1 : s];      // (SWI: gate for the first half, up for the second)
@@ -734,20 +748,30 @@ __device__ __forceinline__ void gemm_dense16_body(const GemmParams& p, t12_f32x4
         const size_t e0 = (size_t)min(row, M - 1) * K;              // rows past the end are clamped, never stored
         smp[rg] = sr.sm + e0 + 32 * g + (size_t)wblk * 128;
         grp[rg] = sr.gr + (e0 >> 1) + 16 * g + (size_t)wblk * 64;
+        if (TURN) {
+            smp[rg] = sr.sm + (size_t)min(m0 + 16 * rg + (lane >> 3), M - 1) * K + 16 * (lane & 7) + (size_t)wblk * 128;
+            smp8[rg] = sr.sm + (size_t)min(m0 + 16 * rg + 8 + (lane >> 3), M - 1) * K + 16 * (lane & 7) + (size_t)wblk * 128;
+            grp[rg] = sr.gr + ((size_t)min(m0 + 16 * rg + (lane >> 2), M - 1) * K >> 1) + 16 * (lane & 3) + (size_t)wblk * 64;
+        }
     }
-    const uint16_t* xp[NBT];                          // NBT tiles of 16 batch rows share every weight load and decode
+    constexpr int NXP = TURN ? NX * NBT : NBT;
+    const uint16_t* xp[NXP];                          // NBT tiles of 16 batch rows share every weight load and decode
 #pragma unroll
-    for (int t = 0; t < NBT; t++) xp[t] = act + (size_t)min(16 * t + n, B - 1) * p.act_stride + 32 * g + (size_t)wblk * 128;
-    uint4 rS[D][RG][2], rG[D][RG], rX[D][NBT][4];
+    for (int t = 0; t < NXP; t++)
+        xp[t] = TURN ? act + (size_t)min(4 * t + g, B - 1) * p.act_stride + 8 * n + (size_t)wblk * 128
+                     : act + (size_t)min(16 * t + n, B - 1) * p.act_stride + 32 * g + (size_t)wblk * 128;
+    // (copied on to LDS as they are, members of uint4 arrays end up in scratch; native vectors stay in registers)
+    using Piece = std::conditional_t<TURN, t12_u32x4, uint4>;
+    Piece rS[D][RG][2], rG[D][RG], rX[D][NXP][TURN ? 1 : 4];
 #define T12_DS_FETCH(slot, j)                                                              \
     {                                                                                      \
-        _Pragma("unroll") for (int t = 0; t < NBT; t++)                                    \
-            _Pragma("unroll") for (int q = 0; q < 4; q++)                                  \
-                rX[slot][t][q] = *(const uint4*)(xp[t] + (size_t)(j) * (NW * 128) + 8 * q); \
+        _Pragma("unroll") for (int t = 0; t < NXP; t++)                                    \
+            _Pragma("unroll") for (int q = 0; q < (TURN ? 1 : 4); q++)                     \
+                rX[slot][t][q] = *(const Piece*)(xp[t] + (size_t)(j) * (NW * 128) + 8 * q); \
         _Pragma("unroll") for (int rg = 0; rg < RG; rg++) {                                \
-            rS[slot][rg][0] = *(const uint4*)(smp[rg] + (size_t)(j) * (NW * 128));         \
-            rS[slot][rg][1] = *(const uint4*)(smp[rg] + (size_t)(j) * (NW * 128) + 16);    \
-            rG[slot][rg] = *(const uint4*)(grp[rg] + (size_t)(j) * (NW * 64));             \
+            rS[slot][rg][0] = *(const Piece*)(smp[rg] + (size_t)(j) * (NW * 128));         \
+            rS[slot][rg][1] = *(const Piece*)((TURN ? smp8[rg] : smp[rg] + 16) + (size_t)(j) * (NW * 128)); \
+            rG[slot][rg] = *(const Piece*)(grp[rg] + (size_t)(j) * (NW * 64));             \
         }                                                                                  \
     }
 #pragma unroll
@@ -775,13 +799,38 @@ __device__ __forceinline__ void gemm_dense16_body(const GemmParams& p, t12_f32x4
     for (int t = 0; t < NBT; t++)
 #pragma unroll
         for (int rg = 0; rg < RG; rg++) acc[t][rg] = t12_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // TURN: a slot's loads -> the wave's buffer -> the operands' lanes (a wave's LDS accesses keep their order: no wait between them)
+    uint8_t* const sm_ = TURN ? turn + wave * d16_turn_bytes(NX) : nullptr;
+    uint8_t* const gr_ = sm_ + 16 * D16_SM;
+    uint8_t* const act_ = gr_ + 16 * D16_GR;
+#define T12_DS_TURN(slot)                                                                                    \
+    _Pragma("unroll") for (int rg = 0; rg < RG; rg++) {                                                      \
+        *(Piece*)(sm_ + (lane >> 3) * D16_SM + (lane & 7) * 16) = rS[slot][rg][0];                           \
+        *(Piece*)(sm_ + (8 + (lane >> 3)) * D16_SM + (lane & 7) * 16) = rS[slot][rg][1];                     \
+        *(Piece*)(gr_ + (lane >> 2) * D16_GR + (lane & 3) * 16) = rG[slot][rg];                              \
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                                               \
+        _Pragma("unroll") for (int h = 0; h < 2; h++) oS[rg][h] = *(const Piece*)(sm_ + n * D16_SM + g * 32 + h * 16); \
+        oG[rg] = *(const Piece*)(gr_ + n * D16_GR + g * 16);                                                 \
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                                               \
+    }                                                                                                        \
+    _Pragma("unroll") for (int t = 0; t < NBT; t++) {                                                        \
+        _Pragma("unroll") for (int i = 0; i < NXP / NBT; i++)                                                \
+            *(Piece*)(act_ + (4 * i + g) * D16_ACT + n * 16) = rX[slot][t * (NXP / NBT) + i][0];             \
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                                               \
+        _Pragma("unroll") for (int q = 0; q < 4; q++)                                                        \
+            oX[t][q] = *(const Piece*)(act_ + min(n, 4 * (NXP / NBT) - 1) * D16_ACT + g * 64 + q * 16);      \
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                                               \
+    }
 #define T12_DS_CONSUME(slot)                                                                                 \
+    Piece oS[RG][2], oG[RG], oX[NBT][4];                                                                     \
+    if constexpr (TURN) { T12_DS_TURN(slot) }                                                                \
     _Pragma("unroll") for (int q = 0; q < 4; q++) {                                                          \
         uint4 xa[NBT];                                                                                       \
-        _Pragma("unroll") for (int t = 0; t < NBT; t++) xa[t] = t12_pair_acts(rX[slot][t][q]);               \
+        _Pragma("unroll") for (int t = 0; t < NBT; t++) xa[t] = t12_pair_acts(__builtin_bit_cast(uint4, TURN ? oX[t][q] : rX[slot][t][TURN ? 0 : q])); \
         _Pragma("unroll") for (int rg = 0; rg < RG; rg++) {                                                  \
-            const uint4 sv = rS[slot][rg][q >> 1];                                                           \
-            const uint32_t gq = q == 0 ? rG[slot][rg].x : (q == 1 ? rG[slot][rg].y : (q == 2 ? rG[slot][rg].z : rG[slot][rg].w)); \
+            const Piece sv = TURN ? oS[rg][q >> 1] : rS[slot][rg][q >> 1];                                       \
+            const Piece gv = TURN ? oG[rg] : rG[slot][rg];                                                       \
+            const uint32_t gq = q == 0 ? gv.x : (q == 1 ? gv.y : (q == 2 ? gv.z : gv.w));                    \
             uint32_t w_[4];                                                                                  \
             if (q & 1) t12_decode8(sv.z, sv.w, gq, be2r[rg], w_);                                            \
             else t12_decode8(sv.x, sv.y, gq, be2r[rg], w_);                                                  \
@@ -811,6 +860,7 @@ __device__ __forceinline__ void gemm_dense16_body(const GemmParams& p, t12_f32x4
     }
 #undef T12_DS_FETCH
 #undef T12_DS_CONSUME
+#undef T12_DS_TURN
 
     // ---- escapes.  Accumulator register r of lane (n, g) in batch tile t is D[batch 16t + 4g + r][row n].
     {
@@ -840,6 +890,7 @@ __device__ __forceinline__ void gemm_dense16_body(const GemmParams& p, t12_f32x4
         }
     }
 
+    if (TURN) __syncthreads();                        // (the reduction takes the other waves' buffers over)
     // ---- the waves' partial tiles, added in wave order; thread (r, l) = (tid / 64, tid % 64) of the first four waves
     //      finishes element D[batch 16 t + 4 (l / 16) + r][row l % 16] of every batch tile and row group
 #pragma unroll
@@ -876,6 +927,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_dense16_kernel(const GemmParams 
 {
     __shared__ t12_f32x4 red[NBT * RG][NW][64];
     gemm_dense16_body<NW, D, RG, DEV, NBT>(p, red);
+}
+
+// The sweep with its loads turned through LDS, B <= 4 NX NBT.
+template <int NW, int D, int NX, int RG = 1, int NBT = 1>
+__global__ __launch_bounds__(NW * 64) void gemm_dense16_turned_kernel(const GemmParams p)
+{
+    constexpr int BYTES = d16_turn_bytes(NX) * NW, RED = RG * NBT * NW * 64 * 16;      // (the reduction takes the buffers over)
+    __shared__ __align__(16) uint8_t turn[BYTES > RED ? BYTES : RED];
+    gemm_dense16_body<NW, D, RG, false, NBT, false, NX>(p, (t12_f32x4(*)[NW][64])turn, turn);
 }
 
 // The sweep over one gate / up pair with the SiLU * mul in its last step (blockIdx.x counts sets of 16 RG / 2 rows).
@@ -1534,7 +1594,8 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         // 17 .. 32 batch rows on tensors of few rows, which the plan above left to the sweep (or whose planes the ring kernel cannot
         // copy): the sweep of up to 16 rows with two batch tiles per weight load and decode.  One round of workgroups takes
         // ~4.5 us + (K / 4096) (3.7 + 0.2 B) us whatever the row count, because every workgroup reads all B activation rows
-        // for its 16 (32) weight rows.  Measured at B = 17 / 24 / 32: 4096 x 4096 11.7 / 12.7 / 14.6 us, 4096 x 2048 7.6 / 8.5 / 9.1.
+        // for its 16 (32) weight rows.  Measured at B = 17 / 24 / 32: 4096 x 4096 10.4 / 11.0 / 11.3 us (12.0 / 13.1 / 14.4 before the turn
+        // through LDS, which the rule was fitted to).
         int groups16 = 0, sets2 = 0;
         for (int i = 0; i < nseg; i++) {
             groups16 += (segs[i].M + 15) / 16;
@@ -1550,8 +1611,8 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
             p.blk_start[nseg] = groups;
             p.ksplit = 1;
             p.kslice = K;
-            if (rg == 2) hipLaunchKernelGGL((gemm_dense16_kernel<8, 2, 2, false, 2>), dim3(groups), dim3(512), 0, st, p);
-            else hipLaunchKernelGGL((gemm_dense16_kernel<8, 2, 1, false, 2>), dim3(groups), dim3(512), 0, st, p);
+            if (rg == 2) hipLaunchKernelGGL((gemm_dense16_turned_kernel<8, 2, 4, 2, 2>), dim3(groups), dim3(512), 0, st, p);
+            else hipLaunchKernelGGL((gemm_dense16_turned_kernel<8, 2, 4, 1, 2>), dim3(groups), dim3(512), 0, st, p);
             T12_CHECK_LAUNCH("t12_gemm(dense16, two batch tiles)");
             return T12_OK;
         }
@@ -1578,7 +1639,9 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         p.kslice = K;
         if (rg == 4) hipLaunchKernelGGL((gemm_dense16_kernel<8, 2, 4>), dim3(groups), dim3(512), 0, st, p);
         else if (rg == 2) hipLaunchKernelGGL((gemm_dense16_kernel<8, 2, 2>), dim3(groups), dim3(512), 0, st, p);
-        else hipLaunchKernelGGL((gemm_dense16_kernel<8, 2, 1>), dim3(groups), dim3(512), 0, st, p);
+        else if (B <= 4) hipLaunchKernelGGL((gemm_dense16_turned_kernel<8, 2, 1>), dim3(groups), dim3(512), 0, st, p);
+        else if (B <= 8) hipLaunchKernelGGL((gemm_dense16_turned_kernel<8, 2, 2>), dim3(groups), dim3(512), 0, st, p);
+        else hipLaunchKernelGGL((gemm_dense16_turned_kernel<8, 2, 4>), dim3(groups), dim3(512), 0, st, p);
         T12_CHECK_LAUNCH("t12_gemm(dense16)");
         return T12_OK;
     }
