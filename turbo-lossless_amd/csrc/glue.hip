@@ -23,7 +23,6 @@
 #include <utility>
 #include <vector>
 
-#include "t12_act.h"
 #include "t12_device.h"
 #include "t12_host.h"
 
@@ -218,15 +217,15 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
     if (i + 3 < total) {
         const float4 g = *(const float4*)(gate + i);
         const float4 u = *(const float4*)(up + i);
-        const uint32_t lo = t12_f32_to_bf16(t12_gate(g.x, g.x) * u.x) |
-                            ((uint32_t)t12_f32_to_bf16(t12_gate(g.y, g.y) * u.y) << 16);
-        const uint32_t hi = t12_f32_to_bf16(t12_gate(g.z, g.z) * u.z) |
-                            ((uint32_t)t12_f32_to_bf16(t12_gate(g.w, g.w) * u.w) << 16);
+        const uint32_t lo = t12_f32_to_bf16(g.x / (1.0f + expf(-g.x)) * u.x) |
+                            ((uint32_t)t12_f32_to_bf16(g.y / (1.0f + expf(-g.y)) * u.y) << 16);
+        const uint32_t hi = t12_f32_to_bf16(g.z / (1.0f + expf(-g.z)) * u.z) |
+                            ((uint32_t)t12_f32_to_bf16(g.w / (1.0f + expf(-g.w)) * u.w) << 16);
         *(uint2*)(out + i) = make_uint2(lo, hi);
     } else {
         for (size_t j = i; j < total; j++) {
             const float g = gate[j];
-            out[j] = t12_f32_to_bf16(t12_gate(g, g) * up[j]);
+            out[j] = t12_f32_to_bf16(g / (1.0f + expf(-g)) * up[j]);
         }
     }
 }
