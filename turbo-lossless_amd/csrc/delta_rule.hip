@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "delta_plan.h"
 #include "delta_rule.h"
 #include "t12_act.h"
 #include "t12_device.h"
@@ -24,14 +25,6 @@
 using namespace delta_rule;
 
 namespace {
-
-constexpr int CHUNK_FLOATS = 6 * 16 * 64 + 64;
-// Fewest tokens taken in chunks, whole calls of 16 heads of 64, token by token against chunks: 31 / 33 tokens 15.4 / 15.9 us against 16.1 / 16.1,
-// 64 / 100 / 512 tokens 19.4 / 24.5 / 72.6 against 15.8 / 18.3 / 37.7 (64 heads: 105.5 against 60.9).
-constexpr int CHUNK_FROM = 40;
-// The most a chunk's floats come to per token of a run: 49 tokens are four chunks.
-constexpr int CHUNK_ROW = (4 * CHUNK_FLOATS + 48) / 49;
-static_assert(CHUNK_FROM > 33 && CHUNK_FROM <= 49, "CHUNK_ROW is that of the shortest run of four chunks");
 
 // Workgroup = 16 tokens of one head.  Dynamic LDS: tanh(w1) [rank][16].
 constexpr int PREP_TOK = 16;
@@ -281,7 +274,6 @@ __global__ __launch_bounds__(64) void delta_run_direct_kernel(const DeltaParams 
 // formed without the tokens from it on, their outputs and the state behind the chunk are NaN, as the norm over a head's
 // outputs makes them anyway.  (An r that is not finite stays in its own token's row.)
 // ---------------------------------------------------------------------------------------------------------------------
-constexpr int CHUNK = 16, CD = 64;
 constexpr int CDP = CD + 4, CP = CHUNK + 4;                // LDS rows of 68 and 20 floats: sixteen rows read 16 bytes each over all banks
 // A chunk in the workspace, [head][chunk][CHUNK_FLOATS]: TU, RU, -A~, K~, v, Y of 16 x 64 floats each, in the order in which the scan's waves take
 // them (a wave's load is one stretch of 1 KB; row by row they were 4 to 16 pieces, and the scan waited for its cache), then P [64].
@@ -699,9 +691,7 @@ int t12_delta_rule(const T12DeltaRule* d, const float* in, const float* bias, in
     p.run = run;
     p.out_scale = out_scale;
     p.rec = work;
-    // (the factors of a chunk are those of decay rates up to one; heads of 16 channels: sums so short that token by token is the more
-    // exact, 1.37e-7 against 1.46e-7 over 48 tokens; 2^20 tokens: 32-bit offsets in the scan)
-    const bool chunked = run && d->dim_p == 64 && d->dim >= 32 && n >= CHUNK_FROM && n <= 1 << 20 && d->decay_rate >= 0.0f && d->decay_rate <= 1.0f;
+    const bool chunked = run && d->dim_p == CD && takes_chunks(d->heads, d->dim, n, d->decay_rate);
     p.o = work + (size_t)n * d->heads * (chunked ? CHUNK_ROW : rec_floats(d->dim_p));
     p.out = out;
     p.out_ld = out_ld;
