@@ -135,7 +135,7 @@ int t12_window_attention(const T12WindowAttn* a, const float* in, const float* b
 
 /* ---- generalized delta rule --------------------------------------------------------------------------------------
  * Per head, with u = k / sqrt(sum k^2 + unit_eps), removal rate a = sigmoid(a_in), decay
- * w = exp(-decay_rate * sigmoid(W2 tanh(w1_in) + w0)), all per key channel, 32-bit throughout:
+ * w = exp(-decay_rate * sigmoid(W2 tanh(w1_in) + w0)), all per key channel, 32-bit (runs of many tokens: 64-bit inside):
  *     S <- diag(w) S - (a u) (u^T S) + k v^T   (both terms read the old S),    o = S^T r
  *     out = out_scale * norm_w * (o / sqrt(mean(o^2) + out_eps)) * sigmoid(g)
  * A row at position 0 starts from S = 0, whatever its region holds. */

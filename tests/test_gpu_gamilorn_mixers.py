@@ -238,10 +238,10 @@ class Delta:
             self.parity[g] ^= 1
         return out.float().cpu().numpy().astype(np.float64)
 
-    def oracle(self, x, S=None):
+    def oracle(self, x, S=None, rate=np.exp(-0.5)):
         n, hd, heads = len(x), self.N * self.D, lambda y: y.reshape(len(x), self.N, self.D)
         r, k, v, a, g = (x[:, i * hd:(i + 1) * hd] for i in range(5))
-        w = np.exp(-np.exp(-0.5) * go.sigmoid(np.tanh(x[:, 5 * hd:]) @ self.w2.T + self.w0))
+        w = np.exp(-rate * go.sigmoid(np.tanh(x[:, 5 * hd:]) @ self.w2.T + self.w0))
         S = np.zeros((self.N, self.D, self.D)) if S is None else S
         o, S = go.delta_scan(heads(r), heads(k), heads(v), heads(w), heads(go.sigmoid(a)), S)
         return go.delta_output(o, g, self.norm, 1e-5), S
@@ -264,8 +264,8 @@ def test_delta_scan_matches_the_oracle_in_any_portions(t12, heads, dim, rank):
 @pytest.mark.parametrize("heads, dim", [(2, 64), (1, 128), (24, 64), (25, 64), (40, 24)])
 @pytest.mark.parametrize("n", [1, 4, 5, 15, 16, 17, 20, 21, 31, 32, 33, 36, 37, 47, 63, 101])
 def test_delta_scan_of_runs_that_end_inside_a_chunk(t12, heads, dim, n):
-    """Chunks of 16 or 32 tokens (32 up to 192 workgroups of eight columns: 24 heads of 64), then up to four last tokens from memory
-    or more of them through LDS, then one more call on the state that is left."""
+    """Token by token: sixteen at a time through LDS, then up to four last tokens from memory or more of them through LDS.  In chunks (52
+    tokens and more of heads of 64): a last chunk of fewer tokens.  Then one more call on the state that is left."""
     D = Delta(t12, heads, dim, 3)
     x = np.random.default_rng(n).standard_normal((n + 6, D.ld))
     want, _ = D.oracle(x)
@@ -273,11 +273,11 @@ def test_delta_scan_of_runs_that_end_inside_a_chunk(t12, heads, dim, n):
     assert rel_err(D.feed(x[n:], range(n, n + 6), 0), want[n:]) < 1e-4
 
 
-@pytest.mark.parametrize("heads, dim, rank", [(2, 64, 64), (3, 48, 65), (1, 32, 5), (2, 33, 1), (1, 31, 3)])
-@pytest.mark.parametrize("n", [39, 40, 48, 49, 64, 65, 113])
+@pytest.mark.parametrize("heads, dim, rank", [(2, 64, 64), (3, 48, 65), (1, 32, 5), (2, 33, 1), (1, 31, 3), (1, 64, 512), (1, 40, 449)])
+@pytest.mark.parametrize("n", [39, 40, 48, 49, 51, 52, 64, 65, 81, 100, 113])
 @pytest.mark.parametrize("decay", [0.0, float(np.exp(-0.5)), 1.0, 1.5])
 def test_delta_chunks_equal_the_tokens_one_by_one(t12, heads, dim, rank, n, decay):
-    """Runs of 40 tokens and more of heads of 32 to 64 channels go through the chunked kernels at decay rates up to one, portions of
+    """Runs of 52 tokens and more of heads of 32 to 64 channels go through the chunked kernels at decay rates up to one, portions of
     13 token by token: same outputs, same state, from a state that is not zero."""
     x = np.random.default_rng(n + dim).standard_normal((n + 7, Delta(t12, heads, dim, rank).ld))
     x[20, dim * heads] = 30.0                                          # a key that dwarfs the others
@@ -294,6 +294,47 @@ def test_delta_chunks_equal_the_tokens_one_by_one(t12, heads, dim, rank, n, deca
     # (32-bit sums of up to 64 terms, state and outputs of the order of their terms: some 1e-7 each)
     assert rel_err(got[0][1], got[1][1]) < 1e-5
     assert rel_err(got[0][0], got[1][0]) < 1e-5
+
+
+@pytest.mark.parametrize("alike, removal", [(0.0, 0.0), (0.9, 0.0), (0.9, 3.0), (0.99, 3.0), (0.999, 8.0)])
+@pytest.mark.parametrize("rate", [0.0, float(np.exp(-0.5)), 1.0])
+@pytest.mark.parametrize("dim", [32, 64])
+def test_delta_chunks_are_as_exact_as_the_tokens_one_by_one(t12, dim, rate, alike, removal):
+    """Against 64 bits, for keys that resemble each other and removal rates near one as well: there a token takes away most of what the one
+    before it put in, and a sum over a chunk's tokens is much larger than what is left of it."""
+    n, heads = 304, 4
+    rng = np.random.default_rng(dim)
+    D = Delta(t12, heads, dim, 16)
+    hd = heads * dim
+    x = rng.standard_normal((n, D.ld))
+    base = rng.standard_normal((heads, dim))
+    x[:, hd:2 * hd] = (np.sqrt(alike) * base + np.sqrt(1 - alike) * x[:, hd:2 * hd].reshape(n, heads, dim)).reshape(n, hd)
+    x[:, 3 * hd:4 * hd] += removal
+    x = np.round(x * 4096) / 4096                                      # (what the kernels add a bias of a quarter back to, exactly)
+    D.w2, D.w0, D.norm = (y.astype(np.float32).astype(np.float64) for y in (D.w2, D.w0, D.norm))
+    want, S = D.oracle(x, rate=rate)
+    err = []
+    for cuts in ([n], [38] * 8):
+        D = Delta(t12, heads, dim, 16)
+        D.d.decay_rate = rate
+        got = np.concatenate([D.feed(x[i * cuts[0]:i * cuts[0] + c], range(i * cuts[0], i * cuts[0] + c), 0) for i, c in enumerate(cuts)])
+        state = D.state.view(2, heads, dim, -1)[D.parity[0]].cpu().numpy()[:, :, :dim].transpose(0, 2, 1).astype(np.float64)
+        err.append([np.linalg.norm(got - want) / np.linalg.norm(want), np.linalg.norm(state - S) / np.linalg.norm(S)])
+    # (the inputs' own rounding, in both; the recurrence's share is 0.5 to 0.9 of that of the tokens one by one)
+    print("outputs %.2e %.2e state %.2e %.2e" % (err[0][0], err[1][0], err[0][1], err[1][1]))
+    assert err[0][0] <= 1.05 * err[1][0] and err[0][1] <= 1.05 * err[1][1], err
+
+
+def test_large_finite_tokens_leave_those_before_them_alone(t12):
+    """Keys and values whose products 32 bits cannot hold: what they put into the state is not finite, the outputs before them are."""
+    D, n, at = Delta(t12, 2, 64, 8), 64, 37
+    x = np.random.default_rng(6).standard_normal((n, D.ld))
+    want = D.feed(x, range(n), 0)
+    x[at, D.d.k_off + 64:D.d.k_off + 128] *= 1e15
+    x[at, D.d.v_off + 64:D.d.v_off + 128] *= 1e25
+    got = D.feed(x, range(n), 0)
+    assert np.array_equal(got[:at], want[:at]) and np.array_equal(got[:, :64], want[:, :64])
+    assert not np.isfinite(got[at + 1, 64:]).all()
 
 
 @pytest.mark.parametrize("field", ["k", "v", "a", "w1", "r"])

@@ -11,10 +11,11 @@
 // S_new^T r = S^T (w r) - (r . a u) (u^T S) + (r . k) v, so that of a token's two reductions only u^T S is in the way of
 // the next token; the other one is put off and taken for sixteen tokens at once.
 //
-// Runs of heads of 32 to 64 channels take sixteen tokens at a time instead (CHUNK below), on the matrix cores.
+// Runs of heads of 32 to 64 channels take sixteen tokens at a time instead (delta_plan.h), on the matrix cores.
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "delta_plan.h"
 #include "delta_rule.h"
@@ -261,43 +262,55 @@ __global__ __launch_bounds__(64) void delta_run_direct_kernel(const DeltaParams 
 // and everything but S0 is known beforehand: delta_chunk_kernel forms it for all chunks side by side, and what is left of the chain
 // is two dependent products of 16 x 16 x 64 per sixteen tokens (delta_scan_kernel) in place of sixteen reductions.
 //
-// 1 / P_s stays below e^(16 decay_rate): the path is for decay rates up to one (9e6 at most; 1.6e4 at e^-0.5).  All in 32 bits: the fp32
-// matrix instruction multiplies and adds like FMAs, and S is rounded once per chunk instead of three times per token.  Error of
-// outputs / state against 64 bits, mean of eight inputs, 16 heads of 64 over 512 tokens: 2.34e-7 / 2.70e-7, token by token 2.47e-7 / 2.85e-7;
-// 4 heads of 32 over 300: 1.80e-7 / 1.70e-7 and 1.83e-7 / 1.76e-7.
+// 1 / P_s stays below e^(16 decay_rate): the path is for decay rates up to one (9e6 at most; 1.6e4 at e^-0.5).
 //
-// Times (16 heads of 64, 512 tokens): delta_chunk_kernel 17 us, two workgroups per CU, each a serial chain of its own (memory, sums over 64 channels, the
-// triangular solution); delta_scan_kernel 18.6, 0.58 us per chunk: two products of four dependent matrix instructions and one
-// exchange through LDS.  Token by token they were 12 and 67.
+// Where keys resemble each other, a token takes away most of what the one before it put in: K~^T v and A~^T z, sums over sixteen tokens, are much
+// larger than their difference, and Y comes out of such differences too.  In 32 bits that was 1.3 to 4 times the error of the rule token by
+// token, which rounds after every difference.  So a chunk is formed in 64 bits (each operand rounded once, when it is stored), and the scan takes the
+// two products into S on the 64-bit matrix instruction and keeps S itself in 64 bits over the run; z and o, sums of like size, stay on
+// the 32-bit one.  Products that 32 bits cannot hold then do no harm to the tokens before them either.  Error against 64 bits, outputs and state,
+// chunks / token by token (4 heads of 64, 304 tokens, decay rate e^-0.5; the inputs' rounding is in both): independent keys 2.05e-7 / 2.37e-7 and
+// 2.57e-7 / 2.89e-7, cosine 0.9 2.81e-7 / 3.21e-7 and 4.53e-7 / 4.82e-7, 0.999 and removal near one 4.94e-7 / 6.07e-7 and 3.08e-7 / 3.47e-7.
+//
+// Times (16 heads of 64, 512 tokens): delta_chunk_kernel 18.6 us (17.6 in 32 bits), two workgroups per CU, each a serial chain of its own (memory,
+// sums over 64 channels, the triangular solution); delta_scan_kernel 25 (18.6), 0.78 us per chunk: two products of four dependent matrix
+// instructions, 64 cycles each in the second, and one exchange through LDS.  Token by token they were 12 and 67.
 //
 // A token that is not finite (in k, a, w or v) must not reach the tokens before it, which a product with a zero would do: the chunk is
 // formed without the tokens from it on, their outputs and the state behind the chunk are NaN, as the norm over a head's
 // outputs makes them anyway.  (An r that is not finite stays in its own token's row.)
 // ---------------------------------------------------------------------------------------------------------------------
-constexpr int CDP = CD + 4, CP = CHUNK + 4;                // LDS rows of 68 and 20 floats: sixteen rows read 16 bytes each over all banks
+// LDS rows of 66 and 18 doubles: sixteen rows read 16 bytes each over all banks.
+constexpr int CDP = CD + 2, CP = CHUNK + 2, CV = CD + 4;
 // A chunk in the workspace, [head][chunk][CHUNK_FLOATS]: TU, RU, -A~, K~, v, Y of 16 x 64 floats each, in the order in which the scan's waves take
 // them (a wave's load is one stretch of 1 KB; row by row they were 4 to 16 pieces, and the scan waited for its cache), then P [64].
 //   token order (-A~, K~, v, Y): [channel / 16][token / 4][channel % 16][token % 4]
-//   key order   (TU, RU):        [channel / 16][channel / 4 % 4][token][channel % 4]
+//   key order   (TU, RU):        [channel / 16][channel % 4][token][channel / 4 % 4];  P: [channel / 16][channel % 4][channel / 4 % 4]
+// (Register e of lane 16 g + m is row 4 g + e of a 32-bit product's result and row 4 e + g of a 64-bit one's: z is 32-bit, S 64-bit.)
 enum { C_TU, C_RU, C_NA, C_K, C_V, C_Y, C_P };
 constexpr int C_ARRAY = CHUNK * CD;
 
-// x times a 64-bit factor given as the sum of two floats
-struct Factor {
-    float hi, lo;
-    __device__ __forceinline__ explicit Factor(double x) : hi((float)x), lo((float)(x - (double)(float)x)) {}
-    __device__ __forceinline__ float operator*(float x) const { return fmaf(x, hi, x * lo); }     // (rounded once)
-};
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ f64x4 mfma64(double a, double b, f64x4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ t12_f32x4 mfma32(float a, float b, t12_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+// four neighbouring doubles of LDS
+__device__ __forceinline__ f64x4 four_doubles(const double* x)
+{
+    const f64x2 lo = *(const f64x2*)x, hi = *(const f64x2*)(x + 2);
+    return f64x4{lo[0], lo[1], hi[0], hi[1]};
+}
 
 // Workgroup = one chunk of one head.  Wave w has the channels 16 w .. 16 w + 15, lane group g of it the tokens 4 g .. 4 g + 3: where the
-// matrix product with W2 leaves them.  Dynamic LDS: tanh(w1) [16][rank rounded up to 64, + 4].
+// matrix product with W2 leaves them.
 __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
 {
-    extern __shared__ float4 th4[];
-    float* th = (float*)th4;
-    __shared__ __align__(16) float us[CHUNK * CDP], as[CHUNK * CDP], ks[CHUNK * CDP], rs[CHUNK * CDP], vs[CHUNK * CDP], pair[4][CHUNK * CP];
-    __shared__ float norm[4][CHUNK];
+    __shared__ __align__(16) double token[4][CHUNK * CDP], pair[4][CHUNK * CP];
+    __shared__ float vs[CHUNK * CV], norm[4][CHUNK];
     __shared__ int bad;
+    double *const us = token[0], *const as = token[1], *const ks = token[2], *const rs = token[3];
+    float* const th = (float*)token;                       // tanh(w1) [16][rank rounded up to 64, + 4], before the tokens' vectors
+    static_assert(CHUNK * (CHUNK_MAX_RANK + 4) * sizeof(float) <= sizeof(token) && CHUNK_MAX_RANK % 64 == 0, "tanh(w1) in the place of the vectors");
     const T12DeltaRule& d = p.d;
     const int head = blockIdx.y, t0 = blockIdx.x * CHUNK, nt = min(CHUNK, p.n - t0);
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, m = lane & 15, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -339,7 +352,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
 #pragma unroll
                 for (int e = 0; e < 16; e++) w2[e] = w2_at(q0, e);
 #pragma unroll
-            for (int e = 0; e < 16; e++) z = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q0 + (e & 12) * 4 + (e & 3)], w2[e], z, 0, 0, 0);
+            for (int e = 0; e < 16; e++) z = mfma32(x[q0 + (e & 12) * 4 + (e & 3)], w2[e], z);
         }
     }
     double own = 1.0;                                      // decay of the thread's four tokens
@@ -359,7 +372,6 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
         if (!in) k[j] = a[j] = v[j] = 0.0f;
         own *= w[j];
     }
-    // (64-bit products of the decays: every scaled operand is rounded once)
     double before = 1.0, after = 1.0, all = 1.0;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -377,9 +389,8 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
 #pragma unroll
         for (int j = 3; j >= 0; j--) {
             if (g * 4 + j >= first_bad) k[j] = a[j] = v[j] = z[j] = 0.0f;
-            const Factor tail(after);                      // decay of the tokens behind this one
-            na[j] = -(tail * a[j]);
-            kt[j] = tail * k[j];
+            na[j] = (float)(-after * (double)a[j]);        // (after: decay of the tokens behind this one)
+            kt[j] = (float)(after * (double)k[j]);
             vt[j] = v[j];
             after *= w[j];
         }
@@ -390,102 +401,103 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int at = (g * 4 + j) * CDP + ch;
-        us[at] = Factor(before) * z[j];
+        us[at] = before * (double)z[j];
         before *= w[j];
-        const Factor here(before);
-        const float guess = 1.0f / here.hi;                // 1 / before: what is left of one step from there
-        const Factor back(fma((double)guess, fma(-before, (double)guess, 1.0), (double)guess));
-        as[at] = back * a[j];
-        ks[at] = back * k[j];
-        rs[at] = here * r[j];
-        vs[at] = v[j];
+        const double guess = (double)(1.0f / (float)before);   // 1 / before to 24 bits, and to 48 with what is left of one step from there
+        const double back = fma(guess, fma(-before, guess, 1.0), guess);
+        as[at] = back * (double)a[j];
+        ks[at] = back * (double)k[j];
+        rs[at] = before * (double)r[j];
+        vs[(g * 4 + j) * CV + ch] = v[j];
     }
-    if (g == 0) chunk[C_P * C_ARRAY + ch] = first_bad < CHUNK ? __builtin_nanf("") : (float)all;
+    if (g == 0) chunk[C_P * C_ARRAY + wave * 16 + (m & 3) * 4 + (m >> 2)] = first_bad < CHUNK ? __builtin_nanf("") : (float)all;
     __syncthreads();
     {
         // wave 0: u~ . a / P (token, earlier token; the other way round in LDS), 1: u~ . k / P, 2: - r~ . a / P, 3: r~ . k / P
-        const float *x = (wave < 2 ? us : rs) + m * CDP + g * 4, *y = (wave & 1 ? ks : as) + m * CDP + g * 4;
-        t12_f32x4 part[8], acc;                            // (short sums: the products of a long one would each be rounded to the size of all)
+        const double *x = (wave < 2 ? us : rs) + m * CDP + g * 4, *y = (wave & 1 ? ks : as) + m * CDP + g * 4;
+        f64x4 c[2] = {(f64x4)(0.0), (f64x4)(0.0)};
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const t12_f32x4 xa = *(const t12_f32x4*)(x + q * 16), yb = *(const t12_f32x4*)(y + q * 16);
+            const f64x4 xa = four_doubles(x + q * 16), yb = four_doubles(y + q * 16);
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                part[q * 2 + e / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[e], yb[e], e & 1 ? part[q * 2 + e / 2] : (t12_f32x4)(0.0f), 0, 0, 0);
+            for (int e = 0; e < 4; e++) c[e & 1] = mfma64(xa[e], yb[e], c[e & 1]);
         }
-        acc = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+        c[0] += c[1];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int t = g * 4 + e;
-            const float c = m < t + (wave >> 1) ? acc[e] : 0.0f;
-            pair[wave][wave ? t * CP + m : m * CP + t] = wave == 2 ? -c : c;
+            const int t = e * 4 + g;
+            const double x_ = m < t + (wave >> 1) ? c[0][e] : 0.0;
+            pair[wave][wave ? t * CP + m : m * CP + t] = wave == 2 ? -x_ : x_;
         }
     }
     __syncthreads();
     // the v terms, sixteen value channels per wave; that of z goes where k was
-    t12_f32x4 bv4 = (t12_f32x4)(0.0f), lv = (t12_f32x4)(0.0f);
+    f64x4 bv4 = (f64x4)(0.0), lv = (f64x4)(0.0);
     {
-        const t12_f32x4 cb = *(const t12_f32x4*)(pair[1] + m * CP + g * 4), cl = *(const t12_f32x4*)(pair[3] + m * CP + g * 4);
+        const f64x4 cb = four_doubles(pair[1] + m * CP + g * 4), cl = four_doubles(pair[3] + m * CP + g * 4);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const float x = vs[(g * 4 + e) * CDP + wave * 16 + m];
-            bv4 = __builtin_amdgcn_mfma_f32_16x16x4f32(cb[e], x, bv4, 0, 0, 0);
-            lv = __builtin_amdgcn_mfma_f32_16x16x4f32(cl[e], x, lv, 0, 0, 0);
+            const double x = (double)vs[(g * 4 + e) * CV + ch];
+            bv4 = mfma64(cb[e], x, bv4);
+            lv = mfma64(cl[e], x, lv);
         }
 #pragma unroll
-        for (int e = 0; e < 4; e++) ks[(g * 4 + e) * CDP + wave * 16 + m] = bv4[e];
+        for (int e = 0; e < 4; e++) ks[(e * 4 + g) * CDP + ch] = bv4[e];
     }
     __syncthreads();
     if (wave < 2) {                                        // wave 0: the columns of u~, wave 1: those of the v term; solved in place
-        float* col = (wave ? ks : us) + lane;
-        float x[CHUNK];
+        double* col = (wave ? ks : us) + lane;
+        double x[CHUNK];
 #pragma unroll
         for (int t = 0; t < CHUNK; t++) x[t] = col[t * CDP];
 #pragma unroll
         for (int t = 0; t < CHUNK; t++) {
 #pragma unroll
-            for (int q = 0; q < CHUNK / 4; q++)
-                if (q * 4 + 3 > t) {
-                    const t12_f32x4 c = *(const t12_f32x4*)(pair[0] + t * CP + q * 4);
+            for (int q = 0; q < CHUNK / 2; q++)
+                if (q * 2 + 1 > t) {
+                    const f64x2 c = *(const f64x2*)(pair[0] + t * CP + q * 2);
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (q * 4 + e > t) x[q * 4 + e] -= c[e] * x[t];
+                    for (int e = 0; e < 2; e++)
+                        if (q * 2 + e > t) x[q * 2 + e] = fma(-c[e], x[t], x[q * 2 + e]);
                 }
             col[t * CDP] = x[t];
         }
     }
     __syncthreads();
     // what a token takes off its own output and off that of those behind it: sixteen columns each of RU and of Q per wave
-    t12_f32x4 ru = (t12_f32x4)(0.0f), taken = (t12_f32x4)(0.0f), y;
+    f64x4 ru = (f64x4)(0.0);
+    t12_f32x4 y, tu;
     {
-        const t12_f32x4 cm = *(const t12_f32x4*)(pair[2] + m * CP + g * 4);
+        const f64x4 cm = four_doubles(pair[2] + m * CP + g * 4);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int at = (g * 4 + e) * CDP + ch;
-            y[e] = ks[at];
-            ru = __builtin_amdgcn_mfma_f32_16x16x4f32(cm[e], us[at], ru, 0, 0, 0);
-            taken = __builtin_amdgcn_mfma_f32_16x16x4f32(cm[e], y[e], taken, 0, 0, 0);
+            const int t = g * 4 + e;
+            const double x = ks[t * CDP + ch];
+            ru = mfma64(cm[e], us[t * CDP + ch], ru);
+            lv = mfma64(cm[e], x, lv);
+            y[e] = (float)x;
         }
     }
-#pragma unroll
-    for (int e = 0; e < 4; e++) ru[e] += rs[(g * 4 + e) * CDP + ch];
-    lv += taken;
     *(t12_f32x4*)(out + C_Y * C_ARRAY) = y;
-    *(t12_f32x4*)(out + C_TU * C_ARRAY) = *(const t12_f32x4*)(us + m * CDP + wave * 16 + g * 4);
 #pragma unroll
-    for (int e = 0; e < 4; e++) rs[(g * 4 + e) * CDP + ch] = ru[e];      // (turned round inside the wave's own sixteen columns)
+    for (int e = 0; e < 4; e++) tu[e] = (float)us[m * CDP + wave * 16 + e * 4 + g];
+    *(t12_f32x4*)(out + C_TU * C_ARRAY) = tu;
+#pragma unroll
+    for (int e = 0; e < 4; e++) rs[(e * 4 + g) * CDP + ch] += ru[e];     // (turned round inside the wave's own sixteen columns)
     float* o = p.o + ((size_t)t0 * d.heads + head) * D + ch;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        const int t = g * 4 + e;
-        if (t < nt && ch < D) o[(size_t)t * HD] = t < first_bad ? lv[e] : __builtin_nanf("");
+        const int t = e * 4 + g;
+        if (t < nt && ch < D) o[(size_t)t * HD] = t < first_bad ? (float)lv[e] : __builtin_nanf("");
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    *(t12_f32x4*)(out + C_RU * C_ARRAY) = *(const t12_f32x4*)(rs + m * CDP + wave * 16 + g * 4);
+#pragma unroll
+    for (int e = 0; e < 4; e++) tu[e] = (float)rs[m * CDP + wave * 16 + e * 4 + g];
+    *(t12_f32x4*)(out + C_RU * C_ARRAY) = tu;
 }
 
 // What a wave takes of one chunk: operands of its sixteen key channels and sixteen value channels.  The four registers of an operand are
-// the four steps of a product: step e contracts the indices 4 g + e of lane groups g, which is where a product's result has them.
+// the four steps of a product: step e contracts what register e of a result holds, the tokens 4 g + e of z and the keys 4 e + g of S.
 struct ChunkOperands {
     t12_f32x4 tu, ru, na, k, v, y, decay;
     float q;
@@ -531,9 +543,11 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaParams p)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const T12Row first = p.rows[0];
     const size_t region = (size_t)(first.slot >> 1) * 2 * d.state_elems;
-    const size_t cell = ((size_t)head * d.dim + min(j0 + m, d.dim - 1)) * CD + wave * 16 + g * 4;
-    t12_f32x4 S = (t12_f32x4)(0.0f);
-    if (first.position != 0) S = *(const t12_f32x4*)(d.state + region + (size_t)(first.slot & 1) * d.state_elems + cell);
+    const size_t cell = ((size_t)head * d.dim + min(j0 + m, d.dim - 1)) * CD + wave * 16 + g;
+    t12_f32x4 Sf = (t12_f32x4)(0.0f);
+    if (first.position != 0)
+#pragma unroll
+        for (int e = 0; e < 4; e++) Sf[e] = d.state[region + (size_t)(first.slot & 1) * d.state_elems + cell + e * 4];
     const int chunks = (p.n + CHUNK - 1) / CHUNK, o_step = d.heads * d.dim;
     float* o_head = p.o + (size_t)head * d.dim + j0;
     constexpr uint32_t STEP = CHUNK_FLOATS * 4;            // bytes from chunk to chunk
@@ -549,59 +563,83 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaParams p)
         op[f].q = load1(outs, (uint32_t)(f * CHUNK * o_step) * 4 + o_at);
         __builtin_amdgcn_sched_barrier(0);
     }
-    asm volatile("" : "+v"(S));                            // (waited for here, not by a wait at the loop's head that would hold for the others too)
+    asm volatile("" : "+v"(Sf));                           // (waited for here, not by a wait at the loop's head that would hold for the others too)
+    f64x4 S = {Sf[0], Sf[1], Sf[2], Sf[3]};
     const float* ow = (const float*)&os[0][0][lane] + wave;
     // Each wave finishes the outputs of the tokens 4 g + wave of a chunk, one chunk later (and in the end).
     uint32_t store_at = 0xFFFFFFFFu;                       // (outside the buffer: not stored)
     float q = 0.0f;
-    // (chunks past the last one, up to three, are gone through on zeros without their S: with ways out of the loop inside it the
-    // compiler moves the operands' registers about and waits for all of them)
-    for (int c = 0; c < chunks; c += 4) {
+    int c = 0;
+    // chunk c + F of the run, F = (c + F) % 4: the registers its operands are in
+    auto step = [&](auto F) __attribute__((always_inline)) {
+        constexpr int f = decltype(F)::value;
+        ChunkOperands &x = op[f], &y = op[(f + 3) & 3];
+        const int buf = f & 1;
+        const uint32_t ahead = (uint32_t)(c + f + 3) * STEP;
+        t12_f32x4 z = (t12_f32x4)(0.0f), o = (t12_f32x4)(0.0f);
+        f64x4 to_s = (f64x4)(0.0);
 #pragma unroll
-        for (int f = 0; f < 4; f++) {
-            ChunkOperands &x = op[f], &y = op[(f + 3) & 3];
-            const int buf = f & 1;
-            const uint32_t ahead = (uint32_t)(c + f + 3) * STEP;
-            t12_f32x4 z = (t12_f32x4)(0.0f), o = (t12_f32x4)(0.0f), in = (t12_f32x4)(0.0f), out = (t12_f32x4)(0.0f);
+        for (int e = 0; e < 4; e++) z = mfma32(x.tu[e], Sf[e], z);
+        __builtin_amdgcn_sched_barrier(0);                 // (the matrix cores have work while z crosses)
+        to_s = mfma64((double)x.k[0], (double)x.v[0], to_s);
+        __builtin_amdgcn_sched_barrier(0);
+        zs[buf][wave][lane] = z;
+        __builtin_amdgcn_sched_barrier(0);
+        to_s = mfma64((double)x.k[1], (double)x.v[1], to_s);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();                                   // (a buffer is written again two chunks on, behind the next barrier)
+        t12_f32x4 part[4];
+        float done[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) z = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tu[e], S[e], z, 0, 0, 0);
-            zs[buf][wave][lane] = z;
-            __syncthreads();                               // (a buffer is written again two chunks on, behind the next barrier)
-            t12_f32x4 part[4];
-            float done[4];
+        for (int w = 0; w < 4; w++) part[w] = zs[buf][w][lane];
 #pragma unroll
-            for (int w = 0; w < 4; w++) part[w] = zs[buf][w][lane];
+        for (int w = 0; w < 4; w++) done[w] = ow[(buf ^ 1) * 1024 + w * 256];
+        // what the chain does not need runs while these are on their way
 #pragma unroll
-            for (int w = 0; w < 4; w++) done[w] = ow[(buf ^ 1) * 1024 + w * 256];
-            // what the chain does not need runs while these are on their way
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                __builtin_amdgcn_sched_barrier(0);
-                in = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[e], x.v[e], in, 0, 0, 0);
-                request_step(y, e, operands, ahead + keys, ahead + values, ahead + decay);
-                o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.ru[e], S[e], o, 0, 0, 0);
-            }
+        for (int e = 0; e < 4; e++) {
             __builtin_amdgcn_sched_barrier(0);
-            z = (part[0] + part[1]) + (part[2] + part[3]);
-#pragma unroll
-            for (int e = 0; e < 4; e++) z[e] += x.y[e];
-#pragma unroll
-            for (int e = 0; e < 4; e++) out = __builtin_amdgcn_mfma_f32_16x16x4f32(x.na[e], z[e], out, 0, 0, 0);
-            os[buf][wave][lane] = o;
-            store1((done[0] + done[1]) + (done[2] + done[3]) + q, outs, store_at);
-            q = x.q;
-            y.q = load1(outs, (uint32_t)((c + f + 3) * CHUNK * o_step) * 4 + o_at);
-            store_at = j0 + m < d.dim ? (uint32_t)((c + f) * CHUNK * o_step) * 4 + o_at : 0xFFFFFFFFu;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {                  // (S is rounded once per chunk)
-                const float next = fmaf(x.decay[e], S[e], in[e] + out[e]);
-                S[e] = c + f < chunks ? next : S[e];
-            }
+            if (e < 2) to_s = mfma64((double)x.k[e + 2], (double)x.v[e + 2], to_s);
+            request_step(y, e, operands, ahead + keys, ahead + values, ahead + decay);
+            o = mfma32(x.ru[e], Sf[e], o);
         }
+        double na[4], own_y[4], all[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            na[e] = (double)x.na[e];
+            own_y[e] = (double)x.y[e];
+            all[e] = (double)x.decay[e];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        z = (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) to_s = mfma64(na[e], (double)z[e] + own_y[e], to_s);
+        os[buf][wave][lane] = o;
+        store1((done[0] + done[1]) + (done[2] + done[3]) + q, outs, store_at);
+        q = x.q;
+        y.q = load1(outs, (uint32_t)((c + f + 3) * CHUNK * o_step) * 4 + o_at);
+        store_at = j0 + m < d.dim ? (uint32_t)((c + f) * CHUNK * o_step) * 4 + o_at : 0xFFFFFFFFu;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {                      // (in 64 bits over the whole run)
+            S[e] = fma(all[e], S[e], to_s[e]);
+            Sf[e] = (float)S[e];
+        }
+    };
+    // (the last one to three behind the loop: with ways out inside it the compiler moves the operands' registers about and waits for all of them)
+    for (; c + 4 <= chunks; c += 4) {
+        step(std::integral_constant<int, 0>());
+        step(std::integral_constant<int, 1>());
+        step(std::integral_constant<int, 2>());
+        step(std::integral_constant<int, 3>());
     }
+    if (c < chunks) step(std::integral_constant<int, 0>());
+    if (c + 1 < chunks) step(std::integral_constant<int, 1>());
+    if (c + 2 < chunks) step(std::integral_constant<int, 2>());
+    ow += ((chunks - 1) & 1) * 1024;
     __syncthreads();
-    store1((ow[1024] + ow[1280]) + (ow[1536] + ow[1792]) + q, outs, store_at);
-    if (j0 + m < d.dim) *(t12_f32x4*)(d.state + region + (size_t)((first.slot & 1) ^ 1) * d.state_elems + cell) = S;
+    store1((ow[0] + ow[256]) + (ow[512] + ow[768]) + q, outs, store_at);
+    if (j0 + m < d.dim)
+#pragma unroll
+        for (int e = 0; e < 4; e++) d.state[region + (size_t)((first.slot & 1) ^ 1) * d.state_elems + cell + e * 4] = Sf[e];
 }
 
 // One wave per (row, head): o over its RMS, times the plain weight and the sigmoid gate.
@@ -691,14 +729,13 @@ int t12_delta_rule(const T12DeltaRule* d, const float* in, const float* bias, in
     p.run = run;
     p.out_scale = out_scale;
     p.rec = work;
-    const bool chunked = run && d->dim_p == CD && takes_chunks(d->heads, d->dim, n, d->decay_rate);
+    const bool chunked = run && d->dim_p == CD && takes_chunks(d->heads, d->dim, d->rank, n, d->decay_rate);
     p.o = work + (size_t)n * d->heads * (chunked ? CHUNK_ROW : rec_floats(d->dim_p));
     p.out = out;
     p.out_ld = out_ld;
     int rc;
     if (chunked) {
-        hipLaunchKernelGGL(delta_chunk_kernel, dim3((n + CHUNK - 1) / CHUNK, d->heads), dim3(256),
-                           (size_t)CHUNK * (((d->rank + 63) & ~63) + 4) * sizeof(float), st, p);
+        hipLaunchKernelGGL(delta_chunk_kernel, dim3((n + CHUNK - 1) / CHUNK, d->heads), dim3(256), 0, st, p);
         hipLaunchKernelGGL(delta_scan_kernel, dim3(d->heads, (d->dim + 15) / 16), dim3(256), 0, st, p);
         T12_CHECK_LAUNCH("t12_delta_rule(chunks)");
         rc = T12_OK;
