@@ -325,6 +325,25 @@ def test_delta_chunks_are_as_exact_as_the_tokens_one_by_one(t12, dim, rate, alik
     assert err[0][0] <= 1.05 * err[1][0] and err[0][1] <= 1.05 * err[1][1], err
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("dim, at", [(64, 37), (40, 47), (64, 48)])
+def test_a_value_channel_that_is_not_finite_keeps_to_its_column(t12, dim, at, value):
+    """A column of the state never meets another one: only that of the value channel is lost, as token by token."""
+    n, states = 64, []
+    x = np.random.default_rng(7).standard_normal((n, Delta(t12, 2, dim, 8).ld))
+    x[at, 2 * 2 * dim + dim + 5] = value
+    for cuts in ([n], [32, 32]):
+        D, pos = Delta(t12, 2, dim, 8), 0
+        for c in cuts:
+            D.feed(x[pos:pos + c], range(pos, pos + c), 0)
+            pos += c
+        states.append(D.state.view(2, 2, dim, -1)[D.parity[0]].cpu().numpy()[:, :, :dim])
+    assert np.array_equal(np.isfinite(states[0]), np.isfinite(states[1]))
+    lost = ~np.isfinite(states[0])
+    assert lost[1, 5].all() and lost.sum() == dim
+    assert rel_err(states[0][~lost], states[1][~lost]) < 1e-5
+
+
 def test_large_finite_tokens_leave_those_before_them_alone(t12):
     """Keys and values whose products 32 bits cannot hold: what they put into the state is not finite, the outputs before them are."""
     D, n, at = Delta(t12, 2, 64, 8), 64, 37

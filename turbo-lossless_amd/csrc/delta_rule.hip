@@ -276,9 +276,10 @@ __global__ __launch_bounds__(64) void delta_run_direct_kernel(const DeltaParams 
 // sums over 64 channels, the triangular solution); delta_scan_kernel 25 (18.6), 0.78 us per chunk: two products of four dependent matrix
 // instructions, 64 cycles each in the second, and one exchange through LDS.  Token by token they were 12 and 67.
 //
-// A token that is not finite (in k, a, w or v) must not reach the tokens before it, which a product with a zero would do: the chunk is
-// formed without the tokens from it on, their outputs and the state behind the chunk are NaN, as the norm over a head's
-// outputs makes them anyway.  (An r that is not finite stays in its own token's row.)
+// A token that is not finite must not reach the tokens before it, which a product with a zero would do.  In k, a or w: the chunk is formed
+// without the tokens from it on; their outputs and the state behind the chunk are NaN.  In a channel of v: the channel is formed without it, and from that
+// token on its z and its outputs are NaN, which makes its column of the state NaN and no other.  (An r that is not finite stays in its
+// own token's row.)
 // ---------------------------------------------------------------------------------------------------------------------
 // LDS rows of 66 and 18 doubles: sixteen rows read 16 bytes each over all banks.
 constexpr int CDP = CD + 2, CP = CHUNK + 2, CV = CD + 4;
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
 {
     __shared__ __align__(16) double token[4][CHUNK * CDP], pair[4][CHUNK * CP];
     __shared__ float vs[CHUNK * CV], norm[4][CHUNK];
-    __shared__ int bad;
+    __shared__ int bad, bad_v[CD];
     double *const us = token[0], *const as = token[1], *const ks = token[2], *const rs = token[3];
     float* const th = (float*)token;                       // tanh(w1) [16][rank rounded up to 64, + 4], before the tokens' vectors
     static_assert(CHUNK * (CHUNK_MAX_RANK + 4) * sizeof(float) <= sizeof(token) && CHUNK_MAX_RANK % 64 == 0, "tanh(w1) in the place of the vectors");
@@ -332,6 +333,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
 #pragma unroll
     for (int e = 0; e < 16; e++) w2[e] = w2_at(0, e);
     if (tid == 0) bad = CHUNK;
+    if (tid < CD) bad_v[tid] = CHUNK;
     for (int q = tid; q < CHUNK * rank_p; q += 256) {      // (past the rank: zeros)
         const int t = q / rank_p, c = q % rank_p, from = d.w1_off + min(c, rank - 1);
         const float x = tanhf(p.in[(size_t)(t0 + min(t, nt - 1)) * p.ld + from] + p.bias[from]);
@@ -364,12 +366,13 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
         a[j] = t12_sigmoid(a[j] + ba) * u;
         w[j] = expf(-d.decay_rate * t12_sigmoid(z[j] + w0));
         v[j] += bv;
-        const bool fine = __builtin_isfinite(k[j]) && __builtin_isfinite(a[j]) && __builtin_isfinite(w[j]) && __builtin_isfinite(v[j]);
-        if (in && !fine) atomicMin(&bad, t);
+        if (in && !(__builtin_isfinite(k[j]) && __builtin_isfinite(a[j]) && __builtin_isfinite(w[j]))) atomicMin(&bad, t);
+        if (in && !__builtin_isfinite(v[j])) atomicMin(&bad_v[ch], t);
         if (!in || !__builtin_isfinite(w[j])) w[j] = 1.0f; // (tokens and channels that are not there leave the state alone)
+        if (!in || !__builtin_isfinite(v[j])) v[j] = 0.0f;
         r[j] = in ? r[j] + br : 0.0f;
         z[j] = in ? u : 0.0f;                              // from here on: u
-        if (!in) k[j] = a[j] = v[j] = 0.0f;
+        if (!in) k[j] = a[j] = 0.0f;
         own *= w[j];
     }
     double before = 1.0, after = 1.0, all = 1.0;
@@ -467,6 +470,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
     // what a token takes off its own output and off that of those behind it: sixteen columns each of RU and of Q per wave
     f64x4 ru = (f64x4)(0.0);
     t12_f32x4 y, tu;
+    const int first_bad_v = bad_v[ch];
     {
         const f64x4 cm = four_doubles(pair[2] + m * CP + g * 4);
 #pragma unroll
@@ -475,7 +479,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
             const double x = ks[t * CDP + ch];
             ru = mfma64(cm[e], us[t * CDP + ch], ru);
             lv = mfma64(cm[e], x, lv);
-            y[e] = (float)x;
+            y[e] = t < first_bad_v ? (float)x : __builtin_nanf("");
         }
     }
     *(t12_f32x4*)(out + C_Y * C_ARRAY) = y;
@@ -488,7 +492,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaParams p)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const int t = e * 4 + g;
-        if (t < nt && ch < D) o[(size_t)t * HD] = t < first_bad ? (float)lv[e] : __builtin_nanf("");
+        if (t < nt && ch < D) o[(size_t)t * HD] = t < first_bad && t < first_bad_v ? (float)lv[e] : __builtin_nanf("");
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
