@@ -6,6 +6,7 @@ missing, importing this module fails.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 import struct
@@ -283,6 +284,27 @@ def current_stream() -> int:
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
+_IN_ORDER = contextlib.nullcontext()
+
+
+@contextlib.contextmanager
+def _forked(stream):
+    """What is launched on `stream` inside comes behind the work of torch's current stream so far and ahead of what follows there: buffers
+    are the current stream's, taken and given back in its order, and so are the host's reads."""
+    torch = _torch()
+    here = torch.cuda.current_stream()
+    other = torch.cuda.ExternalStream(stream) if stream else torch.cuda.default_stream()
+    other.wait_stream(here)
+    try:
+        yield
+    finally:
+        here.wait_stream(other)
+
+
+def _on(stream):
+    return _IN_ORDER if stream is None or stream == current_stream() else _forked(stream)
+
+
 def _dp(t):
     return None if t is None else t.data_ptr()
 
@@ -390,13 +412,15 @@ def find_base_exp_device(w, stream=None) -> int:
     torch = _torch()
     st = current_stream() if stream is None else stream
     hist = torch.empty(256, dtype=torch.int64, device=w.device)
-    check(lib.t12_pack_histogram(w.data_ptr(), w.numel(), hist.data_ptr(), st), "t12_pack_histogram")
+    with _on(stream):
+        check(lib.t12_pack_histogram(w.data_ptr(), w.numel(), hist.data_ptr(), st), "t12_pack_histogram")
     h = hist.cpu().numpy().astype(np.uint64)       # synchronises
     return int(lib.t12_pack_base_exp(h.ctypes.data_as(C.POINTER(C.c_uint64))))
 
 
 def pack_device(w, base_exp=None, stream=None) -> DeviceTensor12:
-    """Pack a bf16 matrix [M, K] (torch.bfloat16 or int16 bits, on the GPU) into split-12 on the GPU."""
+    """Pack a bf16 matrix [M, K] (torch.bfloat16 or int16 bits, on the GPU) into split-12 on the GPU.  The result is torch's current
+    stream's, on whichever stream the work runs."""
     torch = _torch()
     assert w.dim() == 2 and w.is_contiguous() and w.element_size() == 2
     M, K = w.shape
@@ -410,20 +434,23 @@ def pack_device(w, base_exp=None, stream=None) -> DeviceTensor12:
     row_off = off[:M + 1]
     if base_exp is None:
         hist = torch.empty(256, dtype=torch.int64, device=dev)
-        check(lib.t12_pack_begin(w.data_ptr(), M, K, hist.data_ptr(), off.data_ptr() + 4 * (M + 1), sm.data_ptr(), gr.data_ptr(),
-                                 cnt.data_ptr(), off.data_ptr(), st), "t12_pack_begin")
+        with _on(stream):
+            check(lib.t12_pack_begin(w.data_ptr(), M, K, hist.data_ptr(), off.data_ptr() + 4 * (M + 1), sm.data_ptr(), gr.data_ptr(),
+                                     cnt.data_ptr(), off.data_ptr(), st), "t12_pack_begin")
         P, base_exp = off[M:].tolist()              # synchronises
     else:
-        check(lib.t12_pack_planes(w.data_ptr(), M, K, base_exp, sm.data_ptr(), gr.data_ptr(), cnt.data_ptr(), st),
-              "t12_pack_planes")
-        check(lib.t12_pack_row_offsets(cnt.data_ptr(), M, row_off.data_ptr(), st), "t12_pack_row_offsets")
+        with _on(stream):
+            check(lib.t12_pack_planes(w.data_ptr(), M, K, base_exp, sm.data_ptr(), gr.data_ptr(), cnt.data_ptr(), st),
+                  "t12_pack_planes")
+            check(lib.t12_pack_row_offsets(cnt.data_ptr(), M, row_off.data_ptr(), st), "t12_pack_row_offsets")
         P = int(row_off[M].item())                  # synchronises
     cols = torch.empty(P, dtype=torch.int32, device=dev)
     correct = torch.empty(P, dtype=torch.int16, device=dev)
     wrong = torch.empty(P, dtype=torch.int16, device=dev)
     if P:
-        check(lib.t12_pack_escapes_plane(w.data_ptr(), gr.data_ptr(), M, K, base_exp, row_off.data_ptr(), cols.data_ptr(),
-                                         correct.data_ptr(), wrong.data_ptr(), st), "t12_pack_escapes_plane")
+        with _on(stream):
+            check(lib.t12_pack_escapes_plane(w.data_ptr(), gr.data_ptr(), M, K, base_exp, row_off.data_ptr(), cols.data_ptr(),
+                                             correct.data_ptr(), wrong.data_ptr(), st), "t12_pack_escapes_plane")
     return DeviceTensor12(M, K, base_exp, sm, gr, row_off, cols, correct, wrong)
 
 
