@@ -27,6 +27,17 @@ def test_segments_are_what_the_structures_hold(t12, patched, P, shape):
     assert t12._segments([o], outs[:1], patched)[0].base_exp == 7
 
 
+@pytest.mark.parametrize("name", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_current_stream_without_torchs_private_calls(t12, monkeypatch, name):
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: _Stream(17))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 5, raising=False)
+    assert t12.current_stream() == 5
+    monkeypatch.delattr(torch._C, name)
+    assert t12.current_stream() == 17
+
+
 class _Stream:
     """A stream whose work is done when another one waits for it."""
 

@@ -281,7 +281,10 @@ def current_stream() -> int:
     torch = _torch()
     if not torch.cuda.is_initialized():
         return torch.cuda.current_stream().cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:                         # (not part of torch's documented face)
+        return torch.cuda.current_stream().cuda_stream
 
 
 _IN_ORDER = contextlib.nullcontext()
