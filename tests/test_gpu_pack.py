@@ -80,6 +80,20 @@ def test_row_offsets(t12, M):
     assert off[0] == 0 and off[M + 1] == -7 and torch.equal(off[1:M + 1].long(), torch.cumsum(c.long(), 0))
 
 
+@pytest.mark.parametrize("M", [2 ** 31 - 8193, 2 ** 31 - 1])
+def test_row_offsets_up_to_the_largest_row_count(t12, M):
+    c = torch.zeros(M, dtype=torch.int32, device="cuda")
+    at = [0, 5, 2 ** 30, M - 8192, M - 1]
+    for i, r in enumerate(at):
+        c[r] = 10 ** i
+    off = torch.full((M + 2,), -7, dtype=torch.int32, device="cuda")
+    t12.check(t12.lib.t12_pack_row_offsets(c.data_ptr(), M, off.data_ptr(), t12.current_stream()))
+    assert off[0] == 0 and off[M + 1] == -7
+    ends = at[1:] + [M]
+    for i, (r, end) in enumerate(zip(at, ends)):                       # constant between the rows that count
+        assert off[r + 1] == off[end] == int("1" * (i + 1)), (i, r)
+
+
 def test_base_exponent_on_the_device(t12, oracle):
     """The window rule where windows tie (the first wins), where nothing is in a window's reach, and at both ends of the exponents."""
     for exps in ([0], [255], [1, 200], [15, 100], [254, 255], [16, 31, 46], list(range(256))):

@@ -145,23 +145,24 @@ __global__ __launch_bounds__(256) void base_exp_kernel(const unsigned long long*
         }
         if (t == 0) *base = at[0] - 1;
     }
-    for (int r = blockIdx.x * 256 + threadIdx.x; r < M; r += gridDim.x * 256) row_cnt[r] = 0;
+    for (uint32_t r = blockIdx.x * 256 + threadIdx.x; r < (uint32_t)M; r += gridDim.x * 256) row_cnt[r] = 0;
 }
 
 // row_off[0] = 0, row_off[r+1] = sum of cnt[0..r]; one workgroup of 1024 lanes, eight neighbouring counts per lane and step, the next
 // step's requested ahead (14336 rows: 15.2 us with a stretch of the rows per lane, 8.7).
-__global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ cnt, int M,
+// (Row numbers unsigned: a step past the last of up to 2^31 - 1 rows.)
+__global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ cnt, uint32_t M,
                                                     int32_t* __restrict__ row_off)
 {
     __shared__ int part[2][16];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    constexpr int OWN = 8, STEP = 1024 * OWN;
+    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    constexpr uint32_t OWN = 8, STEP = 1024 * OWN;
     const bool vec = (uintptr_t)cnt % 16 == 0;
-    auto fetch = [&](int r0, int (&c)[OWN]) __attribute__((always_inline)) {
-        const int r = r0 + OWN * t;
+    auto fetch = [&](uint32_t r0, int (&c)[OWN]) __attribute__((always_inline)) {
+        const uint32_t r = r0 + OWN * t;
         if (vec && r + OWN <= M) {
 #pragma unroll
-            for (int i = 0; i < OWN; i += 4) {
+            for (uint32_t i = 0; i < OWN; i += 4) {
                 const int4 v = *(const int4*)(cnt + r + i);
                 c[i] = v.x;
                 c[i + 1] = v.y;
@@ -170,20 +171,20 @@ __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ 
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < OWN; i++) c[i] = r + i < M ? cnt[r + i] : 0;
+            for (uint32_t i = 0; i < OWN; i++) c[i] = r + i < M ? cnt[r + i] : 0;
         }
     };
     int c[OWN], next[OWN] = {}, carry = 0;
     fetch(0, c);
     if (t == 0) row_off[0] = 0;
-    for (int r0 = 0, k = 0; r0 < M; r0 += STEP, k ^= 1) {
+    for (uint32_t r0 = 0, k = 0; r0 < M; r0 += STEP, k ^= 1) {
         if (r0 + STEP < M) fetch(r0 + STEP, next);
         int own = 0;
 #pragma unroll
-        for (int i = 0; i < OWN; i++) own += c[i];
+        for (uint32_t i = 0; i < OWN; i++) own += c[i];
         int sum = own;                                      // inclusive over the wave
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
+        for (uint32_t o = 1; o < 64; o <<= 1) {
             const int v = __shfl_up(sum, o, T12_WAVE);
             if (lane >= o) sum += v;
         }
@@ -191,13 +192,13 @@ __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ 
         __syncthreads();                                    // (two tables: one barrier per step)
         int run = carry + sum - own;
 #pragma unroll
-        for (int w = 0; w < 16; w++) {
+        for (uint32_t w = 0; w < 16; w++) {
             const int v = part[k][w];
             run += w < wave ? v : 0;
             carry += v;
         }
 #pragma unroll
-        for (int i = 0; i < OWN; i++) {
+        for (uint32_t i = 0; i < OWN; i++) {
             run += c[i];
             if (r0 + OWN * t + i < M) row_off[r0 + OWN * t + i + 1] = run;
             c[i] = next[i];
@@ -412,7 +413,7 @@ int t12_pack_begin(const void* w_bf16, int M, int K, void* hist_u64x256, void* b
     hipStream_t st = (hipStream_t)stream;
     int rc = t12_pack_histogram(w_bf16, (size_t)M * K, hist_u64x256, stream);
     if (rc) return rc;
-    const int blocks = (M + 4095) / 4096 < 64 ? (M + 4095) / 4096 : 64;
+    const int blocks = M < 64 * 4096 ? (M + 4095) / 4096 : 64;
     hipLaunchKernelGGL(base_exp_kernel, dim3(blocks), dim3(256), 0, st, (const unsigned long long*)hist_u64x256, (int32_t*)base_exp,
                        (int32_t*)row_cnt, M);
     T12_CHECK_LAUNCH("t12_pack_begin(base)");
