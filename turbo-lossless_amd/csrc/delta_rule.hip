@@ -131,21 +131,21 @@ __global__ __launch_bounds__(256) void delta_token_kernel(const DeltaParams p)
 }
 
 // A run of tokens of one sequence.  Workgroup = two waves = eight columns of one head, so that the heads of a model spread
-// over the chip.  The records of CH tokens are brought into LDS together, the next CH (or the last few tokens) are on their way
-// meanwhile; the outputs of sixteen tokens are added up across the lanes at once.  Dynamic LDS: run_lds_bytes().
-template <int RL, int CH>
+// over the chip.  The records of sixteen tokens are brought into LDS together, the next sixteen (or the last few tokens) are on their way
+// meanwhile; the outputs of the sixteen are added up across the lanes at once.  Dynamic LDS: run_lds_bytes().
+constexpr int RUN_TOK = 16;
+template <int RL>
 constexpr size_t run_lds_bytes()
 {
-    return (size_t)2 * ((CH * rec_floats(RL * 16) / 4 + 127) / 128) * 128 * 16;
+    return (size_t)2 * ((RUN_TOK * rec_floats(RL * 16) / 4 + 127) / 128) * 128 * 16;
 }
 // Tokens past the last whole chunk that are worth bringing through LDS: straight from memory each costs 0.68 us, in a chunk 0.12 and
 // all together 1.5 us more (16 heads of 64, whole call: 1 / 4 / 15 tokens 10.5 / 13.4 / 18.4 us straight, 11.5 / 13.4 / 14.5 staged).
 constexpr int RUN_STAGED_TAIL = 5;
-template <int RL, int CH>
+template <int RL>
 __global__ __launch_bounds__(128) void delta_run_kernel(const DeltaParams p)
 {
-    constexpr int DP = RL * 16, RF = rec_floats(DP), PIECES = CH * RF / 4, NP = (PIECES + 127) / 128;
-    static_assert(CH % 16 == 0, "outputs are added up sixteen tokens at a time");
+    constexpr int CH = RUN_TOK, DP = RL * 16, RF = rec_floats(DP), PIECES = CH * RF / 4, NP = (PIECES + 127) / 128;
     extern __shared__ float4 lds4[];
     float* lds = (float*)lds4;
     const T12DeltaRule& d = p.d;
@@ -184,19 +184,15 @@ __global__ __launch_bounds__(128) void delta_run_kernel(const DeltaParams p)
         const float* x = lds + (size_t)(c & 1) * (NP * 128 * 4);
         Token<RL> t[2];
         t[0].read(x, C.l, C.jc);
+        float y[CH];
 #pragma unroll
-        for (int s = 0; s < CH; s += 16) {
-            float y[16];
-#pragma unroll
-            for (int f = 0; f < 16; f++) {
-                const int at = s + f;
-                if (at + 1 < CH) t[(at + 1) & 1].read(x + (at + 1) * RF, C.l, C.jc);
-                y[f] = t[at & 1].advance(C);
-                __builtin_amdgcn_sched_barrier(0);         // (a token's reads stay one token ahead)
-            }
-            const float v = transpose_sum16(y, C.l);
-            if (C.live) o[(size_t)(c * CH + s + C.l) * o_step] = v;
+        for (int f = 0; f < CH; f++) {
+            if (f + 1 < CH) t[(f + 1) & 1].read(x + (f + 1) * RF, C.l, C.jc);
+            y[f] = t[f & 1].advance(C);
+            __builtin_amdgcn_sched_barrier(0);             // (a token's reads stay one token ahead)
         }
+        const float v = transpose_sum16(y, C.l);
+        if (C.live) o[(size_t)(c * CH + C.l) * o_step] = v;
     }
 #undef T12_REQUEST
     if (tail < RUN_STAGED_TAIL) {                          // a few last tokens straight from memory
@@ -212,21 +208,19 @@ __global__ __launch_bounds__(128) void delta_run_kernel(const DeltaParams p)
         for (int i = 0; i < NP; i++) buf[tid + i * 128] = ahead[i];
         __syncthreads();
         const float* x = lds + (size_t)(chunks & 1) * (NP * 128 * 4) + (chunks ? CH - tail : 0) * RF;
-        for (int s = 0; s < tail; s += 16) {
-            Token<RL> t[2];
-            t[0].read(x + s * RF, C.l, C.jc);
-            float y[16];
+        Token<RL> t[2];
+        t[0].read(x, C.l, C.jc);
+        float y[CH];
 #pragma unroll
-            for (int f = 0; f < 16; f++) {
-                y[f] = 0.0f;
-                if (s + f < tail) {
-                    t[(f + 1) & 1].read(x + min(s + f + 1, tail - 1) * RF, C.l, C.jc);
-                    y[f] = t[f & 1].advance(C);
-                }
+        for (int f = 0; f < CH; f++) {
+            y[f] = 0.0f;
+            if (f < tail) {
+                t[(f + 1) & 1].read(x + min(f + 1, tail - 1) * RF, C.l, C.jc);
+                y[f] = t[f & 1].advance(C);
             }
-            const float v = transpose_sum16(y, C.l);
-            if (C.live && s + C.l < tail) o[(size_t)(chunks * CH + s + C.l) * o_step] = v;
         }
+        const float v = transpose_sum16(y, C.l);
+        if (C.live && C.l < tail) o[(size_t)(chunks * CH + C.l) * o_step] = v;
     }
     C.store();
 }
@@ -667,27 +661,28 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const DeltaParams p)
     }
 }
 
-template <int RL, int CH>
+// STAGED: records through LDS, which has room for those of heads of up to 128 channels.
+template <int RL, bool STAGED>
 int launch_rule(const DeltaParams& p, hipStream_t st)
 {
     hipLaunchKernelGGL((delta_prep_kernel<RL * 16>), dim3((p.n + PREP_TOK - 1) / PREP_TOK, p.d.heads), dim3(256),
                        (size_t)PREP_TOK * p.d.rank * sizeof(float), st, p);
     if (!p.run) {
         hipLaunchKernelGGL(delta_token_kernel<RL>, dim3(p.n, p.d.heads, (p.d.dim + 15) / 16), dim3(256), 0, st, p);
-    } else if constexpr (CH > 0) {
-        constexpr size_t lds = run_lds_bytes<RL, CH>();
+    } else if constexpr (STAGED) {
+        constexpr size_t lds = run_lds_bytes<RL>();
         if (lds > 64 * 1024) {
             static std::once_flag once[16];                // the attribute is per device
             int dev = 0;
             if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) dev = 0;
             hipError_t e = hipSuccess;
-            std::call_once(once[dev], [&] { e = hipFuncSetAttribute((const void*)delta_run_kernel<RL, CH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+            std::call_once(once[dev], [&] { e = hipFuncSetAttribute((const void*)delta_run_kernel<RL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
             if (e != hipSuccess) {
                 t12_set_error("t12_delta_rule: cannot reserve %zu bytes of LDS", lds);
                 return T12_ELAUNCH;
             }
         }
-        hipLaunchKernelGGL((delta_run_kernel<RL, CH>), dim3(p.d.heads, (p.d.dim + 7) / 8), dim3(128), lds, st, p);
+        hipLaunchKernelGGL(delta_run_kernel<RL>, dim3(p.d.heads, (p.d.dim + 7) / 8), dim3(128), lds, st, p);
     } else {
         hipLaunchKernelGGL(delta_run_direct_kernel<RL>, dim3(p.d.heads, (p.d.dim + 3) / 4), dim3(64), 0, st, p);
     }
@@ -745,10 +740,10 @@ int t12_delta_rule(const T12DeltaRule* d, const float* in, const float* bias, in
         rc = T12_OK;
     } else
     switch (d->dim_p) {
-        case 64: rc = launch_rule<4, 16>(p, st); break;    // (short runs, and decay rates the chunks are not for)
-        case 128: rc = launch_rule<8, 16>(p, st); break;
-        case 256: rc = launch_rule<16, 0>(p, st); break;
-        default: rc = launch_rule<32, 0>(p, st); break;
+        case 64: rc = launch_rule<4, true>(p, st); break;  // (short runs, and decay rates the chunks are not for)
+        case 128: rc = launch_rule<8, true>(p, st); break;
+        case 256: rc = launch_rule<16, false>(p, st); break;
+        default: rc = launch_rule<32, false>(p, st); break;
     }
     if (rc) return rc;
     const int items = n * d->heads;

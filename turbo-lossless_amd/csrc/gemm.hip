@@ -344,7 +344,7 @@ __device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt
                 }
                 cur[y][i] = behind[y][i];
                 nc[y][i] = ++pp[y][i] < pe[y][i] ? (int)(cur[y][i] & 0xFFFFu) : NO_ESCAPE;
-                behind[y][i] = lpat[pp[y][i] + 1];                  // (at most one past the list: the offsets behind it)
+                behind[y][i] = lpat[pp[y][i] + 1];                  // (at most two past the list: the offsets behind it)
             }
         }
     };
