@@ -1592,10 +1592,9 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
     }
     if (B > 16 && B <= 32 && K % 128 == 0) {
         // 17 .. 32 batch rows on tensors of few rows, which the plan above left to the sweep (or whose planes the ring kernel cannot
-        // copy): the sweep of up to 16 rows with two batch tiles per weight load and decode.  One round of workgroups takes
-        // ~4.5 us + (K / 4096) (3.7 + 0.2 B) us whatever the row count, because every workgroup reads all B activation rows
-        // for its 16 (32) weight rows.  Measured at B = 17 / 24 / 32: 4096 x 4096 10.4 / 11.0 / 11.3 us (12.0 / 13.1 / 14.4 before the turn
-        // through LDS, which the rule was fitted to).
+        // copy): the sweep of up to 16 rows with two batch tiles per weight load and decode.  One round of workgroups takes the same
+        // whatever the row count, because every workgroup reads all B activation rows for its 16 (32) weight rows: at B = 17 / 24 / 32 and
+        // 4096 columns 10.4 / 11.0 / 11.3 us (12.0 / 13.1 / 14.4 before the turn through LDS, which the rule was fitted to).
         int groups16 = 0, sets2 = 0;
         for (int i = 0; i < nseg; i++) {
             groups16 += (segs[i].M + 15) / 16;
