@@ -436,7 +436,7 @@ def run_moe(args, t12, torch, dev):
         "TFLOPs": flops / ms / 1e9, "weight_GBps": wbytes / ms / 1e6,
         "small_batches": small,
         "roofline": {"bound": "hbm", "achieved": wbytes / ms / 1e6, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": wbytes / ms / 1e6 / HBM_PEAK_GBS, "traffic": None, "kernel": "gemm_mfma_kernel"},
+                     "frac": wbytes / ms / 1e6 / HBM_PEAK_GBS, "traffic": None, "kernel": "gemm_strip_kernel, gemm_tile_kernel"},
         "setup_s": t_build,
     }
 
@@ -926,7 +926,7 @@ def gemm_b256_roofline(layers):
                  "vendor_bf16_gate_up_frac": layers["vendor_bf16_gate_up_b256"]["mfma_frac"]}
     return {**extra, "bound": "mfma", "achieved": fl / us / 1e6, "peak": 2500.0, "unit": "TFLOP/s", "frac": fl / us / 1e6 / 2500.0,
             "traffic": None, "gate_up_traffic": measured_traffic("gemm_gate_up_b256"),
-            "kernel": "gemm_mfma_kernel, QKV + O + gate|up + down at B=256", "flops_per_step": fl,
+            "kernel": "gemm_tile_kernel, QKV + O + gate|up + down at B=256", "flops_per_step": fl,
             "us_per_step": us, "gate_up_frac": layers["gate_up_b256"]["mfma_frac"],
             # the same four products as the engine's layer issues them: gate|up with SiLU*mul in its epilogue
             "gate_up_swiglu_frac": layers["gate_up_swiglu_b256"]["mfma_frac"],
@@ -1062,7 +1062,7 @@ def run_gemm_layers(args, t12, torch, dev):
         "reference_named_launchers_gate_14336x4096": named,
         "roofline": {"bound": "mfma", "achieved": gu["TFLOPs"], "peak": 2500.0, "unit": "TFLOP/s",
                      "frac": gu["TFLOPs"] / 2500.0, "traffic": measured_traffic("gemm_gate_up_b256"),
-                     "kernel": "gemm_mfma_kernel<4,2,2,2> on gate|up at B=256", "flops_per_launch": gu["flops"],
+                     "kernel": "gemm_tile_kernel on gate|up at B=256", "flops_per_launch": gu["flops"],
                      "us_per_launch": gu["us"],
                      "vendor_bf16_gemm_frac": layers.get("vendor_bf16_gate_up_b256", {}).get("mfma_frac"),
                      "clock_ghz_mfma_decode_lds_256wg": probe["mfma_decode_lds_256wg"]["ghz"],

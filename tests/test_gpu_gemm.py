@@ -63,6 +63,28 @@ def test_gemm_few_stages(t12, oracle, synth, K, B):
     assert rel_err(got, oracle.gemm(p, X)) < TOL
 
 
+@pytest.mark.parametrize("rows,K,B,p_out", [((16400,), 64, 257, 2e-3), ((16400,), 128, 300, 1e-3), ((16400,), 192, 512, 0.0), ((8000, 500, 8001), 320, 384, 2e-3),
+                                            ((16640,), 448, 511, 0.1), ((16387,), 4096, 260, 3e-3), ((33000,), 256, 256, 1e-2), ((33000,), 320, 513, 1e-2)])
+def test_gemm_more_than_256_rows_on_many_weight_rows(t12, rows, K, B, p_out):
+    """Tiles of 256 x 256 (all but the one of 256 rows of activations, which keeps 128 x 256): one to seven stages, one row past a batch tile and one
+    short of it, ragged last tiles, tensors that end inside a tile, lists that fit the 4096 places of a tile and ones that do not; escapes in
+    neighbouring columns.  Against the same products in 64 bits; fp32 sums of K exact products of one size differ by K^0.5 2^-24 of them at most."""
+    g = torch.Generator(device=dev()).manual_seed(K + B)
+    W = []
+    for m in rows:
+        w = torch.randn((m, K), generator=g, device=dev()) * 0.02
+        if p_out:
+            w = torch.where(torch.rand((m, K), generator=g, device=dev()) < p_out, 8.0 * torch.randn((m, K), generator=g, device=dev()), w)
+            w[::37, K - 5:] = 16.0
+            w[1::41, :3] = -4.0
+        W.append(w.to(torch.bfloat16))
+    X = torch.randn((B, K), generator=g, device=dev()).to(torch.bfloat16)
+    outs = t12.gemm([t12.pack_device(w) for w in W], X.view(torch.int16))
+    for o, w in zip(outs, W):
+        want = X.double() @ w.double().T
+        assert float((o.double() - want).norm() / want.norm()) < 8 * K ** 0.5 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("B", [3, 4, 5, 8, 9, 16, 17, 20, 31, 32])
 @pytest.mark.parametrize("M, K", [(1, 128), (15, 256), (17, 1152), (33, 896), (513, 2176)])
 def test_gemm_sweep_with_loads_turned_through_lds(t12, oracle, synth, B, M, K):

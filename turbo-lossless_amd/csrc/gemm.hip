@@ -7,34 +7,18 @@
 // plus nv_apply_patches_batch (nvidia_kernels.cu:295-319), re-designed for
 // wave64 MFMA instead of warp-level mma.sync:
 //
-//   * v_mfma_f32_32x32x16_bf16, activations as the A operand (rows = batch),
-//     weights as the B operand (columns = output features), so that an
-//     accumulator register holds 32 consecutive m of one batch row and the
-//     stores to out[b, m] coalesce without a transpose through LDS.
-//   * The whole batch tile (up to 256 rows) lives in one workgroup: every
-//     weight byte is fetched once per launch (the reference re-decodes per
+//   * More than 64 rows: tiles of 128 or 256 weight rows x up to 256 batch rows (gemm_tile.h).  3 .. 64 rows, where the weight stream is the
+//     bound, have a kernel of their own (gemm_ring.h) and, on short or few rows, the whole-row sweep.
+//   * Up to 256 batch rows live in one workgroup: every weight byte is fetched once per launch (the reference re-decodes per
 //     batch tile, nvidia_kernels.cu:456).
-//   * The compressed planes are loaded into registers, rebuilt to bf16 there, two
-//     weights per VGPR (t12_decode8), and written once per workgroup into a bf16 tile
-//     in LDS from which the waves read their MFMA B fragments: every weight is
-//     decoded once per workgroup, no bf16 copy of W ever exists in HBM.  The
-//     activations are staged already paired the way t12_decode8 orders its
-//     outputs, so no operand shuffling is needed.
-//   * Eight waves per workgroup (two per SIMD), laid out WB x WM; a wave owns FB x FM 32x32
-//     accumulator tiles: batch tiles of 64 (2 x 4 waves, 1 x 1), 128 (2 x 4, 2 x 1) and
-//     256 rows (4 x 2, 2 x 2).
 //   * Few row tiles (small M) are split along K across workgroups; the partial
 //     sums go to a workspace and a second kernel adds them in a fixed order
 //     (deterministic) -- or the caller's next kernel does (t12_gemm_deferred).
-//   * Escapes are EXACT and cost no extra pass: the (column, exact bf16) pairs of
-//     the workgroup's 128 rows -- one contiguous slice of the CSR list -- are
-//     staged in LDS once; the thread that decoded 16 columns of a row walks that
-//     row's slice in step with the K loop and overwrites the decoded half-words
-//     in the LDS tile.
+//   * Escapes are EXACT and cost no extra pass: the (column, exact bf16) pairs of a workgroup's rows -- one contiguous slice of
+//     the CSR list -- are staged in LDS once, and the exact values take the places of the decoded ones.
 //
 // Fast path requirements: K % 64 == 0, 0 <= base_exp <= 240, 16-byte aligned
-// activation rows.  Everything else goes to the general kernel below.  3 .. 64 rows, where the weight stream is the
-// bound, have a kernel of their own (gemm_ring.h) and, on short or few rows, the whole-row sweep.
+// activation rows.  Everything else goes to the general kernel below.
 
 #include <map>
 #include <mutex>
@@ -48,6 +32,7 @@
 #include "dense16_plan.h"
 #include "gemm_params.h"
 #include "gemm_ring.h"
+#include "gemm_tile.h"
 #include "ring_plan.h"
 
 // library-internal (hidden: not part of the ABI)
@@ -55,507 +40,6 @@ extern "C" __attribute__((visibility("hidden"))) void t12_glue_release_stream(hi
 extern "C" __attribute__((visibility("hidden"))) void t12_sampler_release_stream(hipStream_t st);   // engine/sampler.cpp
 
 namespace {
-
-constexpr int KC = 64;          // K columns staged per pipeline stage
-constexpr int TM = 128;         // weight rows per workgroup
-constexpr int PCAP = 2048;      // escape entries a workgroup can stage in LDS
-constexpr int PATCH_BYTES = PCAP * 4 + (TM + 1) * 4 + 12;
-constexpr int NO_ESCAPE = 0x7FFFFFFF;
-
-// How far apart two arrays lie, one value in the wave.  A lane that picks one of the two tensors of a pair adds it or not: between the
-// pointers themselves the compiler would choose a pointer to load, a chain of loads per lane.
-__device__ __forceinline__ int64_t apart(const void* a, const void* b)
-{
-    const uint64_t d = (uint64_t)(uintptr_t)b - (uint64_t)(uintptr_t)a;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)d), hi = __builtin_amdgcn_readfirstlane((uint32_t)(d >> 32));
-    return (int64_t)((uint64_t)hi << 32 | lo);
-}
-// A word that is one value in the wave and that no kernel in flight writes.
-__device__ __forceinline__ int scalar_load(const int* p) { return *(const __attribute__((address_space(4))) int*)(uintptr_t)p; }
-
-// LDS slot of (unit, row) in a [units][rows] array of 16-byte units.  Rows are rotated
-// inside their aligned block of eight by the unit index, so that both access patterns are
-// bank-conflict free: the staging writes (neighbouring lanes = the units of one row) and
-// the fragment reads (neighbouring lanes = consecutive rows of one unit).
-__device__ __forceinline__ int lds_slot(int u, int r, int rows) { return u * rows + (r & ~7) + ((r + u) & 7); }
-
-// Order in which a thread's staging units are stored: the ndec decode units (18 VALU each) and as many of the nact activation units (4
-// VALU each) in turn, then the other activation units; the escapes among the decoded go over them in between, under the stage's last
-// products.  Behind the last one, in front of the barrier, they and their two reads of the list cost 28672 x 4096 at 512 rows 149.0 us (2e-4 of the weights)
-// and 149.4 (1e-3); now 143.2 both; without any escapes 138.  8256 x 2048 at 512 36.7 / 39.2 -> 34.7 / 35.3, 28672 x 4096 at 100 49.2 / 52.8 -> 47.7 / 49.6.
-// Position pos -> unit index (activation units 0 .. nact-1, decode units nact .. nact+ndec-1).
-__device__ __forceinline__ constexpr int stage_unit_order(int pos, int nact, int ndec)
-{
-    const int mixed = nact < ndec ? nact : ndec;
-    if (pos < 2 * mixed) return pos & 1 ? pos / 2 : nact + pos / 2;
-    return nact < ndec ? nact + pos - mixed : pos - ndec;
-}
-// position of the last decode unit
-__device__ __forceinline__ constexpr int last_decode_unit(int nact, int ndec) { return nact < ndec ? nact + ndec - 1 : 2 * ndec - 2; }
-
-// ---------------------------------------------------------------------------
-// LDS stage layout (one of two buffers), unit u = (k % 64) / 8 = eight bf16 of one row,
-// paired (i, i + 4) per dword the way t12_decode8 / t12_pair_acts order them:
-//   act  [8 units][TB rows] x 16 B
-//   w    [8 units][TM rows] x 16 B     decoded weights
-// MFMA k-step t of a stage covers columns 16t .. 16t+15; the lanes of wave half h take
-// unit 2t + h of their row, for both operands.
-//
-// Global loads.  A stage is 64 columns: 128 B of an activation row (one cache line) but
-// only 64 B of a row's sm plane and 32 B of its gr plane.  Fetching those a stage at a
-// time asks HBM for every line twice or more (the rows of a tile are K bytes apart, a
-// power of two: they fall into a handful of L2 sets and are evicted before the next
-// stage comes back for the other half).  So weights are loaded per WINDOW of two stages
-// (128 columns), both halves of a line in back-to-back instructions:
-//   piece X (used by the even stage): lanes c8 < 4 take row rr, columns 16*c8 ..;
-//                                     lanes c8 >= 4 take row 64 + (rr^1), columns 16*(c8-4) ..
-//   piece Y (used by the odd stage) : the other halves of the same two lines, lanes swapped
-// where c8 = tid % 8, rr = item / 8 in 0..63.  Every lane decodes one piece per item and
-// stage (balanced), every sm line is requested whole within two instructions, and the
-// rr^1 keeps the LDS writes of the two lane groups on different banks.
-// ---------------------------------------------------------------------------
-// SWI (two segments of equal M, gate and up; FM == 2): a tile holds 64 rows of each, interleaved in
-// blocks of 32 -- local rows [0,32) gate rows 0..31, [32,64) up rows 0..31, [64,96) gate 32..63, [96,128) up
-// 32..63 -- so that the two accumulator tiles of a wave are gate and up of the SAME 32 rows and the epilogue
-// writes bf16( silu(gate) * up ) straight from registers: the reference's silu_mul_bf16 kernel
-// (engine/kernels.hip:447-459) and the fp32 round trip of both projections folded away.
-// EPI (T12_ACT_*, one segment, no K split): the unary function of every sum is stored as bf16 to out_bf16.
-// bt: batch tile.  Returns false when the tile lies past the segment's rows (nothing was done).
-template <int WB, int WM, int FB, int FM, bool SWI, int EPI, bool DEV>
-__device__ __forceinline__ bool gemm_mfma_body(const GemmParams& p, const int bt)
-{
-    static_assert(!SWI || FM == 2, "the SwiGLU epilogue pairs the two row tiles of a wave");
-    constexpr int TB = WB * FB * 32;                  // batch rows per workgroup
-    constexpr int NT = WB * WM * 64;                  // threads per workgroup
-    static_assert(NT == 512, "eight waves per workgroup");
-    static_assert(WM * FM * 32 == TM, "row tile is 128");
-    constexpr int ACT_UNITS = TB * 8;                 // 16-byte units per stage
-    constexpr int ACT_LD = ACT_UNITS / NT;            // per thread
-    constexpr int W_LD = TM * 4 / NT;                 // 16-column weight pieces per thread and stage
-    static_assert(ACT_LD >= 1 && ACT_LD * NT == ACT_UNITS, "activation tile divides over the threads");
-    constexpr int STAGE_BYTES = ACT_UNITS * 16 + TM * 128;
-
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wb = wave / WM, wm = wave % WM;
-    const int ln = lane & 31, lh = lane >> 5;
-
-    const int tile = blockIdx.x;
-    const int pair = SWI ? find_pair(p, tile) : 0;
-    const int s = SWI ? 2 * pair : find_segment(p, tile);          // SWI: the gate segment of the tile's pair
-    const T12Segment& sg = p.seg[s];
-    const T12Segment& sg1 = p.seg[SWI ? s + 1 : s];
-    const int M = sg.M, K = p.K;
-    const int B = DEV ? p.dev_counts[p.group_of_seg[s]] : p.seg_B[s];
-    const int row_base = DEV ? p.dev_base[p.group_of_seg[s]] : 0;            // first row of this group in act / out
-    const int act_stride = p.seg_act_stride[s];
-    const uint16_t* const act = p.seg_act[s] + (size_t)row_base * act_stride;
-    if (bt * (WB * FB * 32) >= B) return false;            // grouped launch: this segment has fewer batch tiles than the grid
-    const int m0 = SWI ? (tile - p.blk_start[pair]) * (TM / 2) : (tile - p.blk_start[s]) * TM;
-    // local row r of the tile -> matrix row
-    auto row_mat = [&](int r) { return SWI ? m0 + ((r >> 6) << 5) + (r & 31) : m0 + r; };
-    const int b0 = bt * TB;
-    const int k_begin = blockIdx.z * p.kslice;
-    const int k_end = min(K, k_begin + p.kslice);
-    const int nstage = (k_end - k_begin) / KC;
-    const int be0 = __builtin_amdgcn_readfirstlane(sg.base_exp), be1 = __builtin_amdgcn_readfirstlane(sg1.base_exp);
-    const int64_t sm_apart = SWI ? apart(sg.sm, sg1.sm) : 0, gr_apart = SWI ? apart(sg.gr, sg1.gr) : 0;
-
-    // ---- this thread's share of the global -> LDS staging
-    //  acts: item idx = tid + NT*i -> batch row idx / 8, unit idx % 8 (8 lanes = 128 contiguous bytes)
-    // rows past the end are clamped: their products are computed and never stored
-    const uint16_t* a_src[ACT_LD];
-    int a_dst[ACT_LD];
-#pragma unroll
-    for (int i = 0; i < ACT_LD; i++) {
-        const int idx = tid + NT * i;
-        const int r = idx >> 3, u = idx & 7;
-        a_src[i] = act + (size_t)min(b0 + r, B - 1) * act_stride + k_begin + u * 8;
-        a_dst[i] = lds_slot(u, r, TB) * 16;
-    }
-    //  weights: pieces X / Y of item i (see above); [0] = X, [1] = Y
-    const int c8 = tid & 7, hi = c8 >> 2, cc = c8 & 3;
-    const uint8_t* s_src[2][W_LD];
-    const uint8_t* g_src[2][W_LD];
-    int w_row[2][W_LD];
-    int w_dst[2][W_LD][2];
-    uint32_t w_be2[2][W_LD];
-#pragma unroll
-    for (int i = 0; i < W_LD; i++) {
-        const int rr = (tid + NT * i) >> 3;                   // 0..63
-        const int r_lo = rr, r_hi = 64 + (rr ^ 1);
-#pragma unroll
-        for (int y = 0; y < 2; y++) {
-            const int r = (hi ^ y) ? r_hi : r_lo;
-            const bool second = SWI && ((r >> 5) & 1);
-            const size_t e = (size_t)min(row_mat(r), M - 1) * K + k_begin + 64 * y + 16 * cc;
-            w_row[y][i] = r;
-            const uint32_t be = second ? be1 : be0;
-            w_be2[y][i] = t12_opaque((be << 7) | (be << 23));
-            s_src[y][i] = sg.sm + ((second ? sm_apart : 0) + (int64_t)e);
-            g_src[y][i] = sg.gr + ((second ? gr_apart : 0) + (int64_t)(e >> 1));
-            w_dst[y][i][0] = ACT_UNITS * 16 + lds_slot(2 * cc, r, TM) * 16;
-            w_dst[y][i][1] = ACT_UNITS * 16 + lds_slot(2 * cc + 1, r, TM) * 16;
-        }
-    }
-
-    // Register rings.  Activations: 4 slots, stage s + 4 is requested while stage s is
-    // multiplied.  Weights: 2 window slots, window w + 2 is requested during the odd stage of
-    // window w, when both of the slot's pieces have been decoded.  A stage is decoded and moved
-    // registers -> LDS one iteration before it is consumed (double-buffered LDS).
-    constexpr int DA = 4;
-    uint4 ra[DA][ACT_LD];
-    uint4 rs[2][2][W_LD];      // [window slot][X / Y][item]
-    uint2 rg[2][2][W_LD];
-    // The staging work of a thread is cut into units so that it can be spread between the
-    // MFMAs of a stage.  Load units: ACT_LD activation pieces, then (odd stages) 4 per item:
-    // sm X, sm Y, gr X, gr Y.  Store units: ACT_LD activation pieces, 2 decode units per item.
-    auto load_act = [&](int slot, int stg, int u) { ra[slot][u] = *(const uint4*)(a_src[u] + (size_t)stg * KC); };
-    auto load_w = [&](int slot, int win, int u, bool do_x, bool do_y) {
-        const int i = u >> 2, y = u & 1;
-        if (y == 0 ? !do_x : !do_y) return;
-        if ((u & 2) == 0) rs[slot][y][i] = *(const uint4*)(s_src[y][i] + (size_t)win * (2 * KC));
-        else rg[slot][y][i] = *(const uint2*)(g_src[y][i] + (size_t)win * KC);
-    };
-    auto store_unit = [&](int aslot, int wslot, int y, int buf, int u) {
-        uint8_t* base_ = lds + buf * STAGE_BYTES;
-        if (u < ACT_LD) {
-            *(uint4*)(base_ + a_dst[u]) = t12_pair_acts(ra[aslot][u]);
-        } else {
-            const int i = (u - ACT_LD) >> 1, h = (u - ACT_LD) & 1;
-            const uint4 sv = rs[wslot][y][i];
-            const uint2 gv = rg[wslot][y][i];
-            uint32_t w_[4];
-            if (h == 0) t12_decode8(sv.x, sv.y, gv.x, w_be2[y][i], w_);
-            else t12_decode8(sv.z, sv.w, gv.y, w_be2[y][i], w_);
-            *(uint4*)(base_ + w_dst[y][i][h]) = make_uint4(w_[0], w_[1], w_[2], w_[3]);
-        }
-    };
-
-    t12_f32x16 acc[FB][FM];
-#pragma unroll
-    for (int i = 0; i < FB; i++)
-#pragma unroll
-        for (int j = 0; j < FM; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    // ---- escape list of this workgroup's rows -> LDS.  The rows are consecutive, so
-    //      their entries are one contiguous slice [e0, e1) of cols[] / correct[].
-    //      esc_mode: 0 none, 1 staged (exact values written over the decoded ones in LDS),
-    //      2 too many for LDS (or K > 65536): wrong values multiplied, corrected in the epilogue.
-    //      What a workgroup waits for before its first product is a chain of loads, 1 us each: the rows' offsets, the
-    //      list, the tiles.  So the ends of the slice come by scalar loads, every row's offset and the first stages'
-    //      tiles are requested along with them, the list behind the first two stages' tiles, and the rest of the tiles
-    //      behind the list (4096 x 4096 at B = 100 / 256, 8 / 4 slices: 18.5 / 23.3 -> 17.0 / 22.5 us).
-    uint32_t* lpat = (uint32_t*)(lds + 2 * STAGE_BYTES);       // col | correct << 16
-    int* lrow = (int*)(lpat + PCAP);                           // [TM + 1] offsets into lpat (SWI: [2][TM/2 + 1])
-    constexpr int ER = SWI ? TM / 2 : TM;                      // rows of a tensor
-    const bool has0 = sg.row_off, has1 = SWI && sg1.row_off;
-    int esc_mode = 0;
-    int e00 = 0, e10 = 0, n0 = 0, n1 = 0;                      // first entry and number of entries, per tensor
-    int my_off = 0;                                            // thread t: offset of row t (SWI: of up's row t - ER - 1)
-    if (has0 || has1) {
-        // (a tensor without a list: any readable address)
-        const int* r0 = has0 ? sg.row_off : (const int*)sg.sm;
-        const int* r1 = has1 ? sg1.row_off : (const int*)sg.sm;
-        const int lo = min(m0, M), hi = min(m0 + ER, M);
-        e00 = scalar_load(r0 + (has0 ? lo : 0));
-        n0 = scalar_load(r0 + (has0 ? hi : 0));
-        e10 = scalar_load(r1 + (has1 ? lo : 0));
-        n1 = scalar_load(r1 + (has1 ? hi : 0));
-        if (SWI && tid > ER) {
-            if (has1 && tid <= 2 * ER + 1) my_off = sg1.row_off[min(m0 + tid - ER - 1, M)];
-        } else if (has0 && tid <= ER) {
-            my_off = sg.row_off[min(m0 + tid, M)];
-        }
-    }
-    // window w (0 or 1) of the slice; what lies past its end is not used: the last window, or its first half, again
-    auto load_first = [&](int w) {
-        const int win = min(w, (nstage - 1) / 2), back = 2 * win + 1 < nstage ? 0 : KC;
-#pragma unroll
-        for (int i = 0; i < W_LD; i++)
-#pragma unroll
-            for (int y = 0; y < 2; y++) {
-                rs[w][y][i] = *(const uint4*)(s_src[y][i] + win * (2 * KC) - y * back);
-                rg[w][y][i] = *(const uint2*)(g_src[y][i] + ((win * (2 * KC) - y * back) >> 1));
-            }
-    };
-    // (in the order in which the loop requests them, so that its waits count the same loads on the way in and around)
-#pragma unroll
-    for (int d = 0; d < 2; d++)
-#pragma unroll
-        for (int u = 0; u < ACT_LD; u++) load_act(d, min(d, nstage - 1), u);
-    load_first(0);
-    if (has0 || has1) {
-        n0 = has0 ? n0 - e00 : 0;
-        n1 = has1 ? n1 - e10 : 0;
-        esc_mode = (n0 + n1 <= PCAP && K <= 65536) ? 1 : 2;
-    }
-    const int64_t cols_apart = SWI ? apart(sg.cols, sg1.cols) : 0, exact_apart = SWI ? apart(sg.correct, sg1.correct) : 0;
-    auto list_entry = [&](int t, uint32_t& col, uint32_t& exact) {
-        const bool second = SWI && t >= n0;
-        const int64_t e = second ? e10 + t - n0 : e00 + t;
-        col = *(const uint32_t*)((const uint8_t*)sg.cols + ((second ? cols_apart : 0) + 4 * e));
-        exact = *(const uint16_t*)((const uint8_t*)sg.correct + ((second ? exact_apart : 0) + 2 * e));
-    };
-    uint32_t col = (uint32_t)my_off, exact = col;              // (any value: a constant would draw the shift below, and a wait, into the branch)
-    if (esc_mode == 1 && tid < n0 + n1) list_entry(tid, col, exact);
-#pragma unroll
-    for (int d = 2; d < DA; d++)
-#pragma unroll
-        for (int u = 0; u < ACT_LD; u++) load_act(d, min(d, nstage - 1), u);
-    load_first(1);
-    if (esc_mode == 1) {
-        if (tid < n0 + n1) lpat[tid] = col | exact << 16;
-        for (int t = tid + NT; t < n0 + n1; t += NT) {
-            list_entry(t, col, exact);
-            lpat[t] = col | exact << 16;
-        }
-        if (tid <= ER) lrow[tid] = has0 ? my_off - e00 : 0;
-        else if (SWI && tid <= 2 * ER + 1) lrow[tid] = n0 + (has1 ? my_off - e10 : 0);
-    }
-    // Per piece kind and item: cursor into its row's slice, the column of the next entry, the entry itself and the one behind
-    // it.  The thread that decoded 16 columns of a row into LDS also overwrites the escapes among them
-    // there (same wave, LDS executes its writes in order: no barrier needed in between).  A
-    // thread owns its X row in even stages and its Y row in odd ones; entries of the stages in
-    // between are stepped over.  An entry is in registers a stage before its turn at the latest, unless the row has three close
-    // together: a wave that read the list when it came to an entry held the seven others up.
-    int pp[2][W_LD], pe[2][W_LD], nc[2][W_LD];
-    uint32_t cur[2][W_LD], behind[2][W_LD];
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-        for (int i = 0; i < W_LD; i++) {
-            pp[y][i] = pe[y][i] = 0;
-            nc[y][i] = NO_ESCAPE;
-            cur[y][i] = behind[y][i] = 0;
-        }
-    auto patch_stage = [&](int y, int buf, int kabs) {
-        if (esc_mode != 1) return;
-        uint8_t* base_ = lds + buf * STAGE_BYTES + ACT_UNITS * 16;
-#pragma unroll
-        for (int i = 0; i < W_LD; i++) {
-            while (nc[y][i] < kabs + KC) {
-                const int e = nc[y][i] - kabs - 16 * cc;            // 0..15: one of this piece's
-                if ((unsigned)e < 16u) {
-                    const int off = lds_slot(2 * cc + (e >> 3), w_row[y][i], TM) * 16 + (e & 3) * 4 + ((e >> 2) & 1) * 2;
-                    *(uint16_t*)(base_ + off) = (uint16_t)(cur[y][i] >> 16);
-                }
-                cur[y][i] = behind[y][i];
-                nc[y][i] = ++pp[y][i] < pe[y][i] ? (int)(cur[y][i] & 0xFFFFu) : NO_ESCAPE;
-                behind[y][i] = lpat[pp[y][i] + 1];                  // (at most two past the list: the offsets behind it)
-            }
-        }
-    };
-
-    // One stage = 64 columns = 4 MFMA k-steps; the fragments of k-step t + 1 are read from LDS
-    // at the start of k-step t.  The staging work for later stages is placed between the MFMAs,
-    // a unit after every few of them, and pinned there with scheduling barriers: whatever is
-    // not issued under a running MFMA is serial time for the wave.
-    //   d = stage number modulo 4 (selects ring slots and LDS buffers at compile time)
-    constexpr int NMMA = 4 * FB * FM;
-    constexpr int NSU = ACT_LD + 2 * W_LD;               // store units per stage
-    constexpr int NLU_ODD = ACT_LD + 4 * W_LD;           // load units of an odd stage
-    constexpr int NCH = NMMA >= 2 * NSU ? NSU : NMMA;    // chunks of staging work per stage
-    constexpr int PATCH_AT = last_decode_unit(ACT_LD, 2 * W_LD) * NCH / NSU;
-    auto run_stage = [&](int d, int stg, bool ld_act, bool ld_x, bool ld_y, bool do_store) {
-        const int buf = d & 1;
-        const bool odd = d & 1;
-        const int nlu = odd ? NLU_ODD : ACT_LD;
-        // stage stg + 1: activation slot, weight window slot, piece kind
-        const int n_aslot = (d + 1) & 3, n_wslot = ((d + 1) >> 1) & 1, n_y = (d + 1) & 1, n_buf = (d + 1) & 1;
-        // requests: activations of stage stg + 4 -> slot d; weights of window stg / 2 + 2 -> slot (d >> 1) & 1
-        const int l_wslot = (d >> 1) & 1, l_win = (stg >> 1) + 2;
-        const uint8_t* base = lds + buf * STAGE_BYTES;
-        const uint4* lact = (const uint4*)base;
-        const uint4* lw = (const uint4*)(base + ACT_UNITS * 16);
-        uint4 A[2][FB], W[2][FM];
-        auto load_frags = [&](int t) {
-#pragma unroll
-            for (int i = 0; i < FB; i++) A[t & 1][i] = lact[lds_slot(2 * t + lh, (wb * FB + i) * 32 + ln, TB)];
-#pragma unroll
-            for (int j = 0; j < FM; j++) W[t & 1][j] = lw[lds_slot(2 * t + lh, (wm * FM + j) * 32 + ln, TM)];
-        };
-        load_frags(0);
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (t < 3) load_frags(t + 1);
-#pragma unroll
-            for (int i = 0; i < FB; i++) {
-#pragma unroll
-                for (int j = 0; j < FM; j++) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(t12_bf16x8, A[t & 1][i]), __builtin_bit_cast(t12_bf16x8, W[t & 1][j]),
-                        acc[i][j], 0, 0, 0);
-                    const int m = (t * FB + i) * FM + j;
-                    // chunk c of the staging work goes after MFMA number (c + 1) * NMMA / NCH - 1
-#pragma unroll
-                    for (int c = 0; c < NCH; c++) {
-                        if ((c + 1) * NMMA / NCH - 1 == m) {
-#pragma unroll
-                            for (int u = 0; u < NLU_ODD; u++) {
-                                if (u < nlu && u * NCH / nlu == c) {
-                                    if (u < ACT_LD) {
-                                        if (ld_act) load_act(d, stg + DA, u);
-                                    } else {
-                                        load_w(l_wslot, l_win, u - ACT_LD, ld_x, ld_y);
-                                    }
-                                }
-                            }
-#pragma unroll
-                            for (int u = 0; u < NSU; u++)
-                                if (do_store && u * NCH / NSU == c)
-                                    store_unit(n_aslot, n_wslot, n_y, n_buf, stage_unit_order(u, ACT_LD, 2 * W_LD));
-                            if (do_store && c == PATCH_AT) {
-                                __builtin_amdgcn_sched_barrier(0);
-                                patch_stage(n_y, n_buf, k_begin + (stg + 1) * KC);
-                            }
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    };
-
-    // escape list visible, stage 0 into LDS
-    __syncthreads();
-    if (esc_mode == 1) {
-#pragma unroll
-        for (int y = 0; y < 2; y++)
-#pragma unroll
-            for (int i = 0; i < W_LD; i++) {
-                const int r = w_row[y][i];
-                const int li = SWI ? ((r >> 5) & 1) * (TM / 2 + 1) + ((r >> 6) << 5) + (r & 31) : r;
-                int q = lrow[li];
-                const int qe = lrow[li + 1];
-                while (q < qe && (int)(lpat[q] & 0xFFFFu) < k_begin) q++;   // K split: skip earlier columns
-                pp[y][i] = q;
-                pe[y][i] = qe;
-                if (q < qe) {
-                    cur[y][i] = lpat[q];
-                    behind[y][i] = lpat[q + 1];
-                    nc[y][i] = (int)(cur[y][i] & 0xFFFFu);
-                }
-            }
-    }
-    if (nstage > 0) {
-#pragma unroll
-        for (int u = 0; u < NSU; u++) store_unit(0, 0, 0, 0, u);
-        patch_stage(0, 0, k_begin);
-    }
-    __syncthreads();
-
-    int st = 0;
-    // steady state, unrolled by 4 so that ring slots and buffers are compile-time; no guards inside
-    for (; st + 2 * DA <= nstage; st += DA) {
-#pragma unroll
-        for (int d = 0; d < DA; d++) run_stage(d, st + d, true, true, true, true);
-    }
-    // drain
-    for (; st < nstage; st += DA) {
-#pragma unroll
-        for (int d = 0; d < DA; d++) {
-            const int sn = st + d;
-            if (sn < nstage)
-                run_stage(d, sn, sn + DA < nstage, 2 * ((sn >> 1) + 2) < nstage, 2 * ((sn >> 1) + 2) + 1 < nstage,
-                          sn + 1 < nstage);
-        }
-    }
-
-    // ---- overflow path only (more escapes than the LDS list holds): the streamed value of an
-    //      escape was its "wrong" decode, so acc[b, m] += (correct - wrong) * X[b, col], added by
-    //      the K split that owns column 0
-    if (blockIdx.z == 0 && esc_mode == 2) {
-#pragma unroll
-        for (int j = 0; j < FM; j++) {
-            const T12Segment& g = p.seg[SWI ? s + j : s];
-            const int m = SWI ? m0 + wm * 32 + ln : m0 + (wm * FM + j) * 32 + ln;
-            if (m < M && g.row_off) {
-                const int beg = g.row_off[m], end = g.row_off[m + 1];
-                for (int pp = beg; pp < end; pp++) {
-                    const float delta = t12_bf16_to_f32((uint16_t)g.correct[pp]) -
-                                        t12_bf16_to_f32((uint16_t)g.wrong[pp]);
-                    const uint16_t* xc = act + g.cols[pp];
-#pragma unroll
-                    for (int i = 0; i < FB; i++)
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const int bb = b0 + (wb * FB + i) * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                            if (bb < B) acc[i][j][r] += delta * t12_bf16_to_f32(xc[(size_t)bb * act_stride]);
-                        }
-                }
-            }
-        }
-    }
-
-    // ---- store: accumulator register r of lane (ln, lh) is
-    //      D[row = 8*(r/4) + 4*lh + r%4][col = ln]   (row = batch, col = m)
-    if (SWI) {
-        const int m = m0 + wm * 32 + ln;
-        uint16_t* const ob = p.out_bf16 + (size_t)row_base * p.out_bf16_ld;
-#pragma unroll
-        for (int i = 0; i < FB; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int b = b0 + (wb * FB + i) * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                if (m < M && b < B)
-                    ob[(size_t)b * p.out_bf16_ld + m] = t12_f32_to_bf16(t12_apply_glu(acc[i][0][r], acc[i][FM - 1][r], p.glu));
-            }
-        return true;
-    }
-    if (EPI != T12_ACT_NONE) {
-#pragma unroll
-        for (int i = 0; i < FB; i++)
-#pragma unroll
-            for (int j = 0; j < FM; j++) {
-                const int m = m0 + (wm * FM + j) * 32 + ln;
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int b = b0 + (wb * FB + i) * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                    if (m < M && b < B)
-                        p.out_bf16[(size_t)b * p.out_bf16_ld + m] = t12_f32_to_bf16(t12_apply_act<EPI>(acc[i][j][r], p.act_a, p.act_b));
-                }
-            }
-        return true;
-    }
-    float* dst;
-    size_t ld;
-    if (p.ksplit > 1) {
-        dst = p.ws + (size_t)blockIdx.z * p.split_stride + p.seg_ws0[s];
-        ld = p.seg_ld[s];
-    } else {
-        dst = sg.out + (size_t)row_base * sg.out_stride;
-        ld = sg.out_stride;
-    }
-#pragma unroll
-    for (int i = 0; i < FB; i++)
-#pragma unroll
-        for (int j = 0; j < FM; j++) {
-            const int m = m0 + (wm * FM + j) * 32 + ln;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int b = b0 + (wb * FB + i) * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                if (m < M && b < B) dst[(size_t)b * ld + m] = acc[i][j][r];
-            }
-        }
-    return true;
-}
-
-// Eight waves per workgroup, two per SIMD: one wave's decode / LDS traffic runs under the other's MFMAs.
-// Batch tiles: one per workgroup (blockIdx.y), except when the rows per group are known on the device only: such
-// a launch has one workgroup per row tile, which takes the group's batch tiles one after the other (a group within
-// the tile -- the usual case -- is streamed once, a larger one once per tile; no group's rows can fall outside the grid).
-template <int WB, int WM, int FB, int FM, bool SWI = false, int EPI = T12_ACT_NONE, bool DEV = false>
-__global__ __launch_bounds__(WB * WM * 64) void gemm_mfma_kernel(const GemmParams p)
-{
-    for (int bt = blockIdx.y;; bt++) {
-        if (!gemm_mfma_body<WB, WM, FB, FM, SWI, EPI, DEV>(p, bt) || !DEV) break;
-        __syncthreads();                                   // the next tile reuses the staging buffers
-    }
-}
 
 // ---------------------------------------------------------------------------
 // K-split reduction: out[b, m] = sum over splits z of the partial sums of (b, m), in ascending z
@@ -1160,35 +644,24 @@ float* static_workspace()
 }
 
 
-template <int WB, int WM, int FB, int FM, bool SWI = false, int EPI = T12_ACT_NONE, bool DEV = false>
-int launch_mfma(GemmParams& p, int tiles, hipStream_t st)
+template <int FB, bool SWI = false, int EPI = T12_ACT_NONE, bool DEV = false>
+int launch_tile(GemmParams& p, int tiles, hipStream_t st)
 {
-    constexpr int TB = WB * FB * 32;
-    constexpr int STAGE_BYTES = TB * 8 * 16 + TM * 128;
-    const dim3 grid(tiles, (p.B + TB - 1) / TB, p.ksplit);   // batch tiles of one row tile are neighbours in time
-    auto kfn = gemm_mfma_kernel<WB, WM, FB, FM, SWI, EPI, DEV>;
-    static bool attr_done[16] = {};                    // the attribute is per device
-    static std::mutex attr_mutex;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) dev = 0;
-    {
-        std::lock_guard<std::mutex> attr_lock(attr_mutex);
-        bool& attr_set = attr_done[dev];
-        if (!attr_set) {
-            if (hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    2 * STAGE_BYTES + PATCH_BYTES) !=
-                hipSuccess) {
-                t12_set_error("t12_gemm: cannot reserve %d bytes of LDS", 2 * STAGE_BYTES);
-                return T12_ELAUNCH;
-            }
-            attr_set = true;
-        }
-    }
-    hipLaunchKernelGGL(kfn, grid, dim3(WB * WM * 64), 2 * STAGE_BYTES + PATCH_BYTES, st, p);
+    const dim3 grid(tiles, (p.B + 64 * FB - 1) / (64 * FB), p.ksplit);   // batch tiles of one row tile are neighbours in time
+    if constexpr (FB == 4) hipLaunchKernelGGL((gemm_tile_kernel<SWI, EPI, DEV>), grid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL((gemm_strip_kernel<FB, SWI, EPI, DEV>), grid, dim3(512), 0, st, p);
     T12_CHECK_LAUNCH("t12_gemm");
     return T12_OK;
 }
 
+
+template <bool SWI = false, int EPI = T12_ACT_NONE>
+int launch_wide(GemmParams& p, int tiles, hipStream_t st)
+{
+    hipLaunchKernelGGL((gemm_wide_kernel<SWI, EPI>), dim3(tiles, (p.B + WIDE - 1) / WIDE, p.ksplit), dim3(512), 0, st, p);
+    T12_CHECK_LAUNCH("t12_gemm");
+    return T12_OK;
+}
 
 template <int RW, int KW, int NBT, bool GLU = false, bool DEV = false>
 int launch_ring(GemmParams& p, int tiles, hipStream_t st)
@@ -1213,6 +686,15 @@ int device_cus()
         cus[dev] = n;
     }
     return cus[dev];
+}
+
+// More than 128 rows, unsplit: tiles of 256 x 256 in place of 128 x 256 where their rounds of one workgroup per CU take less time: a round of theirs
+// takes 1.75 of the others' (a stage 1.6 us against 0.93, the ends alike).  28672 x 4096: 512 rows, one round against two, 139 us and 156; 256 rows, one
+// each, 135 and 89; 32000 x 4096 at 256 138 and 89.
+bool prefers_wide(int tiles, int wide, int cus)
+{
+    const int rounds = (tiles + cus - 1) / cus, rounds_wide = (wide + cus - 1) / cus;
+    return rounds_wide * 1.75f < rounds;
 }
 
 // The ring kernel's form for a launch of p's segments (0 .. nseg - 1), or none: 3 .. 64 rows, K of whole 128-column
@@ -1334,7 +816,7 @@ int t12_gemm_glu(const T12Segment* gate, const T12Segment* up, const T12Glu* glu
         T12_CHECK_LAUNCH("t12_gemm_glu(dense16)");
         return T12_OK;
     }
-    const bool fast = K % KC == 0 && aligned && exps;
+    const bool fast = K % KC == 0 && aligned && exps && act_stride <= TILE_MAX_STRIDE;
     const int tiles = (gate->M + TM / 2 - 1) / (TM / 2);
     const int btiles = B > 128 ? (B + 255) / 256 : 1;
     if (!fast || tiles * btiles * 4 < 256 * 3) return 1;      // would need a K split: partial sums cannot be gated
@@ -1342,8 +824,13 @@ int t12_gemm_glu(const T12Segment* gate, const T12Segment* up, const T12Glu* glu
     p.blk_start[0] = 0;
     p.blk_start[1] = p.blk_start[2] = tiles;
     // batch tile of 256 rows, or of 128 for 65 .. 128 rows (one accumulator pair per wave)
-    if (B <= 128) return launch_mfma<4, 2, 1, 2, true>(p, tiles, st);
-    return launch_mfma<4, 2, 2, 2, true>(p, tiles, st);
+    if (B <= 128) return launch_tile<2, true>(p, tiles, st);
+    const int wide = (gate->M + WIDE / 2 - 1) / (WIDE / 2);
+    if (prefers_wide(tiles * btiles, wide * btiles, device_cus())) {
+        p.blk_start[1] = p.blk_start[2] = wide;
+        return launch_wide<true>(p, wide, st);
+    }
+    return launch_tile<4, true>(p, tiles, st);
 }
 
 // out_bf16[b, m] = bf16(act(W[m,:] . X[b,:])) with the function in the GEMM's epilogue.  Returns T12_OK when launched, 1
@@ -1360,8 +847,8 @@ int t12_gemm_act(const T12Segment* seg, const void* act_bf16, int act_stride, in
     const int tiles = (seg->M + TM - 1) / TM, btiles = B > 128 ? (B + 255) / 256 : 1;
     // more than 64 batch rows, and a shape that is not one of few workgroups, which gemm_impl may split along K
     const bool splits = tiles * btiles * 2 <= 256 + 32 && K / 2 >= 8 * KC;
-    if (act->kind != T12_ACT_XIELU || K % KC || act_stride % 8 || (uintptr_t)act_bf16 % 16 || B <= 64 || seg->base_exp < 0 ||
-        seg->base_exp > 240 || splits)
+    if (act->kind != T12_ACT_XIELU || K % KC || act_stride % 8 || act_stride > TILE_MAX_STRIDE || (uintptr_t)act_bf16 % 16 || B <= 64 ||
+        seg->base_exp < 0 || seg->base_exp > 240 || splits)
         return 1;
     GemmParams p;
     p.seg[0] = *seg;
@@ -1384,8 +871,13 @@ int t12_gemm_act(const T12Segment* seg, const void* act_bf16, int act_stride, in
     p.out_bf16_ld = out_stride;
     p.act_a = act->a;
     p.act_b = act->b;
-    if (B <= 128) return launch_mfma<2, 4, 2, 1, false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
-    return launch_mfma<4, 2, 2, 2, false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
+    if (B <= 128) return launch_tile<2, false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
+    const int wide = (seg->M + WIDE - 1) / WIDE;
+    if (prefers_wide(tiles * btiles, wide * btiles, device_cus())) {
+        p.blk_start[1] = wide;
+        return launch_wide<false, T12_ACT_XIELU>(p, wide, (hipStream_t)stream);
+    }
+    return launch_tile<4, false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
 }
 
 }  // extern "C"
@@ -1506,7 +998,7 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
     }
     p.split_stride = (size_t)B * m_total;
 
-    if (!fast) {
+    auto general = [&]() {
         int tiles = 0;
         for (int i = 0; i < nseg; i++) {
             p.blk_start[i] = tiles;
@@ -1518,7 +1010,8 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         hipLaunchKernelGGL(gemm_general_kernel, dim3(tiles, (B + 7) / 8), dim3(256), 0, st, p);
         T12_CHECK_LAUNCH("t12_gemm(general)");
         return T12_OK;
-    }
+    };
+    if (!fast) return general();
 
     int tiles = 0;
     for (int i = 0; i < nseg; i++) {
@@ -1644,6 +1137,7 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         T12_CHECK_LAUNCH("t12_gemm(dense16)");
         return T12_OK;
     }
+    if (act_stride > TILE_MAX_STRIDE) return general();
     // K split: as many workgroups as the chip has CUs, not more (measured on the four Llama-8B layer shapes at B = 32 ..
     // 256: 32 row tiles run best as 8 splits, 48 as 4, 224 unsplit -- every doubling past ~one workgroup per CU costs more
     // in partial sums than it gains), every split at least 8 stages long.
@@ -1696,9 +1190,23 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         if (rc_ws) return rc_ws;
     }
     int rc;
-    if (B <= 64) rc = launch_mfma<2, 4, 1, 1>(p, tiles, st);
-    else if (B <= 128 || tb128) rc = launch_mfma<2, 4, 2, 1>(p, tiles, st);
-    else rc = launch_mfma<4, 2, 2, 2>(p, tiles, st);
+    if (B <= 64) rc = launch_tile<1>(p, tiles, st);
+    else if (B <= 128 || tb128) rc = launch_tile<2>(p, tiles, st);
+    else {
+        int wide = 0;
+        for (int i = 0; i < nseg; i++) wide += (segs[i].M + WIDE - 1) / WIDE;
+        if (ks == 1 && prefers_wide(tiles * btiles, wide * btiles, cus)) {
+            wide = 0;
+            for (int i = 0; i < nseg; i++) {
+                p.blk_start[i] = wide;
+                wide += (segs[i].M + WIDE - 1) / WIDE;
+            }
+            p.blk_start[nseg] = wide;
+            rc = launch_wide(p, wide, st);
+        } else {
+            rc = launch_tile<4>(p, tiles, st);
+        }
+    }
     return rc ? rc : finish();
 }
 
@@ -1755,7 +1263,7 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
         T12_REQUIRE(w.base_exp >= -1 && w.base_exp <= 254, "t12_gemm_grouped: group %d: base_exp %d out of range", i, w.base_exp);
         T12_REQUIRE(g.act_stride >= K && w.out_stride >= w.M, "t12_gemm_grouped: group %d: act_stride %d < K %d or out_stride %d < M %d",
                     i, g.act_stride, K, w.out_stride, w.M);
-        if (w.base_exp < 0 || w.base_exp > 240 || g.act_stride % 8 != 0 || (uintptr_t)g.act_bf16 % 16 != 0) fast = false;
+        if (w.base_exp < 0 || w.base_exp > 240 || g.act_stride % 8 != 0 || g.act_stride > TILE_MAX_STRIDE || (uintptr_t)g.act_bf16 % 16 != 0) fast = false;
         p.seg[n] = w;
         p.seg_row0[n] = m_total;
         p.seg_act[n] = (const uint16_t*)g.act_bf16;
@@ -1807,9 +1315,9 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
         }
     }
     int rc;
-    if (tb == 64) rc = launch_mfma<2, 4, 1, 1>(p, tiles, st);
-    else if (tb == 128) rc = launch_mfma<2, 4, 2, 1>(p, tiles, st);
-    else rc = launch_mfma<4, 2, 2, 2>(p, tiles, st);
+    if (tb == 64) rc = launch_tile<1>(p, tiles, st);
+    else if (tb == 128) rc = launch_tile<2>(p, tiles, st);
+    else rc = launch_tile<4>(p, tiles, st);
     if (rc) return rc;
     if (ks > 1) {
         launch_reduce(p, max_b, st);
@@ -1831,7 +1339,7 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
 {
     const bool swiglu = pairs == 1;
     if (nseg < 1 || nseg > GMAX || (pairs && nseg % 2)) return 1;
-    if (K % KC || act_stride % 8 || (uintptr_t)act_bf16 % 16) return 1;
+    if (K % KC || act_stride % 8 || act_stride > TILE_MAX_STRIDE || (uintptr_t)act_bf16 % 16) return 1;
     for (int i = 0; i < nseg; i++)
         if (segs[i].base_exp < 0 || segs[i].base_exp > 240 || !segs[i].sm || !segs[i].gr) return 1;
     GemmParams p;
@@ -1901,12 +1409,12 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
         return T12_OK;
     }
     if (swiglu) {
-        if (hint_b <= 128) return launch_mfma<4, 2, 1, 2, true, T12_ACT_NONE, true>(p, tiles, st);
-        return launch_mfma<4, 2, 2, 2, true, T12_ACT_NONE, true>(p, tiles, st);
+        if (hint_b <= 128) return launch_tile<2, true, T12_ACT_NONE, true>(p, tiles, st);
+        return launch_tile<4, true, T12_ACT_NONE, true>(p, tiles, st);
     }
-    if (hint_b <= 64) return launch_mfma<2, 4, 1, 1, false, T12_ACT_NONE, true>(p, tiles, st);
-    if (hint_b <= 128) return launch_mfma<2, 4, 2, 1, false, T12_ACT_NONE, true>(p, tiles, st);
-    return launch_mfma<4, 2, 2, 2, false, T12_ACT_NONE, true>(p, tiles, st);
+    if (hint_b <= 64) return launch_tile<1, false, T12_ACT_NONE, true>(p, tiles, st);
+    if (hint_b <= 128) return launch_tile<2, false, T12_ACT_NONE, true>(p, tiles, st);
+    return launch_tile<4, false, T12_ACT_NONE, true>(p, tiles, st);
 }
 
 // The library keeps device buffers per (device, stream): the K-split partial sums of t12_gemm*, the argmax partials and the

@@ -169,7 +169,7 @@ __device__ __forceinline__ bool gemm_ring_body(const GemmParams& p, const int bt
     copy_x(x0, 0);
     copy_w(min(1, T - 1), 1);                                 // (past the last round: the last one again, not used)
 
-    // ---- the escape list of the workgroup's rows -> LDS (esc_mode as in gemm_mfma_body)
+    // ---- the escape list of the workgroup's rows -> LDS (esc_mode as TileList's mode)
     int esc_mode = 0;
     if (GLU) {
         const int r_lo = min(m0, M), r_hi = min(m0 + WR * RW, M);

@@ -81,18 +81,18 @@ __device__ __forceinline__ void t12_decode8(uint32_t s0, uint32_t s1, uint32_t g
 // The same with neighbours in a pair, w[i] = bf16x2 { weight 2 i (low half), weight 2 i + 1 (high half) }: the order
 // activations have in memory, so they need no shuffle of their own.  One operation more per eight weights (the nibbles are
 // parted into bytes first): 19.
+// Dword i of it, from lo = g & 0x0F0F0F0F (nibbles of weights 0 2 4 6) and hi = (g >> 4) & 0x0F0F0F0F (1 3 5 7).
+__device__ __forceinline__ uint32_t t12_decode2_seq(uint32_t s0, uint32_t s1, uint32_t lo, uint32_t hi, uint32_t be2v, int i)
+{
+    const uint32_t m = __builtin_amdgcn_perm(s1, s0, 0x01010000u + 0x02020202u * (uint32_t)i);
+    const uint32_t n = __builtin_amdgcn_perm(hi, lo, 0x0C040C00u + 0x00010001u * (uint32_t)i);      // selector 0x0C: a zero byte
+    return (n << 7) + ((m & 0x807F807Fu) | be2v);
+}
 __device__ __forceinline__ void t12_decode8_seq(uint32_t s0, uint32_t s1, uint32_t g, uint32_t be2v, uint32_t* w)
 {
-    const uint32_t keep = 0x807F807Fu;
-    const uint32_t lo = g & 0x0F0F0F0Fu, hi = (g >> 4) & 0x0F0F0F0Fu;      // nibbles of weights 0 2 4 6, and 1 3 5 7
-    const uint32_t t0 = (__builtin_amdgcn_perm(s1, s0, 0x01010000u) & keep) | be2v;
-    const uint32_t t1 = (__builtin_amdgcn_perm(s1, s0, 0x03030202u) & keep) | be2v;
-    const uint32_t t2 = (__builtin_amdgcn_perm(s1, s0, 0x05050404u) & keep) | be2v;
-    const uint32_t t3 = (__builtin_amdgcn_perm(s1, s0, 0x07070606u) & keep) | be2v;
-    w[0] = (__builtin_amdgcn_perm(hi, lo, 0x0C040C00u) << 7) + t0;         // selector 0x0C: a zero byte
-    w[1] = (__builtin_amdgcn_perm(hi, lo, 0x0C050C01u) << 7) + t1;
-    w[2] = (__builtin_amdgcn_perm(hi, lo, 0x0C060C02u) << 7) + t2;
-    w[3] = (__builtin_amdgcn_perm(hi, lo, 0x0C070C03u) << 7) + t3;
+    const uint32_t lo = g & 0x0F0F0F0Fu, hi = (g >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = t12_decode2_seq(s0, s1, lo, hi, be2v, i);
 }
 
 // Activations that pair with t12_decode8: from 8 consecutive bf16 (x0..x7 in four
