@@ -193,14 +193,14 @@ struct TileCursor {
     }
 };
 
-// The end of a multiplying wave: acc holds 32 FB batch rows from b0 + row0 on x 64 weight rows (SWI: 32 of gate and of up), mw the first of them.
-template <int FB, bool SWI, int EPI, class Job>
-__device__ __forceinline__ void tile_finish(const GemmParams& p, const Job& j, int esc_mode, int row0, int mw, t12_f32x16 (&acc)[FB][2])
+// The sums of a multiplying wave: acc holds 32 FB batch rows from b0 + row0 on x 64 weight rows (SWI: 32 of gate and of up), mw the first of them.
+// Overflow path only: the streamed value of an escape was its "wrong" decode, so acc[b, m] += (correct - wrong) * X[b, col], added by the K split that
+// owns column 0.
+template <int FB, bool SWI, class Job>
+__device__ __forceinline__ void tile_overflow(const GemmParams& p, const Job& j, int esc_mode, int row0, int mw, t12_f32x16 (&acc)[FB][2])
 {
     const int lane = threadIdx.x & 63, ln = lane & 31, lh = lane >> 5;
     const int b0 = j.b0 + row0;
-    // ---- overflow path only: the streamed value of an escape was its "wrong" decode, so acc[b, m] += (correct - wrong) * X[b, col], added by
-    //      the K split that owns column 0
     if (blockIdx.z == 0 && esc_mode == 2) {
 #pragma unroll
         for (int u = 0; u < 2; u++) {
@@ -224,11 +224,20 @@ __device__ __forceinline__ void tile_finish(const GemmParams& p, const Job& j, i
             }
         }
     }
+}
 
-    // ---- store: accumulator register r of lane (ln, lh) is D[row = 8*(r/4) + 4*lh + r%4][col = ln]   (row = batch, col = m).  A row's
-    //      address is the wave's, the lanes add theirs: 64 addresses and conditions of a lane each would not fit its registers.
+template <bool SWI, int EPI>
+constexpr bool TILE_HALF = SWI || EPI != T12_ACT_NONE;          // bf16 results of a function of the sums
+
+// Stores the sums FIRST .. END - 1 of them, number 16 i + r register r of acc[i].  Register r of lane (ln, lh) is D[row = 8*(r/4) + 4*lh + r%4][col = ln]
+// (row = batch, col = m).  A row's address is the wave's, the lanes add theirs: 64 addresses and conditions of a lane each would not fit its registers.
+template <int FB, bool SWI, int EPI, int FIRST, int END, class Job>
+__device__ __forceinline__ void tile_store(const GemmParams& p, const Job& j, int row0, int mw, const t12_f32x16 (&acc)[FB][2])
+{
+    const int lane = threadIdx.x & 63, ln = lane & 31, lh = lane >> 5;
+    const int b0 = j.b0 + row0;
     const bool in0 = mw + ln < j.M, in1 = !SWI && mw + 32 + ln < j.M;
-    constexpr bool HALF = SWI || EPI != T12_ACT_NONE;          // bf16 results
+    constexpr bool HALF = TILE_HALF<SWI, EPI>;
     uint8_t* dst;
     size_t ld;
     if (HALF) {
@@ -244,23 +253,66 @@ __device__ __forceinline__ void tile_finish(const GemmParams& p, const Job& j, i
     constexpr int ES = HALF ? 2 : 4;
     const size_t lane_at = ((size_t)(4 * lh) * ld + ln) * ES;
 #pragma unroll
-    for (int i = 0; i < FB; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int b = b0 + 32 * i + 8 * (r >> 2) + (r & 3);                      // of the lanes' lower half
-            uint8_t* const at = dst + (size_t)b * ld * ES + lane_at;
-            if (b + 4 * lh < j.B) {
-                if (SWI) {
-                    if (in0) *(uint16_t*)at = t12_f32_to_bf16(t12_apply_glu(acc[i][0][r], acc[i][1][r], p.glu));
-                } else if (EPI != T12_ACT_NONE) {
-                    if (in0) *(uint16_t*)at = t12_f32_to_bf16(t12_apply_act<EPI>(acc[i][0][r], p.act_a, p.act_b));
-                    if (in1) *(uint16_t*)(at + 64) = t12_f32_to_bf16(t12_apply_act<EPI>(acc[i][1][r], p.act_a, p.act_b));
-                } else {
-                    if (in0) *(float*)at = acc[i][0][r];
-                    if (in1) *(float*)(at + 128) = acc[i][1][r];
-                }
+    for (int n = FIRST; n < END; n++) {
+        const int i = n >> 4, r = n & 15;
+        const int b = b0 + 32 * i + 8 * (r >> 2) + (r & 3);                          // of the lanes' lower half
+        uint8_t* const at = dst + (size_t)b * ld * ES + lane_at;
+        if (b + 4 * lh < j.B) {
+            if (SWI) {
+                if (in0) *(uint16_t*)at = t12_f32_to_bf16(t12_apply_glu(acc[i][0][r], acc[i][1][r], p.glu));
+            } else if (HALF) {
+                if (in0) *(uint16_t*)at = t12_f32_to_bf16(t12_apply_act<EPI>(acc[i][0][r], p.act_a, p.act_b));
+                if (in1) *(uint16_t*)(at + 64) = t12_f32_to_bf16(t12_apply_act<EPI>(acc[i][1][r], p.act_a, p.act_b));
+            } else {
+                if (in0) *(float*)at = acc[i][0][r];
+                if (in1) *(float*)(at + 128) = acc[i][1][r];
             }
         }
+    }
+}
+
+// The end of a tile of four multiplying and four copying waves, all eight there.  What follows a function of the sums is bound by that function's
+// operations (gated unit: 45 a pair), so each copying wave takes half of the sums of a multiplying one, through the LDS of the activations (lx, free by
+// then): gated 28672 x 512 at B = 256 24.1 -> 20.2 us, 28672 x 4096 at 100 / 256 64 -> 62.5, 81.2 -> 79.6.  Plain sums are bound by their stores and stay where they are.  wave: 0 .. 3 of its kind.
+template <int FB, bool SWI, int EPI, class Job>
+__device__ __forceinline__ void tile_finish(const GemmParams& p, const Job& j, int esc_mode, int row0, int mw, int wave, uint8_t* lx, t12_f32x16 (&acc)[FB][2])
+{
+    constexpr int N = 16 * FB, KEEP = TILE_HALF<SWI, EPI> ? N / 2 : N;
+    tile_overflow<FB, SWI>(p, j, esc_mode, row0, mw, acc);
+    if (KEEP < N) {
+        tile_barrier();                                        // the copies of both kinds of waves have ended
+        uint8_t* const to = lx + wave * (N / 2 * 512) + (threadIdx.x & 63) * 16;
+#pragma unroll
+        for (int n = KEEP; n < N; n += 4)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const t12_f32x16& a = acc[n >> 4][u];
+                *(t12_f32x4*)(to + ((n - KEEP) / 4 * 2 + u) * 1024) = t12_f32x4{a[n & 15], a[(n & 15) + 1], a[(n & 15) + 2], a[(n & 15) + 3]};
+            }
+        __builtin_amdgcn_s_waitcnt(TILE_LDS_DONE);
+        tile_barrier();
+    }
+    tile_store<FB, SWI, EPI, 0, KEEP>(p, j, row0, mw, acc);
+}
+template <int FB, bool SWI, int EPI, class Job>
+__device__ __forceinline__ void tile_finish_copying(const GemmParams& p, const Job& j, int row0, int mw, int wave, const uint8_t* lx)
+{
+    constexpr int N = 16 * FB, KEEP = N / 2;
+    __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));             // no copy outlives its workgroup or reaches into its next tile
+    if (!TILE_HALF<SWI, EPI>) return;
+    tile_barrier();
+    tile_barrier();                                        // the sums are there
+    t12_f32x16 acc[FB][2];
+    const uint8_t* const at = lx + wave * (N / 2 * 512) + (threadIdx.x & 63) * 16;
+#pragma unroll
+    for (int n = KEEP; n < N; n += 4)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const t12_f32x4 a = *(const t12_f32x4*)(at + ((n - KEEP) / 4 * 2 + u) * 1024);
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[n >> 4][u][(n & 15) + q] = a[q];
+        }
+    tile_store<FB, SWI, EPI, KEEP, N>(p, j, row0, mw, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -404,7 +456,7 @@ __device__ __forceinline__ bool gemm_tile_body(const GemmParams& p, const int ti
                 if (st + 2 < nstage) interval(std::integral_constant<int, 2>(), st + 2, std::false_type());
             }
         }
-        __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));             // no copy outlives its workgroup or reaches into its next tile
+        tile_finish_copying<FB, SWI, EPI>(p, j, ((wave - 4) >> 1) * (FB * 32), j.m0 + (wave & 1) * (SWI ? 32 : 64), wave - 4, lx);
         return true;
     }
 
@@ -487,7 +539,7 @@ __device__ __forceinline__ bool gemm_tile_body(const GemmParams& p, const int ti
             if (st + 2 < nstage) stage(std::integral_constant<int, 2>(), st + 2);
         }
     }
-    tile_finish<FB, SWI, EPI>(p, j, list.mode, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), acc);
+    tile_finish<FB, SWI, EPI>(p, j, list.mode, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), wave, lx, acc);
     return true;
 }
 
@@ -648,7 +700,7 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
         }
         interval(std::integral_constant<int, 0>(), w, std::false_type());
         if (w + 1 < nwin) interval(std::integral_constant<int, 1>(), w + 1, std::false_type());
-        __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));             // no copy outlives its workgroup or reaches into its next tile
+        tile_finish_copying<FB, SWI, EPI>(p, j, ((wave - 4) >> 1) * (FB * 32), j.m0 + (wave & 1) * (SWI ? 32 : 64), wave - 4, lx);
         return true;
     }
 
@@ -744,7 +796,7 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
     } else {
         window(std::integral_constant<int, 0>(), w, odd);
     }
-    tile_finish<FB, SWI, EPI>(p, j, list.mode, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), acc);
+    tile_finish<FB, SWI, EPI>(p, j, list.mode, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), wave, lx, acc);
     return true;
 }
 
@@ -935,7 +987,8 @@ __device__ __forceinline__ void gemm_wide_body(const GemmParams& p, const int ti
     }
     if (st < nstage) stage(std::integral_constant<int, 0>(), st);
     __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));                 // no copy outlives its workgroup
-    tile_finish<FB, SWI, EPI>(p, j, list.mode, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), acc);
+    tile_overflow<FB, SWI>(p, j, list.mode, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), acc);
+    tile_store<FB, SWI, EPI, 0, 16 * FB>(p, j, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), acc);
 }
 
 template <bool SWI = false, int EPI = T12_ACT_NONE>
