@@ -550,3 +550,22 @@ def test_gemm_two_to_four_rows_whole_row_kernel(t12, oracle, synth, M, K, law, B
         outs = run_gemm(t12, ps, X)
         for q, o in zip(ps, outs):
             assert rel_err(o, oracle.gemm(q, X)) < TOL
+
+
+@pytest.mark.parametrize("B", [65, 130])
+def test_gemm_swiglu_rows_further_apart_than_a_tile_reaches(t12, B):
+    """Activation rows 2^22 + 8 elements apart (beyond the 32-bit offsets of a tile): the same bits as rows side by side."""
+    M, K, far = 12300, 128, (1 << 22) + 8
+    st = t12.current_stream()
+    g = torch.Generator(device=dev()).manual_seed(1)
+    gate, up = (t12.pack_device((torch.randn((M, K), generator=g, device=dev()) * 0.02).to(torch.bfloat16)) for _ in range(2))
+    X = torch.randn((B, K), generator=g, device=dev()).to(torch.bfloat16).view(torch.int16)
+    wide = torch.empty((B, far), dtype=torch.int16, device=dev())
+    wide[:, :K] = X
+    want = torch.zeros((B, M), dtype=torch.int16, device=dev())
+    got = torch.zeros_like(want)
+    sg, su = t12._seg_array([gate.segment(None)]), t12._seg_array([up.segment(None)])
+    assert t12.lib.t12_gemm_swiglu(sg, su, X.data_ptr(), K, K, B, want.data_ptr(), M, st) == 0
+    assert t12.lib.t12_gemm_swiglu(sg, su, wide.data_ptr(), far, K, B, got.data_ptr(), M, st) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)

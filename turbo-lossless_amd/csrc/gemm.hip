@@ -688,6 +688,21 @@ int device_cus()
     return cus[dev];
 }
 
+// Activation rows too far apart for the 32-bit offsets of a tile: as many rows per launch as these reach, in the same order of sums.
+template <bool SWI, int EPI>
+int launch_reach(GemmParams p, int tiles, hipStream_t st)
+{
+    const int B = p.B, reach = (int)std::max<int64_t>(1, std::min<int64_t>(128, ((int64_t)TILE_MAX_STRIDE << 8) / p.act_stride));
+    for (int b = 0; b < B; b += reach) {
+        p.B = p.seg_B[0] = std::min(reach, B - b);
+        if (const int rc = launch_tile<2, SWI, EPI>(p, tiles, st)) return rc;
+        p.act += (size_t)reach * p.act_stride;
+        p.seg_act[0] = p.act;
+        p.out_bf16 += (size_t)reach * p.out_bf16_ld;
+    }
+    return T12_OK;
+}
+
 // More than 128 rows, unsplit: tiles of 256 x 256 in place of 128 x 256 where their rounds of one workgroup per CU take less time: a round of theirs
 // takes 1.75 of the others' (a stage 1.6 us against 0.93, the ends alike).  28672 x 4096: 512 rows, one round against two, 139 us and 156; 256 rows, one
 // each, 135 and 89; 32000 x 4096 at 256 138 and 89.
@@ -816,13 +831,14 @@ int t12_gemm_glu(const T12Segment* gate, const T12Segment* up, const T12Glu* glu
         T12_CHECK_LAUNCH("t12_gemm_glu(dense16)");
         return T12_OK;
     }
-    const bool fast = K % KC == 0 && aligned && exps && act_stride <= TILE_MAX_STRIDE;
+    const bool fast = K % KC == 0 && K <= TILE_MAX_STRIDE && aligned && exps;
     const int tiles = (gate->M + TM / 2 - 1) / (TM / 2);
     const int btiles = B > 128 ? (B + 255) / 256 : 1;
     if (!fast || tiles * btiles * 4 < 256 * 3) return 1;      // would need a K split: partial sums cannot be gated
     p.kslice = ((K + 2 * KC - 1) / (2 * KC)) * 2 * KC;
     p.blk_start[0] = 0;
     p.blk_start[1] = p.blk_start[2] = tiles;
+    if (act_stride > TILE_MAX_STRIDE) return launch_reach<true, T12_ACT_NONE>(p, tiles, st);
     // batch tile of 256 rows, or of 128 for 65 .. 128 rows (one accumulator pair per wave)
     if (B <= 128) return launch_tile<2, true>(p, tiles, st);
     const int wide = (gate->M + WIDE / 2 - 1) / (WIDE / 2);
@@ -847,7 +863,7 @@ int t12_gemm_act(const T12Segment* seg, const void* act_bf16, int act_stride, in
     const int tiles = (seg->M + TM - 1) / TM, btiles = B > 128 ? (B + 255) / 256 : 1;
     // more than 64 batch rows, and a shape that is not one of few workgroups, which gemm_impl may split along K
     const bool splits = tiles * btiles * 2 <= 256 + 32 && K / 2 >= 8 * KC;
-    if (act->kind != T12_ACT_XIELU || K % KC || act_stride % 8 || act_stride > TILE_MAX_STRIDE || (uintptr_t)act_bf16 % 16 || B <= 64 ||
+    if (act->kind != T12_ACT_XIELU || K % KC || K > TILE_MAX_STRIDE || act_stride % 8 || (uintptr_t)act_bf16 % 16 || B <= 64 ||
         seg->base_exp < 0 || seg->base_exp > 240 || splits)
         return 1;
     GemmParams p;
@@ -871,6 +887,7 @@ int t12_gemm_act(const T12Segment* seg, const void* act_bf16, int act_stride, in
     p.out_bf16_ld = out_stride;
     p.act_a = act->a;
     p.act_b = act->b;
+    if (act_stride > TILE_MAX_STRIDE) return launch_reach<false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
     if (B <= 128) return launch_tile<2, false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
     const int wide = (seg->M + WIDE - 1) / WIDE;
     if (prefers_wide(tiles * btiles, wide * btiles, device_cus())) {
