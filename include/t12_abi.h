@@ -193,7 +193,7 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream);
  * of 2048 columns and more, every pair is one matrix-vector product with its expert's tensors, picked on the device,
  * gate|up with the SwiGLU in the epilogue).  An id
  * outside 0..E-1 leaves its pair out of the sum and raises a flag that t12_moe_status reads (it waits for the stream).
- * Shapes the tile kernel does not take (n_embd or n_ff not a multiple of 64, base_exp outside 0..240) copy the counts
+ * Shapes the tile kernel does not take (n_embd or n_ff not a multiple of 64 or above 2^22, base_exp outside 0..240) copy the counts
  * to the host and wait once per call.
  * workspace: device memory of t12_moe_workspace_bytes(...) bytes, 256-byte aligned, owned by the caller (used from the
  * first launch to the last).  Up to 128 experts; w1, w3 are [n_ff, n_embd], w2 is [n_embd, n_ff]; their out fields are

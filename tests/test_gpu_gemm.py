@@ -569,3 +569,72 @@ def test_gemm_swiglu_rows_further_apart_than_a_tile_reaches(t12, B):
     assert t12.lib.t12_gemm_swiglu(sg, su, wide.data_ptr(), far, K, B, got.data_ptr(), M, st) == 0
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B, more", [(40, 8), (70, (1 << 24) - (1 << 22) + 8), (130, 8), (512, 8)])
+def test_gemm_rows_far_apart(t12, B, more):
+    """Activation rows beyond a tile's 32-bit offsets (2^22 elements), and beyond what as many bytes reach over a tile of 64 rows (2^24): the same bits
+    as rows side by side, with and without a K split, with lists that fit a tile's 2048 places and ones that do not, through every entry
+    point; the gated form gives the bits of the two launches; what splits too far for the fixed workspace stays refused."""
+    import ctypes as C
+    far, st = (1 << 22) + more, t12.current_stream()
+    g = torch.Generator(device=dev()).manual_seed(B)
+
+    def tensor(m, k, p_out):
+        w = torch.randn((m, k), generator=g, device=dev()) * 0.02
+        return t12.pack_device(torch.where(torch.rand((m, k), generator=g, device=dev()) < p_out, 512.0, w).to(torch.bfloat16))
+
+    space = torch.zeros((B, far), dtype=torch.int16, device=dev())
+
+    def rows(k):
+        near = torch.randn((B, k), generator=g, device=dev()).to(torch.bfloat16).view(torch.int16)
+        space[:, :k] = near
+        return near, space[:, :k]
+
+    for k, sizes, p_out in ((192, (300,), 1e-3), (2112, (300, 129), 2e-3), (2112, (129, 300), 5e-2)):
+        W = [tensor(m, k, p_out) for m in sizes]
+        near, wide = rows(k)
+        want = t12.gemm(W, near)
+        assert all(torch.equal(a, b) for a, b in zip(want, t12.gemm(W, wide)))
+        outs = [torch.empty((B, m), device=dev()) for m in sizes]
+        segs = t12._seg_array([w.segment(o) for w, o in zip(W, outs)])
+        t12.check(t12.lib.t12_gemm_noalloc(segs, len(W), wide.data_ptr(), far, sizes[0], k, B, st))
+        assert all(torch.equal(a, b) for a, b in zip(want, outs))
+        part, part_near = t12.GemmPartials(), t12.GemmPartials()
+        t12.check(t12.lib.t12_gemm_deferred(segs, len(W), near.data_ptr(), k, sizes[0], k, B, C.byref(part_near), st))
+        t12.check(t12.lib.t12_gemm_deferred(segs, len(W), wide.data_ptr(), far, sizes[0], k, B, C.byref(part), st))
+        assert part.nsplit == part_near.nsplit and (part.nsplit > 1) == (k == 2112)
+        moe = importlib.import_module("turbo_lossless_amd.moe")
+        pair = [[(w, x, torch.empty((x.shape[0], w.M), device=dev())) for w, x in zip(W * 2, (y, near[:5], y, y[:1]))] for y in (near, wide)]
+        for items in pair:
+            moe.gemm_grouped(items, k)
+        assert all(torch.equal(a[2], b[2]) for a, b in zip(*pair))
+    if B > 64:
+        M, k = 18688, 128                                                    # whole tiles: all of them hold their list, or none does
+        gate, up = tensor(M, k, 2e-3), tensor(M, k, 0.3)
+        near, wide = rows(k)
+        want, got = (torch.empty((B, M), dtype=torch.int16, device=dev()) for _ in range(2))
+
+        def glu(a, b, x, stride, o):
+            assert t12.lib.t12_gemm_swiglu(t12._seg_array([a.segment(None)]), t12._seg_array([b.segment(None)]), x.data_ptr(), stride, k, B, o.data_ptr(), M, st) == 0
+
+        og, = t12.gemm([gate], wide)
+        t12.lib.launch_silu_mul_bf16_batch(og.data_ptr(), og.data_ptr(), want.data_ptr(), M, B, st)
+        glu(gate, gate, wide, far, got)
+        assert torch.equal(got, want)
+        glu(gate, up, near, k, want)
+        glu(gate, up, wide, far, got)
+        assert torch.equal(got, want)
+        xie = t12.Act(t12.ACT_XIELU, 0.8, 1.1)
+        for w in (gate, up):
+            for x, stride, o in ((near, k, want), (wide, far, got)):
+                assert t12.lib.t12_gemm_act(t12._seg_array([w.segment(None)]), x.data_ptr(), stride, k, B, xie, o.data_ptr(), M, st) == 0
+            assert torch.equal(got, want)
+    if B == 512:
+        k, M = 8192, 2304                                                    # 18 row tiles x 2 batch tiles x 8 slices: 37.7 MB of sums
+        w = tensor(M, k, 0.0)
+        near, wide = rows(k)
+        out = torch.empty((B, M), device=dev())
+        seg = t12._seg_array([w.segment(out)])
+        rc = [t12.lib.t12_gemm_noalloc(seg, 1, x.data_ptr(), s, M, k, B, st) for x, s in ((near, k), (wide, far))]
+        assert rc == [-1, -1]

@@ -655,6 +655,16 @@ int launch_tile(GemmParams& p, int tiles, hipStream_t st)
 }
 
 
+// Activation rows too far apart for a tile's 32-bit offsets: tiles of 128 batch rows whose lanes hold addresses, for any batch.  14336 x 4096 at 100 / 256
+// rows 2^22 + 8 apart 36.0 / 61.6 us, side by side 35.5 / 53.4; the general kernel 3280 / 8130.
+template <bool SWI = false, int EPI = T12_ACT_NONE>
+int launch_far(GemmParams& p, int tiles, hipStream_t st)
+{
+    hipLaunchKernelGGL((gemm_strip_kernel<2, SWI, EPI, false, true>), dim3(tiles, (p.B + 127) / 128, p.ksplit), dim3(512), 0, st, p);
+    T12_CHECK_LAUNCH("t12_gemm");
+    return T12_OK;
+}
+
 template <bool SWI = false, int EPI = T12_ACT_NONE>
 int launch_wide(GemmParams& p, int tiles, hipStream_t st)
 {
@@ -686,21 +696,6 @@ int device_cus()
         cus[dev] = n;
     }
     return cus[dev];
-}
-
-// Activation rows too far apart for the 32-bit offsets of a tile: as many rows per launch as these reach, in the same order of sums.
-template <bool SWI, int EPI>
-int launch_reach(GemmParams p, int tiles, hipStream_t st)
-{
-    const int B = p.B, reach = (int)std::max<int64_t>(1, std::min<int64_t>(128, ((int64_t)TILE_MAX_STRIDE << 8) / p.act_stride));
-    for (int b = 0; b < B; b += reach) {
-        p.B = p.seg_B[0] = std::min(reach, B - b);
-        if (const int rc = launch_tile<2, SWI, EPI>(p, tiles, st)) return rc;
-        p.act += (size_t)reach * p.act_stride;
-        p.seg_act[0] = p.act;
-        p.out_bf16 += (size_t)reach * p.out_bf16_ld;
-    }
-    return T12_OK;
 }
 
 // More than 128 rows, unsplit: tiles of 256 x 256 in place of 128 x 256 where their rounds of one workgroup per CU take less time: a round of theirs
@@ -831,14 +826,14 @@ int t12_gemm_glu(const T12Segment* gate, const T12Segment* up, const T12Glu* glu
         T12_CHECK_LAUNCH("t12_gemm_glu(dense16)");
         return T12_OK;
     }
-    const bool fast = K % KC == 0 && K <= TILE_MAX_STRIDE && aligned && exps;
+    const bool fast = K % KC == 0 && aligned && exps;
     const int tiles = (gate->M + TM / 2 - 1) / (TM / 2);
     const int btiles = B > 128 ? (B + 255) / 256 : 1;
     if (!fast || tiles * btiles * 4 < 256 * 3) return 1;      // would need a K split: partial sums cannot be gated
     p.kslice = ((K + 2 * KC - 1) / (2 * KC)) * 2 * KC;
     p.blk_start[0] = 0;
     p.blk_start[1] = p.blk_start[2] = tiles;
-    if (act_stride > TILE_MAX_STRIDE) return launch_reach<true, T12_ACT_NONE>(p, tiles, st);
+    if (act_stride > TILE_MAX_STRIDE) return launch_far<true>(p, tiles, st);
     // batch tile of 256 rows, or of 128 for 65 .. 128 rows (one accumulator pair per wave)
     if (B <= 128) return launch_tile<2, true>(p, tiles, st);
     const int wide = (gate->M + WIDE / 2 - 1) / (WIDE / 2);
@@ -863,8 +858,8 @@ int t12_gemm_act(const T12Segment* seg, const void* act_bf16, int act_stride, in
     const int tiles = (seg->M + TM - 1) / TM, btiles = B > 128 ? (B + 255) / 256 : 1;
     // more than 64 batch rows, and a shape that is not one of few workgroups, which gemm_impl may split along K
     const bool splits = tiles * btiles * 2 <= 256 + 32 && K / 2 >= 8 * KC;
-    if (act->kind != T12_ACT_XIELU || K % KC || K > TILE_MAX_STRIDE || act_stride % 8 || (uintptr_t)act_bf16 % 16 || B <= 64 ||
-        seg->base_exp < 0 || seg->base_exp > 240 || splits)
+    if (act->kind != T12_ACT_XIELU || K % KC || act_stride % 8 || (uintptr_t)act_bf16 % 16 || B <= 64 || seg->base_exp < 0 ||
+        seg->base_exp > 240 || splits)
         return 1;
     GemmParams p;
     p.seg[0] = *seg;
@@ -887,7 +882,7 @@ int t12_gemm_act(const T12Segment* seg, const void* act_bf16, int act_stride, in
     p.out_bf16_ld = out_stride;
     p.act_a = act->a;
     p.act_b = act->b;
-    if (act_stride > TILE_MAX_STRIDE) return launch_reach<false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
+    if (act_stride > TILE_MAX_STRIDE) return launch_far<false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
     if (B <= 128) return launch_tile<2, false, T12_ACT_XIELU>(p, tiles, (hipStream_t)stream);
     const int wide = (seg->M + WIDE - 1) / WIDE;
     if (prefers_wide(tiles * btiles, wide * btiles, device_cus())) {
@@ -1015,7 +1010,7 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
     }
     p.split_stride = (size_t)B * m_total;
 
-    auto general = [&]() {
+    if (!fast) {
         int tiles = 0;
         for (int i = 0; i < nseg; i++) {
             p.blk_start[i] = tiles;
@@ -1027,8 +1022,7 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         hipLaunchKernelGGL(gemm_general_kernel, dim3(tiles, (B + 7) / 8), dim3(256), 0, st, p);
         T12_CHECK_LAUNCH("t12_gemm(general)");
         return T12_OK;
-    };
-    if (!fast) return general();
+    }
 
     int tiles = 0;
     for (int i = 0; i < nseg; i++) {
@@ -1154,7 +1148,6 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         T12_CHECK_LAUNCH("t12_gemm(dense16)");
         return T12_OK;
     }
-    if (act_stride > TILE_MAX_STRIDE) return general();
     // K split: as many workgroups as the chip has CUs, not more (measured on the four Llama-8B layer shapes at B = 32 ..
     // 256: 32 row tiles run best as 8 splits, 48 as 4, 224 unsplit -- every doubling past ~one workgroup per CU costs more
     // in partial sums than it gains), every split at least 8 stages long.
@@ -1207,7 +1200,8 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         if (rc_ws) return rc_ws;
     }
     int rc;
-    if (B <= 64) rc = launch_tile<1>(p, tiles, st);
+    if (act_stride > TILE_MAX_STRIDE) rc = launch_far(p, tiles, st);
+    else if (B <= 64) rc = launch_tile<1>(p, tiles, st);
     else if (B <= 128 || tb128) rc = launch_tile<2>(p, tiles, st);
     else {
         int wide = 0;
@@ -1268,7 +1262,7 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
     p.out_bf16 = nullptr;
     p.out_bf16_ld = 0;
     bool fast = K % KC == 0;
-    int n = 0, m_total = 0, max_b = 0;
+    int n = 0, m_total = 0, max_b = 0, max_stride = 0;
     size_t ws_floats = 0;
     for (int i = 0; i < ngroups; i++) {
         const T12Group& g = groups[i];
@@ -1280,7 +1274,7 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
         T12_REQUIRE(w.base_exp >= -1 && w.base_exp <= 254, "t12_gemm_grouped: group %d: base_exp %d out of range", i, w.base_exp);
         T12_REQUIRE(g.act_stride >= K && w.out_stride >= w.M, "t12_gemm_grouped: group %d: act_stride %d < K %d or out_stride %d < M %d",
                     i, g.act_stride, K, w.out_stride, w.M);
-        if (w.base_exp < 0 || w.base_exp > 240 || g.act_stride % 8 != 0 || g.act_stride > TILE_MAX_STRIDE || (uintptr_t)g.act_bf16 % 16 != 0) fast = false;
+        if (w.base_exp < 0 || w.base_exp > 240 || g.act_stride % 8 != 0 || (uintptr_t)g.act_bf16 % 16 != 0) fast = false;
         p.seg[n] = w;
         p.seg_row0[n] = m_total;
         p.seg_act[n] = (const uint16_t*)g.act_bf16;
@@ -1290,7 +1284,8 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
         p.seg_ld[n] = w.M;
         ws_floats += (size_t)g.B * w.M;
         m_total += w.M;
-        max_b = g.B > max_b ? g.B : max_b;
+        max_b = std::max(max_b, g.B);
+        max_stride = std::max(max_stride, g.act_stride);
         n++;
     }
     if (n == 0) return T12_OK;
@@ -1332,7 +1327,8 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
         }
     }
     int rc;
-    if (tb == 64) rc = launch_tile<1>(p, tiles, st);
+    if (max_stride > TILE_MAX_STRIDE) rc = launch_far(p, tiles, st);
+    else if (tb == 64) rc = launch_tile<1>(p, tiles, st);
     else if (tb == 128) rc = launch_tile<2>(p, tiles, st);
     else rc = launch_tile<4>(p, tiles, st);
     if (rc) return rc;
@@ -1356,7 +1352,7 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
 {
     const bool swiglu = pairs == 1;
     if (nseg < 1 || nseg > GMAX || (pairs && nseg % 2)) return 1;
-    if (K % KC || act_stride % 8 || act_stride > TILE_MAX_STRIDE || (uintptr_t)act_bf16 % 16) return 1;
+    if (K % KC || act_stride % 8 || (uintptr_t)act_bf16 % 16) return 1;
     for (int i = 0; i < nseg; i++)
         if (segs[i].base_exp < 0 || segs[i].base_exp > 240 || !segs[i].sm || !segs[i].gr) return 1;
     GemmParams p;
@@ -1425,6 +1421,7 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
         T12_CHECK_LAUNCH("t12_moe_ffn(dense16)");
         return T12_OK;
     }
+    if (act_stride > TILE_MAX_STRIDE) return 1;
     if (swiglu) {
         if (hint_b <= 128) return launch_tile<2, true, T12_ACT_NONE, true>(p, tiles, st);
         return launch_tile<4, true, T12_ACT_NONE, true>(p, tiles, st);

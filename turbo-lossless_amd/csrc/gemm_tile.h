@@ -56,7 +56,11 @@ __device__ __forceinline__ int scalar_load(const int* p) { return *(const __attr
 // = consecutive rows of one unit).  Unit u ^ 1 of a row lies at its slot ^ 1, 2 t units on at slot ^ (2 t) (and their rows on).
 __device__ __forceinline__ int lds_slot(int u, int r, int rows) { return u * rows + (r ^ (u & 7)); }
 
-constexpr int TILE_MAX_STRIDE = 1 << 22;      // activation row stride (so K too) up to which a tile's 32-bit offsets reach
+// Activation row stride (so K too) up to which a tile's 32-bit offsets reach: 256 rows of activations or of weights at 2^31 bytes, half of the range.
+// Rows further apart go to gemm_strip_kernel<FAR>, whose lanes hold addresses: same K slices and order of sums, so the same bits.
+constexpr int TILE_MAX_STRIDE = 1 << 22;
+template <class T>
+__device__ __forceinline__ T global_load(const void* p) { return *(const __attribute__((address_space(1))) T*)(uintptr_t)p; }
 
 // Workgroups go round the eight XCDs; the batch tiles of one row tile follow each other on the same one, whose L2 then holds the row tile's planes
 // for all of them.
@@ -575,7 +579,7 @@ struct StripLds {
     static constexpr int NXB = FB == 2 ? 2 : 3;
 };
 
-template <int FB, bool SWI, int EPI, bool DEV>
+template <int FB, bool SWI, int EPI, bool DEV, bool FAR>
 __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int tile, const int bt, uint8_t* const lx, uint8_t* const lw,
                                                 uint32_t* const lpat, int* const lrow)
 {
@@ -596,7 +600,10 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
     const T12Segment& sw = SWI && wave >= 4 ? j.sg1 : j.sg;
     const size_t first = (size_t)j.m0 * j.K + k_begin;
     const auto s_buf = tile_buffer(sw.sm + first), g_buf = tile_buffer(sw.gr + (first >> 1));
-    const uint32_t s_off = (uint32_t)(min(j.m0 + j.rel(w_row), j.M - 1) - j.m0) * (uint32_t)j.K + 16u * cc, g_off = s_off >> 1;
+    const int w_at = min(j.m0 + j.rel(w_row), j.M - 1) - j.m0;
+    const uint32_t s_off = (uint32_t)w_at * (uint32_t)j.K + 16u * cc, g_off = s_off >> 1;
+    const size_t far = first + (size_t)w_at * j.K + 16 * cc;
+    const uint8_t *const s_far = sw.sm + far, *const g_far = sw.gr + (far >> 1);
     const uint32_t be = __builtin_amdgcn_readfirstlane(sw.base_exp);
     const uint32_t be2 = t12_opaque((be << 7) | (be << 23));
     const int w_dst = lds_slot(2 * cc, w_row, TM) * 16;           // unit 2 cc; 2 cc + 1: ^ 16, and a unit on
@@ -605,7 +612,9 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
     // part q (0 .. 3) of a window's loads; past the end: the last stage again
     auto load_w = [&](int slot, int win, int q) __attribute__((always_inline)) {
         const int y = q & 1, st = min(2 * win + y, nstage - 1);
-        if (q < 2) rs[slot][y] = __builtin_amdgcn_raw_buffer_load_b128(s_buf, s_off, st * KC, 0);
+        if (FAR && q < 2) rs[slot][y] = global_load<t12_u32x4>(s_far + (size_t)st * KC);
+        else if (FAR) rg[slot][y] = global_load<t12_u32x2>(g_far + (size_t)st * (KC / 2));
+        else if (q < 2) rs[slot][y] = __builtin_amdgcn_raw_buffer_load_b128(s_buf, s_off, st * KC, 0);
         else rg[slot][y] = __builtin_amdgcn_raw_buffer_load_b64(g_buf, g_off, st * (KC / 2), 0);
     };
     // part q (0 .. 4) of unit u (eight columns of stage u / 2): a pair of weights each, the first with what they share, the last the store
@@ -647,18 +656,24 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
         const int pw = wave - 4;
         const auto x_buf = tile_buffer(j.act + (size_t)j.b0 * j.act_stride + k_begin);
         uint32_t x_off[NXC];
+        const uint16_t* x_far[NXC];
 #pragma unroll
         for (int c = 0; c < NXC; c++) {
             const int r = 8 * (4 * c + pw) + (lane >> 3);      // (rows past the end: the last one again, not stored)
-            x_off[c] = 2u * ((uint32_t)(min(j.b0 + r, j.B - 1) - j.b0) * (uint32_t)j.act_stride + 8u * ((lane & 7) ^ (r & 7) ^ ((r >> 3) & 1)));
+            const int row = min(j.b0 + r, j.B - 1), unit = 8 * ((lane & 7) ^ (r & 7) ^ ((r >> 3) & 1));
+            x_off[c] = 2u * ((uint32_t)(row - j.b0) * (uint32_t)j.act_stride + (uint32_t)unit);
+            x_far[c] = j.act + (size_t)row * j.act_stride + k_begin + unit;
         }
         auto copy_x = [&](int at, int win) __attribute__((always_inline)) {
 #pragma unroll
             for (int y = 0; y < 2; y++)
 #pragma unroll
-                for (int c = 0; c < NXC; c++)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buf, (ring_lptr)(lx + at + y * L::X + (4 * c + pw) * 1024), 16, x_off[c],
-                                                             min(2 * win + y, nstage - 1) * (2 * KC), 0, 0);
+                for (int c = 0; c < NXC; c++) {
+                    const ring_lptr to = (ring_lptr)(lx + at + y * L::X + (4 * c + pw) * 1024);
+                    const int st = min(2 * win + y, nstage - 1);
+                    if (FAR) __builtin_amdgcn_global_load_lds((ring_gptr)(uintptr_t)(x_far[c] + (size_t)st * KC), to, 16, 0, 0);
+                    else __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buf, to, 16, x_off[c], st * (2 * KC), 0, 0);
+                }
             __builtin_amdgcn_sched_barrier(0);                 // (in this order: the waits below count what is behind a copy)
         };
 #pragma unroll
@@ -800,7 +815,7 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
     return true;
 }
 
-template <int FB, bool SWI = false, int EPI = T12_ACT_NONE, bool DEV = false>
+template <int FB, bool SWI = false, int EPI = T12_ACT_NONE, bool DEV = false, bool FAR = false>
 __global__ __launch_bounds__(512) void gemm_strip_kernel(const GemmParams p)
 {
     using L = StripLds<FB>;
@@ -810,7 +825,7 @@ __global__ __launch_bounds__(512) void gemm_strip_kernel(const GemmParams p)
     int tile = blockIdx.x, bt = blockIdx.y;
     if (!DEV && gridDim.y > 1) tile_of_block(tile, bt);
     for (;; bt++) {
-        if (!gemm_strip_body<FB, SWI, EPI, DEV>(p, tile, bt, lx, lw, lpat, lrow) || !DEV) break;
+        if (!gemm_strip_body<FB, SWI, EPI, DEV, FAR>(p, tile, bt, lx, lw, lpat, lrow) || !DEV) break;
         __syncthreads();                                   // the next tile reuses the staging buffers
     }
 }
