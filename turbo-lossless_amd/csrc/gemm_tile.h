@@ -230,9 +230,6 @@ __device__ __forceinline__ void tile_overflow(const GemmParams& p, const Job& j,
     }
 }
 
-template <bool SWI, int EPI>
-constexpr bool TILE_HALF = SWI || EPI != T12_ACT_NONE;          // bf16 results of a function of the sums
-
 // Stores the sums FIRST .. END - 1 of them, number 16 i + r register r of acc[i].  Register r of lane (ln, lh) is D[row = 8*(r/4) + 4*lh + r%4][col = ln]
 // (row = batch, col = m).  A row's address is the wave's, the lanes add theirs: 64 addresses and conditions of a lane each would not fit its registers.
 template <int FB, bool SWI, int EPI, int FIRST, int END, class Job>
@@ -241,7 +238,7 @@ __device__ __forceinline__ void tile_store(const GemmParams& p, const Job& j, in
     const int lane = threadIdx.x & 63, ln = lane & 31, lh = lane >> 5;
     const int b0 = j.b0 + row0;
     const bool in0 = mw + ln < j.M, in1 = !SWI && mw + 32 + ln < j.M;
-    constexpr bool HALF = TILE_HALF<SWI, EPI>;
+    constexpr bool HALF = SWI || EPI != T12_ACT_NONE;          // bf16 results of a function of the sums
     uint8_t* dst;
     size_t ld;
     if (HALF) {
@@ -275,27 +272,26 @@ __device__ __forceinline__ void tile_store(const GemmParams& p, const Job& j, in
     }
 }
 
-// The end of a tile of four multiplying and four copying waves, all eight there.  What follows a function of the sums is bound by that function's
-// operations (gated unit: 45 a pair), so each copying wave takes half of the sums of a multiplying one, through the LDS of the activations (lx, free by
-// then): gated 28672 x 512 at B = 256 24.1 -> 20.2 us, 28672 x 4096 at 100 / 256 64 -> 62.5, 81.2 -> 79.6.  Plain sums are bound by their stores and stay where they are.  wave: 0 .. 3 of its kind.
+// The end of a tile of four multiplying and four copying waves, all eight there.  Each copying wave takes half of the sums of a multiplying one, through
+// the LDS of the activations (lx, free by then): four waves alone neither hide a gated unit's operations (45 a pair; gated 28672 x 512 at B = 256 24.1 -> 20.2
+// us) nor have enough stores in flight where a slice along K is short (us, plain sums: 2 x 8192 x 2048 at 200 rows 40.0 -> 39.2, 6144 x 4096 at 129 / 160 / 256
+// 30.9 -> 29.9, 32.1 -> 31.0, 34.4 -> 33.4, 8320 x 2048 at 512 34.4 -> 33.2, 3072 x 2048 at 200 20.4 -> 19.6).  wave: 0 .. 3 of its kind.
 template <int FB, bool SWI, int EPI, class Job>
 __device__ __forceinline__ void tile_finish(const GemmParams& p, const Job& j, int esc_mode, int row0, int mw, int wave, uint8_t* lx, t12_f32x16 (&acc)[FB][2])
 {
-    constexpr int N = 16 * FB, KEEP = TILE_HALF<SWI, EPI> ? N / 2 : N;
+    constexpr int N = 16 * FB, KEEP = N / 2;
     tile_overflow<FB, SWI>(p, j, esc_mode, row0, mw, acc);
-    if (KEEP < N) {
-        tile_barrier();                                        // the copies of both kinds of waves have ended
-        uint8_t* const to = lx + wave * (N / 2 * 512) + (threadIdx.x & 63) * 16;
+    tile_barrier();                                            // the copies have ended
+    uint8_t* const to = lx + wave * (N / 2 * 512) + (threadIdx.x & 63) * 16;
 #pragma unroll
-        for (int n = KEEP; n < N; n += 4)
+    for (int n = KEEP; n < N; n += 4)
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const t12_f32x16& a = acc[n >> 4][u];
-                *(t12_f32x4*)(to + ((n - KEEP) / 4 * 2 + u) * 1024) = t12_f32x4{a[n & 15], a[(n & 15) + 1], a[(n & 15) + 2], a[(n & 15) + 3]};
-            }
-        __builtin_amdgcn_s_waitcnt(TILE_LDS_DONE);
-        tile_barrier();
-    }
+        for (int u = 0; u < 2; u++) {
+            const t12_f32x16& a = acc[n >> 4][u];
+            *(t12_f32x4*)(to + ((n - KEEP) / 4 * 2 + u) * 1024) = t12_f32x4{a[n & 15], a[(n & 15) + 1], a[(n & 15) + 2], a[(n & 15) + 3]};
+        }
+    __builtin_amdgcn_s_waitcnt(TILE_LDS_DONE);
+    tile_barrier();
     tile_store<FB, SWI, EPI, 0, KEEP>(p, j, row0, mw, acc);
 }
 template <int FB, bool SWI, int EPI, class Job>
@@ -303,7 +299,6 @@ __device__ __forceinline__ void tile_finish_copying(const GemmParams& p, const J
 {
     constexpr int N = 16 * FB, KEEP = N / 2;
     __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));             // no copy outlives its workgroup or reaches into its next tile
-    if (!TILE_HALF<SWI, EPI>) return;
     tile_barrier();
     tile_barrier();                                        // the sums are there
     t12_f32x16 acc[FB][2];
