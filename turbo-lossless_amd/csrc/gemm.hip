@@ -20,6 +20,7 @@
 // Fast path requirements: K % 64 == 0, 0 <= base_exp <= 240, 16-byte aligned
 // activation rows.  Everything else goes to the general kernel below.
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -834,7 +835,7 @@ int t12_gemm_glu(const T12Segment* gate, const T12Segment* up, const T12Glu* glu
     p.blk_start[0] = 0;
     p.blk_start[1] = p.blk_start[2] = tiles;
     if (act_stride > TILE_MAX_STRIDE) return launch_far<true>(p, tiles, st);
-    // batch tile of 256 rows, or of 128 for 65 .. 128 rows (one accumulator pair per wave)
+    // batch tile of 256 rows, or of 128 for 65 .. 128 rows
     if (B <= 128) return launch_tile<2, true>(p, tiles, st);
     const int wide = (gate->M + WIDE / 2 - 1) / (WIDE / 2);
     if (prefers_wide(tiles * btiles, wide * btiles, device_cus())) {
@@ -1343,7 +1344,7 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
 // known on the device only.  pairs = 0: segment i belongs to group first_group + i; 1 or 2: the segments are (gate, up)
 // pairs, segment i belongs to group first_group + i / 2.  Group g has dev_counts[g] rows, which start dev_base[g] rows
 // into act_bf16 and into the outputs: seg.out (fp32), or for pairs = 1 out_bf16 = bf16( silu(gate) * up ), row stride
-// out_bf16_ld.  hint_b is a count few groups exceed: it
+// out_bf16_ld (asked for with hint_b above 128 only: tiles of 256 batch rows).  hint_b is a count few groups exceed: it
 // picks the batch tile (a group above it is streamed once per tile it needs).  K is never split.  Returns 1 when the shape has no such kernel (the caller then sizes launches on the host).
 __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* segs, int nseg, int K, const void* act_bf16,
                                                            int act_stride, const int* dev_counts, const int* dev_base,
@@ -1422,10 +1423,7 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
         return T12_OK;
     }
     if (act_stride > TILE_MAX_STRIDE) return 1;
-    if (swiglu) {
-        if (hint_b <= 128) return launch_tile<2, true, T12_ACT_NONE, true>(p, tiles, st);
-        return launch_tile<4, true, T12_ACT_NONE, true>(p, tiles, st);
-    }
+    if (swiglu) return launch_tile<4, true, T12_ACT_NONE, true>(p, tiles, st);
     if (hint_b <= 64) return launch_tile<1, false, T12_ACT_NONE, true>(p, tiles, st);
     if (hint_b <= 128) return launch_tile<2, false, T12_ACT_NONE, true>(p, tiles, st);
     return launch_tile<4, false, T12_ACT_NONE, true>(p, tiles, st);
