@@ -79,6 +79,11 @@ __device__ __forceinline__ void tile_barrier()
     asm volatile("" ::: "memory");
 }
 constexpr int TILE_LDS_DONE = 0xC07F;         // s_waitcnt: LDS operations done, nothing else
+// The loops count the loads of planes behind a copy, those of their last round too, which nobody decodes: used here, behind the loop, they are not dropped.
+__device__ __forceinline__ void tile_keep(const t12_u32x4 (&s)[2][2], const t12_u32x2 (&g)[2][2])
+{
+    asm volatile("" : : "v"(s[0][0]), "v"(s[0][1]), "v"(s[1][0]), "v"(s[1][1]), "v"(g[0][0]), "v"(g[0][1]), "v"(g[1][0]), "v"(g[1][1]));
+}
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const void* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, -1, 0x00027000); }
 
@@ -423,8 +428,7 @@ __device__ __forceinline__ bool gemm_tile_body(const GemmParams& p, const int ti
         tile_barrier();                                        // stage 0 is there
         // interval st: the copies of stage st + 2, this half of the weights of stage st + 1; ends when both parts of stage st + 1 are there
         int xat = 2 * L::X;
-        // (the copies of stage st + 1 are older than those of stage st + 2 and, in the loop, than one window's loads; at the end of a slice those are of
-        // windows that nobody decodes, and the compiler leaves them out)
+        // (the copies of stage st + 1 are older than those of stage st + 2 and, in the loop, than one window's loads; behind it no window is left to load)
         auto interval = [&](auto dc, int st, auto loop) __attribute__((always_inline)) {
             constexpr int d = decltype(dc)::value;             // st % 4
             copy_x(xat, st + 2);
@@ -432,7 +436,7 @@ __device__ __forceinline__ bool gemm_tile_body(const GemmParams& p, const int ti
             xat = xat == 2 * L::X ? 0 : xat + L::X;
             uint8_t* const to = lw + ((d + 1) & 1) * L::W;
             put_all(to, ((d + 1) >> 1) & 1, (d + 1) & 1);
-            if ((d & 1) == 0) {
+            if (decltype(loop)::value && (d & 1) == 0) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) load_w((d >> 1) & 1, (st >> 1) + 2, q);
             }
@@ -455,6 +459,7 @@ __device__ __forceinline__ bool gemm_tile_body(const GemmParams& p, const int ti
                 if (st + 2 < nstage) interval(std::integral_constant<int, 2>(), st + 2, std::false_type());
             }
         }
+        tile_keep(rs, rg);
         tile_finish_copying<FB, SWI, EPI>(p, j, ((wave - 4) >> 1) * (FB * 32), j.m0 + (wave & 1) * (SWI ? 32 : 64), wave - 4, lx);
         return true;
     }
@@ -687,8 +692,7 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
         for (int q = 0; q < 4; q++) load_w(0, 2, q);
         __builtin_amdgcn_sched_barrier(0);
         // Interval w: the copies of window w + NXB - 1, this half of the weights of window w + 1; ends when both parts of window w + 1 are there: its copies
-        // are older than those of NXB - 2 windows and than NXB - 1 windows' loads of planes (at the end of a slice those are of windows that nobody
-        // decodes, and the compiler leaves them out).
+        // are older than those of NXB - 2 windows and, in the loop, than NXB - 1 windows' loads of planes (behind it no window is left to load).
         int xat = XEND;
         auto interval = [&](auto dc, int w, auto loop) __attribute__((always_inline)) {
             constexpr int d = decltype(dc)::value;             // w % 2
@@ -696,8 +700,10 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
             xat = xat == XEND ? 0 : xat + L::XW;
             uint8_t* const to = lw + (1 - d) * L::W;
             put_all(to, 1 - d);
+            if (decltype(loop)::value) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) load_w(1 - d, w + 3, q);
+                for (int q = 0; q < 4; q++) load_w(1 - d, w + 3, q);
+            }
             patch(to, k_begin + (w + 1) * 2 * KC);
             __builtin_amdgcn_s_waitcnt(ring_vmcnt((NXB - 2) * 2 * NXC + (decltype(loop)::value ? (NXB - 1) * NWL : 0)) & TILE_LDS_DONE);
             tile_barrier();
@@ -710,6 +716,7 @@ __device__ __forceinline__ bool gemm_strip_body(const GemmParams& p, const int t
         }
         interval(std::integral_constant<int, 0>(), w, std::false_type());
         if (w + 1 < nwin) interval(std::integral_constant<int, 1>(), w + 1, std::false_type());
+        tile_keep(rs, rg);
         tile_finish_copying<FB, SWI, EPI>(p, j, ((wave - 4) >> 1) * (FB * 32), j.m0 + (wave & 1) * (SWI ? 32 : 64), wave - 4, lx);
         return true;
     }
@@ -905,6 +912,7 @@ __device__ __forceinline__ void gemm_wide_body(const GemmParams& p, const int ti
     load_w(0, 0, 1);
 #pragma unroll
     for (int c = 0; c < 4; c++) copy_x(x0, 0, c);
+    __builtin_amdgcn_sched_barrier(0);                         // (in this order: the waits below count what is behind a copy)
     list.stage(j, lpat, lrow);
     load_w(1, 1, 0);
     load_w(1, 1, 1);
@@ -965,8 +973,8 @@ __device__ __forceinline__ void gemm_wide_body(const GemmParams& p, const int ti
     for (int f = 0; f < FB + 2; f++) frag(x0, w0, 0, f);
     // Stage st; half the weights and half the copies of stage st + 1 are done; these of stage st + 2 go into its own buffers once everybody has its
     // operands in registers.  The escapes of stage st + 1 are put in before the third step, not before the barrier: then its products cover a
-    // wave that has some.  (Past the last stage: the last one again, read and not used.)
-    auto stage = [&](auto dc, int st) __attribute__((always_inline)) {
+    // wave that has some.  (Past the last stage: the last one again, read and not used; behind the loop no planes are left to load.)
+    auto stage = [&](auto dc, int st, auto loop) __attribute__((always_inline)) {
         constexpr int d = decltype(dc)::value;                 // st % 2
         uint8_t* const xb = d ? x1 : x0;
         uint8_t* const xn = d ? x0 : x1;
@@ -979,7 +987,7 @@ __device__ __forceinline__ void gemm_wide_body(const GemmParams& p, const int ti
         step(1, xb, wbuf, [&](int q) __attribute__((always_inline)) { put(wn, 1 - d, 3, q); });
         patch(wn, k_begin + (st + 1) * KC);
         step(2, xb, wbuf, [&](int q) __attribute__((always_inline)) {
-            if (q == 0 || q == 2) load_w(1 - d, st + 3, q / 2);
+            if (decltype(loop)::value && (q == 0 || q == 2)) load_w(1 - d, st + 3, q / 2);
         });
         // this stage's operands are in registers: its buffers are free; the next stage is there (behind its copies: four loads of planes)
         __builtin_amdgcn_s_waitcnt(ring_vmcnt(4) & TILE_LDS_DONE);
@@ -992,10 +1000,11 @@ __device__ __forceinline__ void gemm_wide_body(const GemmParams& p, const int ti
     };
     int st = 0;
     for (; st + 2 <= nstage; st += 2) {
-        stage(std::integral_constant<int, 0>(), st);
-        stage(std::integral_constant<int, 1>(), st + 1);
+        stage(std::integral_constant<int, 0>(), st, std::true_type());
+        stage(std::integral_constant<int, 1>(), st + 1, std::true_type());
     }
-    if (st < nstage) stage(std::integral_constant<int, 0>(), st);
+    if (st < nstage) stage(std::integral_constant<int, 0>(), st, std::false_type());
+    tile_keep(rs, rg);
     __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));                 // no copy outlives its workgroup
     tile_overflow<FB, SWI>(p, j, list.mode, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), acc);
     tile_store<FB, SWI, EPI, 0, 16 * FB>(p, j, wb * (FB * 32), j.m0 + wm * (SWI ? 32 : 64), acc);
