@@ -160,7 +160,8 @@ int t12_gemm_deferred(const T12Segment* segs, int nseg, const void* act_bf16, in
  * the two projections.  Returns 0 when launched (B = 5 .. 8; B = 9 .. 64 on 8192 rows of gate and more that t12_gemm
  * takes in 128-row tiles without a split; larger B with enough rows), 1 when the shape has no fused kernel (B <= 4,
  * few rows, K not a multiple of 128 (B <= 64) or 64, base_exp outside 0..240, activation rows that are not 16-byte
- * aligned): run t12_gemm on the two segments and launch_silu_mul_bf16_batch then, which give the same bits; negative
+ * aligned): run t12_gemm on the two segments and launch_silu_mul_bf16_batch then, which give the same bits (sums in another
+ * order where one form's tiles hold their rows' escapes in LDS, 2048 per 128 rows, and the other's do not); negative
  * on bad operands. */
 int t12_gemm_swiglu(const T12Segment* gate, const T12Segment* up, const void* act_bf16, int act_stride,
                     int K, int B, void* out_bf16, int out_stride, void* stream);
