@@ -700,8 +700,9 @@ int device_cus()
 }
 
 // More than 128 rows, unsplit: tiles of 256 x 256 in place of 128 x 256 where their rounds of one workgroup per CU take less time: a round of theirs
-// takes 1.75 of the others' (a stage 1.6 us against 0.93, the ends alike).  28672 x 4096: 512 rows, one round against two, 139 us and 156; 256 rows, one
-// each, 135 and 89; 32000 x 4096 at 256 138 and 89.
+// takes 1.75 of the others' (a stage 1.6 us against 0.93, the ends alike).  One round against two: 28672 x 4096 at 512 rows 124 us and 140, 33000 x 256 / 1024 /
+// 4096 at 256 17.7 / 36 / 113 and 22.6 / 48 / 129, 20000 x 512 / 2048 at 512 22.8 / 61 and 28.7 / 73; two against four: 128256 x 4096 at 256 300 and 317; one each: 28672 x
+// 4096 at 160 / 256 101 / 103 and 77 / 76; two against three: 36000 x 2048 at 512 121 and 112, 28672 x 4096 at 700 219 and 203.
 bool prefers_wide(int tiles, int wide, int cus)
 {
     const int rounds = (tiles + cus - 1) / cus, rounds_wide = (wide + cus - 1) / cus;
@@ -1161,8 +1162,9 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
     int ks = splits_for(btiles);
     // A 256-row batch tile whose K slice is under 16 stages (O of the Llama layer: 32 row tiles, 8 splits of 512
     // columns) spends its time filling and draining, and leaves twice the partial sums: such a launch takes 128-row
-    // batch tiles and half the splits (O at B = 256 32 -> 27.5 us with the reduction; down, whose slices are long,
-    // 55 -> 58 us and QKV 34 -> 37 us the same way, so they keep the 256-row tile).
+    // batch tiles and half the splits (with the reduction: O at B = 160 / 256 25.9 / 28.7 -> 23.6 / 25.0 us, 2048 x 8192 at 200 / 256 30 -> 25, 2048 x 2048
+    // at 200 20.4 -> 17.6; down, whose slices are long, level at 256 and 77.7 -> 84.3 us at 512 the same way, QKV at 160 / 256, its sums left to
+    // the next kernel, 24.8 / 25.7 -> 25.5 / 26.0, so they keep the 256-row tile).
     const bool short_slices = B > 128 && ks > 1 && K / ks < 16 * KC;
     const int ks128 = short_slices ? splits_for(btiles128) : ks;
     if (static_ws) {
@@ -1171,14 +1173,15 @@ int gemm_impl(const T12Segment* segs, int nseg, const void* act_bf16, int act_st
         const size_t need = (size_t)p.ksplit * B * m_total * sizeof(float);
         T12_REQUIRE(p.ksplit == 1 || need <= STATIC_WS_BYTES, NOALLOC_TOO_LARGE, p.ksplit, need, STATIC_WS_BYTES, B, m_total);
     }
-    // (where those are more workgroups than CUs, 256-row tiles are the better ones: 8400 x 1024 at B = 512, 264 workgroups 35.3 us,
-    // 132 of the larger ones 25.2)
+    // (where those are more workgroups than CUs, 256-row tiles are the better ones: 8400 x 1024 at B = 512, 264 workgroups 27.6 us,
+    // 132 of the larger ones 22.3)
     const bool tb128 = short_slices && tiles * btiles128 * t12_slices(K, ks128) <= cus;
     if (tb128) ks = ks128;
     // A few workgroups more than CUs are a second round of everything: one round of fewer slices then, or none, by  rounds x (6.5
     // us + stages x c) + what the partial sums cost (2.5 us and 4 TB/s, as for the ring kernel), c = 0.95 us for a stage of 256
-    // batch rows, 0.65 for 128.  8256 x 2048 at B = 512: 260 workgroups of 2 slices 47.4 us and a reduction of 11, unsplit 38.0;
-    // 4224 x 4096: 264 of 4 slices 47.7, 3 slices 34.1; 8704 x 8192: 272 of 2 slices 138, unsplit 120.
+    // batch rows, 0.65 for 128 (unsplit 8256 x 2048 / 8704 x 8192 at 512 rows: 0.86 / 0.78).  8256 x 2048 at B = 512: 260 workgroups of 2 slices 42.8 us and a
+    // reduction of 12, unsplit 34.0; 8400 x 1024 29.2 and 12, unsplit 22.0; 4224 x 4096: 264 of 4 slices 42.5, 3 slices 28.1; 8704 x 8192: 272 of 2
+    // slices 127, unsplit 107.
     if (!tb128 && ks > 1 && tiles * btiles * t12_slices(K, ks) > cus) {
         const int windows = (K + 2 * KC - 1) / (2 * KC);
         float best = 1e30f;
@@ -1302,8 +1305,8 @@ int t12_gemm_grouped(const T12Group* groups, int ngroups, int K, void* stream)
     p.B = max_b;
     p.m_total = m_total;
     p.split_stride = ws_floats;
-    // batch tile by the largest group, so that every tensor is streamed once (a Mixtral layer of 256 tokens, 48 .. 75
-    // rows per expert: 0.80 ms with tiles of 128, 0.94 with tiles of 64 taken twice by the larger groups, 1.05 with 256)
+    // batch tile by the largest group, so that every tensor is streamed once (the two launches of a Mixtral layer of 256 tokens, 48 .. 75
+    // rows per expert: 0.58 ms with tiles of 128, 0.69 with tiles of 64 taken twice by the larger groups, 0.80 with 256)
     const int tb = max_b <= 64 ? 64 : (max_b <= 128 ? 128 : 256);
     int tiles = 0;
     long units = 0;                                               // workgroups per K split
@@ -1395,8 +1398,8 @@ __attribute__((visibility("hidden"))) int t12_gemm_experts(const T12Segment* seg
     if (!swiglu) p.blk_start[nseg] = tiles;
     hipStream_t st = (hipStream_t)stream;
     // More than a few rows per group: the ring kernel, whose workgroups of 128 rows stream at the memory's rate.  Eight
-    // experts of 4096 / 14336, two per token, whole layer: 12 / 40 / 64 / 128 tokens 340 / 359 / 372 / 425 us, 458 / 462 /
-    // 478 / 502 through the tile kernel; 8 tokens (hint 8) 285 against 398 by the sweep below.  It stops at a hint of 6: with
+    // experts of 4096 / 14336, two per token, whole layer: 12 / 40 / 64 / 128 tokens 353 / 365 / 376 / 430 us, 444 / 439 /
+    // 448 / 469 through the strip kernel; 8 tokens (hint 8) 285 against 398 by the sweep below.  It stops at a hint of 6: with
     // a few of many small experts named there are too few workgroups (64 experts of 2048 / 1408, six per token: 4 tokens,
     // hint 3, 236 us against the sweep's 177, 16 tokens, hint 7, 245 against 309; 32 of 4096 / 768, hint 5: 186 against 179).
     bool ring = !swiglu && hint_b > 6 && hint_b <= RING_MAX_B && K % RING_WC == 0;

@@ -10,20 +10,24 @@
 //   * Escapes are exact and cost no extra pass: the (column, exact bf16) pairs of the tile's rows -- one contiguous slice of the CSR list -- are staged in
 //     LDS once; the thread that decoded 16 columns of a row walks that row's slice in step with the K loop and overwrites the decoded half-words.
 //
+// Times here and at the rules of gemm.hip: a loop of one product over copies of its weights of 600 MB, both sides in turn on one card, us, launch gap and
+// the reduction of K slices included; the cards and loops of other days differ by up to 15 % either way, so only pairs compare.
+//
 // gemm_tile_kernel: 256 batch rows x 128 weight rows.  Four waves multiply (one per SIMD, 128 x 64 each), the four others copy the activations; all
 // eight decode.  Against eight multiplying waves of half the tile that also carried the activations through registers: a quarter fewer LDS reads, two
-// thirds fewer LDS writes (13 cycles per 1 KB where a read takes 4), no shuffling of activations.  us, before -> now: 28672 x 4096 at B = 256 92.5 -> 89,
-// 32000 x 4096 at 256 95 -> 89, 4096 x 14336 at 256 / 512 55 -> 53 / 86.5 -> 82.5.  What bounds it, per stage and CU: the matrix cores (1024 cycles), and the
+// thirds fewer LDS writes (13 cycles per 1 KB where a read takes 4), no shuffling of activations.  Those waves -> these: 28672 x 4096 at B = 256 78.5 -> 76.2,
+// 32000 x 4096 at 256 86.3 -> 82.9, 4096 x 14336 at 256 / 512 51.9 -> 50.3 / 80.6 -> 77.3, 6144 x 4096 at 256 33.9 -> 32.7.  What bounds it, per stage and CU: the matrix cores (1024 cycles), and the
 // loads, which the vector cache takes in order (860 cycles of look-ups, and waiting for planes from HBM in between): 1740 together (1300 without loads of
 // planes, 1100 without the decode as well).
 //
-// gemm_strip_kernel: 64 or 128 batch rows x 128 weight rows, the same roles, two stages between barriers.  28672 x 4096 at B = 100 / 128 65.8 -> 54.9 /
-// 66.4 -> 55.6 us, 4096 x 14336 38.5 -> 37.5, 6144 x 4096 at 100 25.4 -> 24.3 (one stage between barriers: 56.5, 60.7, 37.5, 25.6).  Streaming the planes and decoding
-// them alone takes 41 (a plain read 28); loads further ahead (four windows, five to seven buffers of activations) are 2 .. 5 % slower.
+// gemm_strip_kernel: 64 or 128 batch rows x 128 weight rows, the same roles, two stages between barriers.  28672 x 4096 at B = 100 / 128 56.3 -> 51.5 /
+// 56.7 -> 51.7 (gated epilogue 55.8 -> 51.4 / 56.6 -> 51.3), 4096 x 14336 at 100 37.1 -> 35.3, 6144 x 4096 25.6 -> 23.9 (one stage between barriers is 3 / 9 / 0 / 5 %
+// slower).  Streaming the planes and decoding them alone takes 41 (a plain read 28); loads further ahead (four windows, five to seven buffers of
+// activations) are 2 .. 5 % slower.
 //
 // gemm_wide_kernel: 256 batch rows x 256 weight rows, eight waves of 128 x 64: half the activation traffic and half the LDS writes of activations per
-// product.  28672 x 4096 at B = 300 / 512 147 -> 130 / 156 -> 139 us (gemm_tile_kernel -> here), with the gated epilogue at 512 154 -> 128 (the kernel
-// before both -> here); 2850 cycles per stage against 2048 of the matrix cores, at 1.8 GHz (with every CU multiplying the chip runs no faster).
+// product.  28672 x 4096 at B = 512 / 1024 140 -> 124 / 271 -> 238 (gemm_tile_kernel -> here), with the gated epilogue at 512 152 -> 129 (eight multiplying waves of
+// half the 256 x 128 tile -> here); 2850 cycles per stage against 2048 of the matrix cores, at 1.8 GHz (with every CU multiplying the chip runs no faster).
 // Measured and not taken: four waves of 128 x 128 with 512 registers (165: nothing covers a wave's waits), the reads and the decode in other places
 // between the products, wave priorities (all level or slower), the tile kernel's copies spread between the parts of its decode (2 % slower), its
 // stages begun at another column in every row tile (level; with K slices, whose activations then leave L2, 15 % slower).

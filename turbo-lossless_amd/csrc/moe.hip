@@ -307,8 +307,9 @@ int t12_moe_ffn(const T12MoeExpert* experts, int E, const void* x_bf16, int x_st
     // ---- the grouped launches sized on the device: gate|up of eight experts per launch, down of sixteen.  The batch
     //      tile is picked for a count few experts exceed: mean + 4 standard deviations of an even routing (an expert
     //      above the tile streams its planes once per tile it needs, so a tile below the typical maximum costs more than
-    //      a tile above it).  Above 128 rows the SwiGLU goes into the gate|up epilogue; below, the 128-row SwiGLU tile is
-    //      slower than two plain groups and the SiLU*mul kernel (Mixtral shape, ~64 rows per expert: 490 against 468 us).
+    //      a tile above it).  Above 128 rows the SwiGLU goes into the gate|up epilogue.  (The line was drawn with another tile kernel, at
+    //      ~64 rows per expert of Mixtral shape 490 us of the gated tile of 128 rows against 468 of the plain one and 13 of SiLU*mul; with the strip
+    //      kernel the whole layer took 562 / 570 us gated at 64 / 90 rows against 584 / 603 as it is.)
     // ---- a handful of pairs (a decode step of one or a few sequences): every slot is one matrix-vector product with
     //      its expert's tensors, picked on the device -- gate|up with the SwiGLU in the epilogue, then down.  Each named
     //      expert is streamed once per slot that names it, at the rate of the B = 1 kernel (Mixtral shape, one token:
